@@ -430,3 +430,94 @@ def tolerance(case):
     if ty[0] == "i" or k in ("jacobi", "smooth3") or (k == "rows" and case["op"] == "max"):
         return "exact"
     return {"rel": 1.5e-6, "max": 7e-6} if ty == "f32" else {"rel": 2e-14, "max": 6e-14}
+
+
+# ---- the same in 64 bits ------------------------------------------------------------------------
+
+def _wide(t):
+    """A vector on the host for sums of it: the whole numbers in 64 bits; the others in extended
+    precision, so that these sums' own rounding does not count."""
+    v = t.cpu().numpy()
+    return v.astype(np.int64 if v.dtype.kind == "i" else np.longdouble)
+
+
+def _narrow(v, like):
+    v = np.ascontiguousarray(v)
+    return torch.from_numpy(v.astype(np.float64 if v.dtype.kind == "f" else like))
+
+
+def _segment_sums(v, lens):
+    lens = lens.cpu().numpy().astype(np.int64)
+    starts = np.cumsum(lens) - lens
+    out = np.zeros(len(lens), v.dtype)
+    some = lens > 0
+    if some.any():
+        out[some] = np.add.reduceat(v, starts[some])
+    return out
+
+
+def exact(case, seed):
+    """What `run` returns for the inputs of `prepare(case, seed)`, from torch and numpy alone: whole
+    numbers as they are, the others in 64 bits."""
+    k, ty = case["kind"], case.get("type", "i64")
+    args = prepare(case, seed).args
+    types = [ty] * 3 if k == "blackscholes" else None
+    xs = [_view(a, types or [ty]) for a in args] if k in ("dotp", "rows", "scan", "jacobi", "smooth3", "radix",
+                                                          "blackscholes") else None
+    whole = np.int32 if ty == "i32" else np.int64
+    if k == "dotp":
+        return _narrow(np.sum(_wide(xs[0]) * _wide(xs[1])), whole)
+    if k == "rows":
+        x = xs[0]
+        if case["op"] == "max":
+            return x.amax(1)
+        return x.sum(1) if ty == "i64" else _narrow(_wide(x).sum(1), whole)
+    if k == "scan":
+        kind, x = case["scan"], xs[0]
+        right = kind[4] == "r"
+        if ty[0] == "i":
+            s = torch.cumsum(x.flip(0) if right else x, 0, dtype=TORCH[ty])
+        else:
+            v = _wide(x)
+            s = _narrow(np.cumsum(v[::-1] if right else v), whole)
+        turn = (lambda t: t.flip(0)) if right else (lambda t: t)
+        if kind.endswith("1"):
+            return turn(s)
+        from0 = torch.cat([torch.zeros(1, dtype=s.dtype, device=s.device), s])
+        return (turn(from0[:-1]), from0[-1]) if kind.endswith("'") else turn(from0)
+    if k == "foldseg":
+        return _narrow(_segment_sums(_wide(_view(args[0], [ty])), _view(args[1], ["i32"])), whole)
+    if k == "smvm":
+        lens, cols = _view(args[0], ["i64"]), _view(args[1], ["i64"]).cpu().numpy()
+        vals, vec = (_wide(_view(a, [ty])) for a in args[2:])
+        return _narrow(_segment_sums(vals * vec[cols], lens), whole)
+    if k == "histogram":
+        return torch.bincount(_view(args[0], ["i32"]), minlength=case["bins"]).to(TORCH[ty])
+    if k == "jacobi":
+        g = xs[0].double()
+        for _ in range(case["sweeps"]):
+            p = torch.nn.functional.pad(g[None, None], (1, 1, 1, 1), mode="replicate")[0, 0]
+            g = 0.25 * (p[:-2, 1:-1] + p[1:-1, :-2] + p[1:-1, 2:] + p[2:, 1:-1])
+        return g
+    if k == "smooth3":
+        g = xs[0].double()
+        mode = {"clamp": "replicate", "mirror": "reflect", "wrap": "circular"}[case["boundary"]]
+        p = torch.nn.functional.pad(g[None, None], (1,) * 6, mode=mode)[0, 0]
+        for d in range(3):   # 1 2 1 along each axis
+            n = p.shape[d] - 2
+            p = (p.narrow(d, 0, n) + 2 * p.narrow(d, 1, n) + p.narrow(d, 2, n)) / 4
+        return p
+    if k == "radix":
+        return torch.sort(xs[0]).values
+    price, strike, years = (x.double() for x in xs[0])
+    a1, a2, a3, a4, a5 = SPECTRAL_COEFF
+
+    def cnd(d):
+        t = 1 / (1 + 0.2316419 * d.abs())
+        v = 0.3989422804014327 * torch.exp(-0.5 * d * d) * (t * (a1 + t * (a2 + t * (a3 + t * (a4 + t * a5)))))
+        return torch.where(d > 0, 1 - v, v)
+
+    vs = 0.30 * torch.sqrt(years)
+    d1 = (torch.log(price / strike) + (0.02 + 0.5 * 0.30 * 0.30) * years) / vs
+    n1, n2, xe = cnd(d1), cnd(d1 - vs), strike * torch.exp(-0.02 * years)
+    return [price * n1 - xe * n2, xe * (1 - n2) - price * (1 - n1)]
