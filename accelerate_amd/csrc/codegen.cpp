@@ -2113,6 +2113,79 @@ KernelSource Codegen::stencil2d(const Sx& pattern, const TypeP& outElt, const Sx
   return ks;
 }
 
+// Can several sweeps be computed in one pass?  The kernel computes lanes and margins whose taps
+// are no values of the array, so the function has to be total on any bits: it may not index an
+// array with what it computes, nor loop until a value says so.  A boundary `function` has its
+// values depend on the position, which the marching wave would have to carry: left out.
+static bool pureScalar(const Sx& e) {
+  if (e.atom) return true;
+  if (e.is("while") || e.is("index") || e.is("linearindex") || e.is("shape") || e.is("foreign")) return false;
+  for (size_t k = 0; k < e.size(); ++k)
+    if (!pureScalar(e.at(k))) return false;
+  return true;
+}
+
+bool Codegen::stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const ArrayR& src) {
+  if (src.rank != 2 || !typeEq(src.elt, outElt) || outElt->k != Type::Scalar) return false;
+  const ST st = outElt->st;
+  if (stIsVec(st) || (stSize(st) != 4 && stSize(st) != 8)) return false;
+  const std::string kind = bnd.atom ? bnd.s : bnd.head();
+  if (kind != "clamp" && kind != "mirror" && kind != "wrap" && kind != "constant") return false;
+  if (kind == "constant" && !pureScalar(bnd.at(1))) return false;
+  const std::vector<int> halo = stencilHaloOf(pattern);
+  return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && pureScalar(f);
+}
+
+KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& bnd, const Operand& src) {
+  const std::vector<int> halo = stencilHaloOf(pattern);
+  const int hy = halo[0], hx = halo[1];
+  const std::string kind = bnd.atom ? bnd.s : bnd.head();
+  const std::string E = stName(elt->st);
+  const int v = 16 / stSize(elt->st);  // a lane moves 16 bytes of a row
+  const int most = hy <= 1 && hx <= 1 ? 8 : 4;
+  const ArraySlot& slot = slotByName(src.slot);
+  std::string body;
+  body += "#define ACC_SW_MAX " + std::to_string(most) + "\n";
+  body += "  typedef " + E + " E;\n";
+  body += "  static constexpr int HY = " + std::to_string(hy) + ";\n  static constexpr int HX = " + std::to_string(hx) + ";\n";
+  body += "  static constexpr int BOUNDARY = " + std::string(kind == "clamp" ? "0" : kind == "mirror" ? "1" : kind == "wrap" ? "2" : "3") + ";\n";
+  body += "  ACC_DEV const E* source(const Env& env) { return env." + slot.name + "_0; }\n";
+  body += "  ACC_DEV E* target(const Out& out) { return out.o0; }\n";
+  if (kind != "constant") {
+    body += "  ACC_DEV E outside(const Env&) { return (E)0; }\n";  // not asked for
+  } else {
+    Emit em;
+    em.ind = 4;
+    ValP c = exp(bnd.at(1), {}, em);
+    if (!typeEq(valType(c), elt)) throw Error("stencil: boundary value does not have the element type");
+    em.line("return " + c->ex + ";");
+    body += fnHead("E", "outside", "const Env& env") + em.code + "  }\n";
+  }
+  {
+    // the stencil function over the window of rows w, whose element [HY][HX + k] is the focus
+    Emit em;
+    em.ind = 4;
+    const int k0 = stencilWidth(pattern) / 2;
+    ValP arg = vUnit();
+    for (int dy = -k0; dy <= k0; ++dy) {
+      const Sx& row = pattern.at(1 + dy + k0);
+      if (row.head().compare(0, 4, "unit") != 0) throw Error("stencil2d: pattern is not of rank 2");
+      const int k1 = stencilWidth(row) / 2;
+      ValP rv = vUnit();
+      for (int dx = -k1; dx <= k1; ++dx)
+        rv = vPair(rv, bindLeaf(elt->st, "w[" + std::to_string(hy + dy) + "].e[k + " + std::to_string(hx + dx) + "]", em));
+      arg = vPair(arg, rv);
+    }
+    ValP r = applyFun(f, {arg}, {}, em);
+    if (!typeEq(valType(r), elt)) throw Error("stencil: function result does not match the declared element type");
+    body += "  template <class W>\n" + fnHead("Elt", "apply_win", "const Env& env, const W& w, const int k") + returnElt(r, em) + "  }\n";
+  }
+  KernelSource ks = finish(body, elt, typeLeaves(elt), "stencil2d_sweeps.hpp", v, true);
+  ks.group = most;
+  ks.words = hx * 16 + hy;
+  return ks;
+}
+
 // Rank-3 stencils: tiles of ACC_ST_H x ACC_ST_W results in (y, x) that march along z with a
 // ring of 2*HZ+1 staged planes in LDS (stencil3d.hpp).  Same generated members as for rank 2,
 // with a z coordinate; apply() receives the LDS offsets of the planes z-HZ .. z+HZ.

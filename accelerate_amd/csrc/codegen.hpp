@@ -108,6 +108,10 @@ class Codegen {
   // rank-2 single-source stencil through LDS halo tiles
   KernelSource stencil2d(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource stencil3d(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
+  // several sweeps of a rank-2 stencil over its own result in one launch (stencil2d_sweeps.hpp); only where
+  // stencilSweepable holds
+  KernelSource stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& boundary, const Operand& src);
+  static bool stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const ArrayR& src);
   KernelSource scalarKernel(const Sx& exp);  // evaluates a closed Exp with one thread
 
   // type of a closed scalar expression / result of a function, without emitting code

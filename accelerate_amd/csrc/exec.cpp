@@ -338,6 +338,158 @@ static HValP hostEval(const Sx& e, std::vector<HValP> env, const std::vector<DAr
 }
 
 // ------------------------------------------------------------------------------------
+// loops of stencil sweeps
+
+namespace {
+// What the body of an awhile does with the arrays it is given, followed without running it.
+struct SweepSym {
+  enum K { Unit, Grid, Swept, Other, Pair } k = Unit;  // Grid: a component of the state; Swept: the stencil of it
+  std::string path;
+  std::shared_ptr<SweepSym> a, b;
+};
+using SweepSymP = std::shared_ptr<SweepSym>;
+using SweepEnv = std::vector<SweepSymP>;
+
+struct NotSweeps {};
+
+SweepSymP sweepSym(SweepSym::K k, const std::string& path = "") {
+  auto s = std::make_shared<SweepSym>();
+  s->k = k;
+  s->path = path;
+  return s;
+}
+
+// the state's components, as its type lays them out
+SweepSymP sweepState(const ATyP& t, const std::string& path) {
+  if (t->k == ATy::Unit) return sweepSym(SweepSym::Unit);
+  if (t->k == ATy::Arr) return sweepSym(SweepSym::Grid, path);
+  auto s = sweepSym(SweepSym::Pair);
+  s->a = sweepState(t->a, path + "l");
+  s->b = sweepState(t->b, path + "r");
+  return s;
+}
+
+void sweepPush(const Sx& lhs, const SweepSymP& v, SweepEnv& env) {
+  if (lhs.is("single")) env.push_back(v);
+  else if (lhs.is("pair")) {
+    if (v->k != SweepSym::Pair) throw NotSweeps();
+    sweepPush(lhs.at(1), v->a, env);
+    sweepPush(lhs.at(2), v->b, env);
+  }
+}
+
+struct SweepAnalysis {
+  const Sx* node = nullptr;
+  std::string path;                       // of the component that is swept
+  std::vector<std::string> read;          // components whose contents something else reads
+  bool readsSwept = false;
+
+  const SweepSymP& var(const Sx& v, const SweepEnv& env) {  // (avar I), (index I e), (linearindex I e)
+    const size_t ix = (size_t)v.at(1).asInt();
+    if (ix >= env.size()) throw NotSweeps();
+    return env[env.size() - 1 - ix];
+  }
+  // array variables a scalar expression reads (their extents are the same after any number of sweeps)
+  void scalar(const Sx& e, const SweepEnv& env) {
+    if (e.atom || e.size() == 0) return;
+    if (e.is("shape")) return;
+    if (e.is("index") || e.is("linearindex")) {
+      const SweepSymP& v = var(e, env);
+      if (v->k == SweepSym::Grid) read.push_back(v->path);
+      if (v->k == SweepSym::Swept) readsSwept = true;
+    }
+    for (size_t k = 0; k < e.size(); ++k) scalar(e.at(k), env);
+  }
+  SweepSymP eval(const Sx& n, SweepEnv& env) {
+    if (n.isAtom("anil")) return sweepSym(SweepSym::Unit);
+    if (n.atom) throw NotSweeps();
+    if (n.is("avar")) return var(n, env);
+    if (n.is("alet")) {
+      SweepSymP v = eval(n.at(2), env);
+      const size_t mark = env.size();
+      sweepPush(n.at(1), v, env);
+      SweepSymP r = eval(n.at(3), env);
+      env.resize(mark);
+      return r;
+    }
+    if (n.is("apair")) {
+      auto s = sweepSym(SweepSym::Pair);
+      s->a = eval(n.at(1), env);
+      s->b = eval(n.at(2), env);
+      return s;
+    }
+    if (n.is("apply")) {
+      SweepSymP v = eval(n.at(2), env);
+      return fun(n.at(1), v, env);
+    }
+    if (n.is("unit")) {
+      scalar(n.at(2), env);
+      return sweepSym(SweepSym::Other);
+    }
+    if (n.is("stencil") && n.at(5).is("avar")) {
+      const SweepSymP& v = var(n.at(5), env);
+      if (node || v->k != SweepSym::Grid) throw NotSweeps();
+      node = &n;
+      path = v->path;
+      return sweepSym(SweepSym::Swept, v->path);
+    }
+    throw NotSweeps();
+  }
+  SweepSymP fun(const Sx& f, const SweepSymP& arg, SweepEnv& env) {
+    if (!f.is("alam") || f.at(2).is("alam")) throw NotSweeps();
+    const size_t mark = env.size();
+    sweepPush(f.at(1), arg, env);
+    SweepSymP r = eval(f.at(2), env);
+    env.resize(mark);
+    return r;
+  }
+  // the body's result: the swept array in its own component's place, and nowhere else
+  bool placed(const SweepSymP& r, const std::string& at) {
+    if (r->k == SweepSym::Pair) return placed(r->a, at + "l") && placed(r->b, at + "r");
+    if (r->k == SweepSym::Swept || (r->k == SweepSym::Grid && r->path == path)) return r->k == SweepSym::Swept && at == path;
+    return at != path;
+  }
+};
+}  // namespace
+
+// Is this awhile a loop of stencil sweeps?  Then its iterations can be taken several at a time
+// (evalSweeps): the body must hand the swept component to the stencil and to nothing else, and
+// neither the other components nor the predicate may read what is in it.
+void Program::prepareSweeps(const Sx& n, const TEnv& tenv) {
+  if (!ctx_.knobs.stencil_sweeps || ctx_.knobs.stencil_no2d) return;
+  const Sx &cond = n.at(1), &body = n.at(2);
+  SweepAnalysis an;
+  try {
+    if (!body.is("alam")) return;
+    const ATyP ty = lhsType(body.at(1));
+    const SweepSymP state = sweepState(ty, "");
+    SweepEnv env(tenv.size(), sweepSym(SweepSym::Other));
+    const SweepSymP r = an.fun(body, state, env);
+    if (!an.node || !an.placed(r, "")) return;
+    an.fun(cond, state, env);
+  } catch (const NotSweeps&) {
+    return;
+  }
+  if (an.readsSwept) return;
+  for (const std::string& p : an.read)
+    if (p == an.path) return;
+  const Sx& st = *an.node;
+  const Plan& plan = plans_.at(an.node);
+  if (!plan.ty || plan.ty->k != ATy::Arr || plan.mode != "lds2d") return;
+  const ArrayR& r = plan.ty->r;
+  if (!Codegen::stencilSweepable(st.at(1), r.elt, st.at(3), st.at(4), r)) return;
+  Operand src;
+  src.r = r;
+  src.slot = "a0";
+  Codegen cg({r});
+  Sweep sw;
+  sw.node = an.node;
+  sw.path = an.path;
+  sw.k = ctx_.kernel(cg.stencilSweeps(st.at(1), r.elt, st.at(3), st.at(4), src));
+  sweeps_[&n] = sw;
+}
+
+// ------------------------------------------------------------------------------------
 // preparation (type inference + code generation for every node)
 
 Program::Program(Context& ctx, const char* text, size_t len) : ctx_(ctx) {
@@ -366,6 +518,7 @@ Program::Program(Context& ctx, const char* text, size_t len) : ctx_(ctx) {
     ctx_.wait(kv.second.k3);
     for (auto& sk : kv.second.scalarKernels) ctx_.wait(sk.second);
   }
+  for (auto& kv : sweeps_) ctx_.wait(kv.second.k);
   // a program that is one scan can be run without allocating (runInto): its code objects are
   // loaded now, so that no launch of it has set-up work left
   if (ctx_.hasDevice() && (body_->is("scan") || body_->is("scan'"))) {
@@ -384,6 +537,7 @@ std::vector<std::string> Program::kernelKeys() const {
     for (auto& sk : kv.second.scalarKernels)
       if (sk.second) keys.push_back(sk.second->hash);
   }
+  for (auto& kv : sweeps_) keys.push_back(kv.second.k->hash);
   std::sort(keys.begin(), keys.end());
   keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
   return keys;
@@ -489,6 +643,7 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
     ATyP t = prepare(n.at(3), tenv);
     prepareFun(n.at(1), tenv, nullptr);
     prepareFun(n.at(2), tenv, nullptr);
+    prepareSweeps(n, tenv);
     return t;
   }
   if (h == "use") return atArr(parseArrayR(n.at(1)));
@@ -999,6 +1154,88 @@ void Program::runInto(const std::vector<AValP>& args, const std::vector<DArrayP>
   if (destNext_ != dest_.size()) throw Error("internal: acchip_execute_into left a result unwritten");
 }
 
+bool Program::awhileTest(const Sx& cond, AEnv& aenv, const AValP& x) {
+  AValP p = evalFun(cond, aenv, {x});
+  if (p->k != AVal::Arr || p->arr->bufs.size() != 1) throw Error("awhile: predicate must be a scalar boolean array");
+  if (p->arr->hostKnown) return p->arr->hostValue != 0;  // no round trip to the device
+  unsigned char flag = 0;
+  ctx_.peek(&flag, p->arr->bufs[0]->p, 1);
+  return flag != 0;
+}
+
+static DArrayP componentAt(const AValP& x, const std::string& path, size_t i = 0) {
+  if (i == path.size()) return x->arr;
+  return componentAt(path[i] == 'l' ? x->a : x->b, path, i + 1);
+}
+static AValP withComponent(const AValP& x, const std::string& path, const DArrayP& a, size_t i = 0) {
+  if (i == path.size()) return avArr(a);
+  return path[i] == 'l' ? avPair(withComponent(x->a, path, a, i + 1), x->b) : avPair(x->a, withComponent(x->b, path, a, i + 1));
+}
+
+// A loop of stencil sweeps: iterations are run with the stencil left out (it yields its operand,
+// whose contents nothing reads) until the kernel's number of sweeps has come together or the predicate ends
+// the loop, then all of them are computed in one pass.  A single one is run as it stands.
+AValP Program::evalSweeps(const Sx& n, const Sweep& sw, AEnv& aenv, AValP x) {
+  const Sx &cond = n.at(1), &body = n.at(2);
+  const std::vector<int64_t>& ext = componentAt(x, sw.path)->shape;
+  // the kernel's index arithmetic is 32 bits wide, and a strip's margins fold back once at most
+  if (ext[0] < 32 || ext[1] < 32 || ext[0] > (1 << 30) || ext[1] > (1 << 30)) {
+    while (awhileTest(cond, aenv, x)) x = evalFun(body, aenv, {x});
+    return x;
+  }
+  for (bool more = true; more;) {
+    AValP before = x;
+    int64_t count = 0;
+    {
+      struct Defer {  // left again however an iteration ends
+        Program& p;
+        ~Defer() { p.deferred_ = nullptr; }
+      } defer{*this};
+      deferred_ = sw.node;
+      while (count < sw.k->meta.group && (more = awhileTest(cond, aenv, x))) {
+        before = x;
+        x = evalFun(body, aenv, {x});
+        ++count;
+      }
+    }
+    if (count == 1) x = evalFun(body, aenv, {before});
+    else if (count > 1) {
+      // an odd one out is swept alone, after the others: its iteration is run again in full
+      const DArrayP g = launchSweeps(sw, componentAt(x, sw.path), count & ~1);
+      if (count & 1) x = evalFun(body, aenv, {withComponent(before, sw.path, g)});
+      else x = withComponent(x, sw.path, g);
+    }
+  }
+  return x;
+}
+
+// `count` sweeps (even) of g in passes of 8, 4 and 2
+DArrayP Program::launchSweeps(const Sweep& sw, DArrayP g, int64_t count) {
+  const KernelSource& ks = sw.k->meta;
+  const int64_t h = g->shape[0], w = g->shape[1], hx = ks.words >> 4, hy = ks.words & 15, v = ks.vec;
+  while (count > 0) {
+    const int64_t T = count >= 8 && ks.group >= 8 ? 8 : count >= 4 ? 4 : 2;
+    const char* fn = T == 8 ? "acc_sweeps8" : T == 4 ? "acc_sweeps4" : "acc_sweeps2";
+    const int64_t cols = 64 * v - 2 * ((T * hx + v - 1) / v * v);  // SweepGeo::U
+    const int64_t strips = (w + cols - 1) / cols;
+    // one generation of waves, as many as the device holds: a few more would run a second one
+    const int64_t target = ctx_.knobs.stencil_sweeps > 1 ? ctx_.knobs.stencil_sweeps
+                                                         : std::max<int64_t>(1024, 4 * ctx_.residentGroups(sw.k, fn, 256));
+    const int64_t least = std::max<int64_t>(4, T * hy);
+    int64_t chunks = std::max<int64_t>(1, std::min(target / strips, (h + least - 1) / least));
+    const int64_t rows = (h + chunks - 1) / chunks;
+    chunks = (h + rows - 1) / rows;
+    DArrayP out = alloc(g->r, g->shape);
+    std::vector<uint64_t> args = packArgs(ks, {g}, {}, g->shape);
+    packOut(args, *out);
+    for (int64_t a : {h, w, strips, strips * chunks, rows}) args.push_back((uint64_t)a);
+    ctx_.launch(sw.k, fn, (uint64_t)((strips * chunks + 3) / 4), 256, args);
+    g = out;
+    count -= T;
+  }
+  return g;
+}
+
 AValP Program::eval(const Sx& n, AEnv& aenv) {
   if (n.isAtom("anil")) return avUnit();
   const std::string& h = n.head();
@@ -1062,15 +1299,9 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
   if (h == "awhile") {
     // host loop reading one byte back per iteration (Interpreter.hs:222-229)
     AValP x = eval(n.at(3), aenv);
-    for (;;) {
-      AValP p = evalFun(n.at(1), aenv, {x});
-      if (p->k != AVal::Arr || p->arr->bufs.size() != 1) throw Error("awhile: predicate must be a scalar boolean array");
-      unsigned char flag = 0;
-      if (p->arr->hostKnown) flag = p->arr->hostValue != 0;  // no round trip to the device
-      else ctx_.peek(&flag, p->arr->bufs[0]->p, 1);
-      if (!flag) break;
-      x = evalFun(n.at(2), aenv, {x});
-    }
+    auto sw = sweeps_.find(&n);
+    if (sw != sweeps_.end()) return evalSweeps(n, sw->second, aenv, x);
+    while (awhileTest(n.at(1), aenv, x)) x = evalFun(n.at(2), aenv, {x});
     return x;
   }
   if (h == "use") {
@@ -1504,6 +1735,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     ctx_.launch(plan.k, "acc_permute", (uint64_t)grid, 256, args);
     return avArr(out);
   }
+  if (deferred_ == &n) return eval(n.at(5), aenv);
   if (h == "stencil" || h == "stencil2") {
     const bool two = h == "stencil2";
     std::vector<DArrayP> temps = evalTemps(plan.temps, aenv);

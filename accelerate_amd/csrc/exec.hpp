@@ -80,6 +80,14 @@ struct Plan {
   ATyP ty;                                       // result type of the node
 };
 
+// An awhile whose body sweeps one component of the state with a rank-2 stencil, and does nothing
+// else with it: its iterations can be computed several at a time (stencil2d_sweeps.hpp).
+struct Sweep {
+  const Sx* node = nullptr;  // the stencil
+  KernelP k;
+  std::string path;          // where the component lies in the state: 'l' / 'r' per pair
+};
+
 class Program {
  public:
   Program(Context& ctx, const char* text, size_t len);
@@ -103,6 +111,8 @@ class Program {
   const Sx* body_ = nullptr;
   std::vector<const Sx*> lams_;
   std::map<const Sx*, Plan> plans_;
+  std::map<const Sx*, Sweep> sweeps_;   // by awhile node
+  const Sx* deferred_ = nullptr;        // a stencil whose sweeps are being counted: yields its operand unchanged
   const std::vector<DArrayP>* uses_ = nullptr;
   // runInto: alloc() hands out the caller's arrays, in the order the node asks for its results,
   // and fails once they are used up
@@ -124,6 +134,10 @@ class Program {
   // execution
   AValP eval(const Sx& n, AEnv& aenv);
   AValP evalFun(const Sx& f, AEnv& aenv, const std::vector<AValP>& args);
+  void prepareSweeps(const Sx& n, const TEnv& tenv);
+  bool awhileTest(const Sx& cond, AEnv& aenv, const AValP& x);
+  AValP evalSweeps(const Sx& n, const Sweep& sw, AEnv& aenv, AValP x);
+  DArrayP launchSweeps(const Sweep& sw, DArrayP g, int64_t count);
   HValP hostExp(const Sx& e, const AEnv& aenv, const Plan& plan);
   std::vector<int64_t> hostShape(const Sx& e, const AEnv& aenv, const Plan& plan, int rank);
   std::vector<DArrayP> evalTemps(const std::vector<const Sx*>& temps, AEnv& aenv);

@@ -1,0 +1,140 @@
+"""Loops of stencil sweeps (awhile around a rank-2 stencil of its own state): several iterations
+computed in one pass (stencil2d_sweeps.hpp) against the same program with one launch per sweep, which
+the oracle tests cover.  A sweep's function fixes the order of its operations, so results are equal
+bit for bit."""
+import numpy as np
+import pytest
+
+from accelerate_amd import ir as A, programs as P
+
+from . import progs as Q
+
+Int = A.Int
+BOUNDARIES = ["clamp", "mirror", "wrap", "constant"]
+# extents at the edges of the kernel's strips (128 / 256 columns less 2 x 8, 4, 2 margins of 1 or 2) and chunks
+SHAPES = [(32, 32), (33, 47), (37, 240), (64, 241), (40, 255), (95, 256), (41, 497), (257, 112), (130, 1003), (1001, 123)]
+
+
+def _boundary(kind, ty):
+    return A.constant(ty, 3) if kind == "constant" else kind
+
+
+def sweeps(step, ty):
+    """the grid after as many sweeps as the second argument, a scalar, says"""
+    grid, cnt = A.tarray(2, ty), A.tarray(0, Int)
+    state = A.tpair(A.tpair(A.unit, grid), cnt)
+
+    def prog(g0, n):
+        loop = A.awhile(state, lambda st: A.unit_(A.u8, A.gt(Int, A.index(st[1], A.nil), A.constI(0))),
+                        lambda st: A.apair(A.apair(A.anil, A.apply(step(), st[0][1])),
+                                           A.unit_(Int, A.sub(Int, A.index(st[1], A.nil), A.constI(1)))),
+                        A.apair(A.apair(A.anil, g0), A.unit_(Int, A.index(n, A.nil))))
+        return A.alet(state, loop, lambda st: st[0][1])
+
+    return A.alam([grid, cnt], prog)
+
+
+def fixed_sweeps(step, ty, count):
+    """... as many as a constant says: the loop's counter never needs the device"""
+    grid, cnt = A.tarray(2, ty), A.tarray(0, Int)
+    state = A.tpair(cnt, grid)
+
+    def prog(g0):
+        loop = A.awhile(state, lambda st: A.unit_(A.u8, A.lt(Int, A.index(st[0], A.nil), A.constI(count))),
+                        lambda st: A.apair(A.unit_(Int, A.add(Int, A.index(st[0], A.nil), A.constI(1))),
+                                           A.apply(step(), st[1])),
+                        A.apair(A.unit_(Int, A.constI(0)), g0))
+        return A.alet(state, loop, lambda st: st[1])
+
+    return A.alam([grid], prog)
+
+
+def _grid(shape, npty, seed):
+    rng = np.random.default_rng(seed)
+    if np.dtype(npty).kind == "f":
+        g = rng.uniform(-1, 1, shape).astype(npty)
+        g[3, 5], g[-1, -1], g[7, 0] = np.inf if seed == 1 else 1, -0.0, np.finfo(npty).tiny / 4
+        return g
+    return rng.integers(-1 << 30, 1 << 30, shape).astype(npty)
+
+
+def _both(ctx, knobs, prog):
+    fused = ctx.compile(prog)
+    knobs("stencil_sweeps", 0)
+    single = ctx.compile(prog)
+    knobs("stencil_sweeps", 1)
+    assert len(fused.kernel_keys) == len(single.kernel_keys) + 1   # the kernel under test is there
+    return fused, single
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", BOUNDARIES)
+@pytest.mark.parametrize("ty,npty,widths", [
+    (A.f32, np.float32, (3, 3)), (A.f32, np.float32, (5, 5)), (A.f32, np.float32, (3, 5)), (A.f32, np.float32, (5, 3)),
+    (A.f64, np.float64, (3, 3)), (A.f64, np.float64, (3, 5)), (A.i32, np.int32, (3, 3)), (A.i64, np.int64, (5, 5))], ids=str)
+def test_sweeps_equal_single_launches(gpu_ctx, knobs, ty, npty, kind, widths):
+    step = lambda: Q.stencil_weighted(ty, widths, _boundary(kind, ty))
+    fused, single = _both(gpu_ctx, knobs, sweeps(step, ty))
+    for k, shape in enumerate(SHAPES):
+        g = gpu_ctx.to_device(_grid(shape, npty, k), A.tarray(2, ty))
+        # (integer arithmetic wraps; one grid holds an infinity, and its NaNs compare equal)
+        for n in ((1, 2, 3, 7, 8, 13) if k < 3 else (2 + k, 8)):
+            cnt = gpu_ctx.to_device(np.array(n, np.int64), A.tarray(0, Int))
+            got, want = fused.execute(g, cnt).to_host(), single.execute(g, cnt).to_host()
+            assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (shape, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves", [2, 64, 100000])
+def test_jacobi_by_chunks_of_rows(gpu_ctx, knobs, waves):
+    from oracle import c as OC
+    fused, _ = _both(gpu_ctx, knobs, fixed_sweeps(P.jacobi_step, A.f32, 19))
+    knobs("stencil_sweeps", waves)
+    for shape in SHAPES:
+        g = np.random.default_rng(5).uniform(0, 1, shape).astype(np.float32)
+        got = fused.execute(gpu_ctx.to_device(g, A.tarray(2, A.f32))).to_host()
+        assert np.array_equal(got, OC.jacobi_f32(g, 19)), shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 1), (1, 40), (31, 64), (64, 31), (0, 64), (64, 0)], ids=str)
+def test_extents_below_the_kernels(gpu_ctx, knobs, shape):
+    step = lambda: Q.stencil_weighted(A.i32, (3, 3), "clamp")
+    fused, single = _both(gpu_ctx, knobs, fixed_sweeps(step, A.i32, 9))
+    g = gpu_ctx.to_device(np.arange(shape[0] * shape[1], dtype=np.int32).reshape(shape), A.tarray(2, A.i32))
+    assert np.array_equal(fused.execute(g).to_host(), single.execute(g).to_host())
+
+
+def _state_loop(cond, body):
+    grid, cnt = A.tarray(2, A.f32), A.tarray(0, Int)
+    state = A.tpair(cnt, grid)
+    return A.alam([grid], lambda g0: A.alet(
+        state, A.awhile(state, cond, body, A.apair(A.unit_(Int, A.constI(0)), g0)), lambda st: st[1]))
+
+
+def test_loops_that_read_the_grid_are_left_alone(cc_ctx):
+    """No kernel of several sweeps where an iteration's grid is read by anything but the stencil, or
+    where the function could not stand lanes outside the array."""
+    below = lambda st: A.unit_(A.u8, A.lt(Int, A.index(st[0], A.nil), A.constI(9)))
+    up = lambda st: A.unit_(Int, A.add(Int, A.index(st[0], A.nil), A.constI(1)))
+    first = lambda g: A.index(g, A.sh(A.constI(0), A.constI(0)))
+    plain = lambda st: A.apair(up(st), A.apply(P.jacobi_step(), st[1]))
+    extent = lambda st: A.apair(
+        A.unit_(Int, A.add(Int, A.shapesize(2, A.shape(st[1])), A.index(st[0], A.nil))), A.apply(P.jacobi_step(), st[1]))
+    reads_cond = lambda st: A.unit_(A.u8, A.lt(A.f32, first(st[1]), A.const(A.f32, 9.0)))
+    reads_body = lambda st: A.apair(
+        A.unit_(Int, A.cond(A.lt(A.f32, first(st[1]), A.const(A.f32, 0.5)), A.constI(9), A.constI(1))),
+        A.apply(P.jacobi_step(), st[1]))
+    twice = lambda st: A.apair(up(st), A.apply(P.jacobi_step(), A.apply(P.jacobi_step(), st[1])))
+    mapped = lambda st: A.apair(up(st), A.map_(A.f32, A.lam([A.f32], lambda v: v), A.apply(P.jacobi_step(), st[1])))
+    kept = lambda st: A.apair(up(st), st[1])
+    for cond, body, fused in [(below, plain, True), (below, extent, True), (reads_cond, plain, False), (below, reads_body, False),
+                              (below, twice, False), (below, mapped, False), (below, kept, False)]:
+        prog = _state_loop(cond, body)
+        on = cc_ctx.compile(prog).kernel_keys
+        old = cc_ctx.set_knob("stencil_sweeps", 0)
+        try:
+            off = cc_ctx.compile(prog).kernel_keys
+        finally:
+            cc_ctx.set_knob("stencil_sweeps", old)
+        assert len(on) - len(off) == (1 if fused else 0)
