@@ -1256,7 +1256,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
   }
   body += "  static constexpr int G = " + std::to_string(g) + ";\n";
   body += "#define ACC_SCAN_BLOCK " + std::to_string(pipe ? 1024 : block) + "\n";
-  int rowsG = g;
+  int rowsG = g, allG = 0;
   if (!pipe) {
     // prefixes of the lane totals by raking through LDS, when the totals of a workgroup fit
     int sz = 0, al = 1;
@@ -1272,6 +1272,10 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
     // do not fit the registers -- 2^20 rows of 256 Int32: 406 us against 730)
     rowsG = std::max(1, std::min(g, 128 / std::max(1, vec * std::max(1, eltBytes))));
     if (small) body += "#define ACC_ROWS_G " + std::to_string(rowsG) + "\n";
+    if (small) {
+      allG = std::max(1, std::min(8, 64 / std::max(1, vec * std::max(1, eltBytes))));
+      body += "#define ACC_SCAN_ALL_G " + std::to_string(allG) + "\n";
+    }
     if (small && rowsG > 1 && (long)(block / 64) * (64 * (rowsG + 1) + 1) * sz <= 64 * 1024 && !(re && re[0] == '0'))
       body += "#define ACC_ROWS_RAKE 1\n";
   }
@@ -1309,6 +1313,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
   ks.scanRight = right;
   ks.pipeSlot = pipeSlot;
   ks.rowsGroup = rowsG;
+  ks.allGroup = allG;
   return ks;
 }
 

@@ -275,6 +275,56 @@ ACC_DEV bool acc_lookback(const typename S::Env& env, const u64* rowDesc, i64 ti
   return have;
 }
 
+// The same prefix where a row has few tiles and all of them run at once: every tile publishes its
+// aggregate and reads those of all tiles before it, each thread of the workgroup K consecutive
+// ones, in one round trip however far back they lie, and nobody waits for another's prefix.  The
+// values are joined in order (across the lanes, then the waves).  Called by all threads; the
+// result is valid in all of them.  The wait is bounded as in acc_window.
+template <class S>
+ACC_DEV bool acc_lookback_all(const typename S::Env& env, const u64* rowDesc, i64 tile, u64 epoch, u64 limit, u32* err,
+                              typename S::Elt& excl) {
+  typedef typename S::Elt Elt;
+  const int W = AccScanCfg<S>::W;
+  __shared__ Elt sh_all[ACC_SCAN_WAVES];
+  const int K = (int)((tile + ACC_SCAN_BLOCK - 1) / ACC_SCAN_BLOCK);  // tile > 0
+  const int lane = acc_lane(), w = acc_wave();
+  const int wfirst = w * ACC_WAVE * K;                                // this wave's first predecessor
+  const int left = (int)tile - wfirst;
+  const int nv = left <= 0 ? 0 : ((left + K - 1) / K < ACC_WAVE ? (left + K - 1) / K : ACC_WAVE);  // lanes with any
+  Elt r;
+  for (int q = 0; q < K; ++q) {
+    const i64 idx = (i64)wfirst + (i64)lane * K + q;
+    bool need = idx < tile;
+    Elt v;
+    u64 polls = 0;
+    for (;;) {
+      if (need && acc_try_read<Elt>(rowDesc + idx * W, v, epoch) != 0) {
+        r = q == 0 ? v : S::combine(env, r, v);
+        need = false;
+      }
+      if (__ballot(need) == 0) break;
+      if (++polls >= limit) {
+        if (need) {
+          __hip_atomic_store(err, 3u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          if (q == 0) r = S::seed(env);  // (any value: the launch has failed)
+        }
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  if (nv > 0) {
+    r = acc_wave_reduce<S>(env, r, lane, nv);
+    if (lane == 0) sh_all[w] = r;
+  }
+  __syncthreads();
+  const int waves = (int)((tile + (i64)ACC_WAVE * K - 1) / ((i64)ACC_WAVE * K));
+  excl = sh_all[0];
+  for (int k = 1; k < waves; ++k) excl = S::combine(env, excl, sh_all[k]);
+  if (S::kSeeded) excl = S::combine(env, S::seed(env), excl);
+  return true;
+}
+
 // Exclusive prefixes of the 64 * G values t[g] that the lanes of a wave hold, taken in the
 // order (g, lane), by raking: the values go to the wave's stretch of LDS (`mine`, room for
 // 64 * (G + 1) + 1 elements), every lane scans G consecutive ones serially, one ordered wave
@@ -334,8 +384,9 @@ ACC_DEV void acc_rake(const typename S::Env& env, typename S::Elt* mine, const t
 // can move them with one wide request: a caller whose store tests for a special position
 // (the total of scan', which is the sequence's last value) sets it for the tiles that cannot hold
 // that position; in the tile that can, only the run that reaches the end goes value by value.  `settle` delays
-// the first look at the predecessors (see acc_lookback).
-template <class S, class Load, class Store, class StoreRun>
+// the first look at the predecessors (see acc_lookback).  ALL: the prefix comes from all
+// predecessors at once (acc_lookback_all).
+template <class S, bool ALL = false, class Load, class Store, class StoreRun>
 ACC_DEV void acc_scan_tile(const typename S::Env& env, u64* desc, i64 tiles, i64 tile, i64 n, u64 epoch, u64 limit,
                            u32* err, const Load& load, const Store& store, const StoreRun& storeRun, bool plain,
                            bool settle) {
@@ -463,9 +514,9 @@ ACC_DEV void acc_scan_tile(const typename S::Env& env, u64* desc, i64 tiles, i64
     Elt t = sh_wave[lane < ACC_SCAN_WAVES ? lane : 0];
     t = acc_wave_scan<S>(env, t, lane);
     if (lane < ACC_SCAN_WAVES) sh_wave[lane] = t;
-    if (lane == wavesWithData - 1 && tile > 0 && successors) acc_publish<Elt>(desc + tile * W, t, epoch, 1);
+    if (lane == wavesWithData - 1 && (ALL || tile > 0) && successors) acc_publish<Elt>(desc + tile * W, t, epoch, 1);
   }
-  __syncthreads();
+  if constexpr (!ALL) __syncthreads();
 
   Elt excl;
   bool hasExcl = false;
@@ -474,25 +525,32 @@ ACC_DEV void acc_scan_tile(const typename S::Env& env, u64* desc, i64 tiles, i64
       excl = S::seed(env);
       hasExcl = true;
     }
+    if constexpr (ALL) __syncthreads();  // the scanned wave totals
+  } else if constexpr (ALL) {
+    hasExcl = acc_lookback_all<S>(env, desc, tile, epoch, limit, err, excl);  // (a barrier of its own)
   } else {
     hasExcl = acc_lookback<S>(env, desc, tile, epoch, settle, limit, err, excl);  // valid in thread 0
   }
-  if (threadIdx.x == 0) {
-    if (successors && wavesWithData > 0) {
-      Elt inc;
-      acc_join<S>(env, hasExcl, excl, true, sh_wave[wavesWithData - 1], inc);
-      acc_publish<Elt>(desc + tile * W, inc, epoch, 2);
+  if constexpr (!ALL) {
+    if (threadIdx.x == 0) {
+      if (successors && wavesWithData > 0) {
+        Elt inc;
+        acc_join<S>(env, hasExcl, excl, true, sh_wave[wavesWithData - 1], inc);
+        acc_publish<Elt>(desc + tile * W, inc, epoch, 2);
+      }
+      sh_excl = excl;
+      sh_has_excl = hasExcl ? 1 : 0;
     }
-    sh_excl = excl;
-    sh_has_excl = hasExcl ? 1 : 0;
+    __syncthreads();
   }
-  __syncthreads();
 
   // prefix of everything before this wave
   Elt base;
   const bool hasWavePre = w > 0 && w <= wavesWithData;
   Elt wavePre = sh_wave[w > 0 ? w - 1 : 0];
-  bool hasBase = acc_join<S>(env, sh_has_excl != 0, sh_excl, hasWavePre, wavePre, base);
+  bool hasBase;
+  if constexpr (ALL) hasBase = acc_join<S>(env, hasExcl, excl, hasWavePre, wavePre, base);
+  else hasBase = acc_join<S>(env, sh_has_excl != 0, sh_excl, hasWavePre, wavePre, base);
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     const i64 t0 = wlo + ((i64)g * ACC_WAVE + lane) * V;

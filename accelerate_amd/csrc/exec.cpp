@@ -523,8 +523,8 @@ Program::Program(Context& ctx, const char* text, size_t len) : ctx_(ctx) {
   // loaded now, so that no launch of it has set-up work left
   if (ctx_.hasDevice() && (body_->is("scan") || body_->is("scan'"))) {
     const Plan& plan = plans_.at(body_);
-    ctx_.preload(plan.k, {"acc_scan", "acc_scan_rows"});
-    ctx_.preload(plan.k2, {"acc_scan", "acc_scan_rows"});
+    ctx_.preload(plan.k, {"acc_scan"});
+    ctx_.preload(plan.k2, {"acc_scan", "acc_scan_rows", "acc_scan_all", "acc_scan_all2"});
     if (plan.k3) ctx_.preload(plan.k3, {"acc_scan_pipe", "acc_scan_pipe_tail"});
   }
 }
@@ -1903,7 +1903,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     }
     const long long forcedTiles = ctx_.knobs.scan_tiles;  // 1 large / 2 small / 3 rows: override, for tests
     if (forcedTiles == 1 || forcedTiles == 4) small = false;
-    if (forcedTiles == 2 && plan.k2) small = true;
+    if ((forcedTiles == 2 || forcedTiles >= 5) && plan.k2) small = true;
     if (plan.k2 && len >= 1) {
       // many short rows: several whole rows per workgroup (acc_scan_rows)
       const KernelSource& sm = plan.k2->meta;
@@ -1948,7 +1948,29 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     }
     const KernelP& kern = pipe ? plan.k3 : (small ? plan.k2 : plan.k);
     const KernelSource& m = kern->meta;
-    const int64_t tile = (int64_t)m.block * m.group * m.vec;
+    // Of the small tiles, where all of them run at once: a quarter of their size for up to a tile per CU,
+    // half of it for up to three, and every tile reads all its predecessors' aggregates (acc_scan_all,
+    // acc_scan_all2).  Measured, acc_scan / all / all2 in us, scanl: Float32 2^18 7.0 / 4.6 / 5.1, 2^20 (256 tiles
+    // of acc_scan_all) 7.5 / 6.4 / 6.4, 2^21 9.2 / 8.3 / 7.7, 2^22 12.7 / 12.7 / 10.2, 6 million (733 tiles of
+    // acc_scan_all2) 16.9 / 17.9 / 14.0, 2^23 (1024) 17.7 / 26.0 / 18.6; Int64 2^17 7.2 / 4.7 / 5.6, 2^19 (256) 7.6 /
+    // 6.1 / 6.4, 2^20 9.3 / 7.9 / 7.2, 2^21 12.6 / 12.0 / 9.8, 3 million (733) 15.0 / 16.6 / 13.0, 2^22 (1024) 17.1 / 26.2 / 17.3.
+    const char* fn = "acc_scan";
+    int64_t group = m.group;
+    if (small && (forcedTiles == 0 || forcedTiles >= 5) && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0) {
+      for (int two = forcedTiles == 6 ? 1 : 0; two < 2; ++two) {
+        const char* f = two ? "acc_scan_all2" : "acc_scan_all";
+        const int64_t g = (int64_t)m.allGroup * (two + 1), t = (int64_t)m.block * g * m.vec, all = rows * ((len + t - 1) / t);
+        const int64_t most = forcedTiles >= 5 ? 4096 : (two ? 3 : 1) * ctx_.computeUnits();
+        // (every CU holds at least one workgroup of any kernel: the runtime need not be asked)
+        if (all <= most && (all <= ctx_.computeUnits() || all <= ctx_.residentGroups(kern, f, (unsigned)m.block))) {
+          fn = f;
+          group = g;
+          break;
+        }
+        if (forcedTiles == 5) break;
+      }
+    }
+    const int64_t tile = (int64_t)m.block * group * m.vec;
     const int64_t tpr = std::max<int64_t>(1, (len + tile - 1) / tile);
     const int64_t tiles = rows * tpr;
     if (tiles > 0x7fffffffLL) throw Error("scan: too many tiles for one launch");
@@ -1989,9 +2011,10 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     // A launch whose tiles are all on the device at once needs no tickets: a tile's number is its
     // workgroup's, nobody waits for a tile that cannot start, and every workgroup is spared the
     // counter's round trip in front of its loads (one row of 2^20 Int32: 7.5 -> 6.5 us).
-    const bool ticketless = skew == 0 && ctx_.knobs.scan_ticketless != 0 && tiles <= ctx_.residentGroups(kern, "acc_scan", (unsigned)m.block);
+    const bool ticketless = skew == 0 && ctx_.knobs.scan_ticketless != 0 &&
+                            (tiles <= ctx_.computeUnits() || tiles <= ctx_.residentGroups(kern, fn, (unsigned)m.block));
     if (ticketless) args[ticketAt] = 0;
-    ctx_.launch(kern, "acc_scan", (uint64_t)tiles, (unsigned)m.block, args);
+    ctx_.launch(kern, fn, (uint64_t)tiles, (unsigned)m.block, args);
     if (!ticketless) st.ticketBase += (uint64_t)tiles;
     return result;
   }

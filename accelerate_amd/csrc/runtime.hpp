@@ -67,7 +67,7 @@ struct Knobs {
   long long stencil_sweeps = 1;     // 0: a loop of stencil sweeps computes one at a time; > 1: waves a launch of several sweeps aims at
   long long stencil_no2d = 0, stencil_no3d = 0;  // 1: rank-2 / rank-3 stencils through the generic skeleton
   long long pool_async = 1;         // 1: device blocks come from the stream-ordered allocator (hipMallocAsync), 0: hipMalloc
-  long long scan_tiles = 0;         // 0: decide per launch, 1 large, 2 small, 3 rows, 4 pipelined (where the operand allows)
+  long long scan_tiles = 0;         // 0: decide per launch, 1 large, 2 small, 3 rows, 4 pipelined (where the operand allows), 5 / 6 acc_scan_all / acc_scan_all2
   long long scan_spin_limit = (long long)1 << 22;  // polls after which a tile stops waiting (seconds)
   long long scan_test_skew = 0;     // fault injection: the ticket base passed to the kernel lags by this much
   void fromEnv();
