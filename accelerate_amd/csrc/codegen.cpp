@@ -2196,6 +2196,90 @@ KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const S
   return ks;
 }
 
+bool Codegen::stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src) {
+  if (src.delayed || src.r.rank != 3 || src.r.elt->k != Type::Scalar || outElt->k != Type::Scalar) return false;
+  const ST st = src.r.elt->st;
+  if (stIsVec(st) || stIsVec(outElt->st) || (stSize(st) != 4 && stSize(st) != 8)) return false;
+  const std::string kind = bnd.atom ? bnd.s : bnd.head();
+  if (kind != "clamp" && kind != "mirror" && kind != "wrap" && kind != "constant") return false;
+  if (kind == "constant" && !pureScalar(bnd.at(1))) return false;
+  const std::vector<int> halo = stencilHaloOf(pattern);
+  // (the window has to fit the registers: 3 planes x 6 rows of 4 values are 72 of them, 3 x 4 of twice the size 96)
+  return halo.size() == 3 && halo[0] == 1 && halo[1] == 1 && halo[2] <= 1 && pureScalar(f);
+}
+
+KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src, int& taps) {
+  const std::vector<int> halo = stencilHaloOf(pattern);
+  const std::string kind = bnd.atom ? bnd.s : bnd.head();
+  const TypeP elt = src.r.elt;
+  const std::string E = stName(elt->st);
+  // Two columns a lane, four rows of 4-byte elements, two of 8-byte ones.  (columns, rows), smoothing with 27
+  // taps, 401 x 387 x 393 / 512^3 / 200^3 in us: Float32 (2, 4) 162 / 323 / 24, (4, 4) 200 / 584 / 32, (4, 2) 206 / 563 / 30,
+  // (2, 2) 196 / 375 / 23, (2, 6) 261 / 496 / 33, through LDS 211 / 332 / 35; Float64, launches of two generations of workgroups,
+  // (2, 2) 317 / 586 / 33, (1, 4) 323 / 692 / 31, (2, 4) 323 / 637 / 46, through LDS 346 / 600 / 54.
+  const int v = 2;
+  const int rows = stSize(elt->st) == 4 ? 4 : 2;
+  const ArraySlot& slot = slotByName(src.slot);
+  std::string body;
+  body += "  typedef " + E + " E;\n  static constexpr int R = " + std::to_string(rows) + ";\n";
+  const char* names[3] = {"HZ", "HY", "HX"};
+  for (int k = 0; k < 3; ++k) body += std::string("  static constexpr int ") + names[k] + " = " + std::to_string(halo[k]) + ";\n";
+  body += "  static constexpr int BOUNDARY = " + std::string(kind == "clamp" ? "0" : kind == "mirror" ? "1" : kind == "wrap" ? "2" : "3") + ";\n";
+  body += "  ACC_DEV const E* source(const Env& env) { return env." + slot.name + "_0; }\n";
+  if (kind != "constant") {
+    body += "  ACC_DEV E outside(const Env&) { return (E)0; }\n";  // not asked for
+  } else {
+    Emit em;
+    em.ind = 4;
+    ValP c = exp(bnd.at(1), {}, em);
+    if (!typeEq(valType(c), elt)) throw Error("stencil: boundary value does not have the element type");
+    em.line("return " + c->ex + ";");
+    body += fnHead("E", "outside", "const Env& env") + em.code + "  }\n";
+  }
+  {
+    Emit em;
+    em.ind = 4;
+    const int k0 = stencilWidth(pattern) / 2;
+    std::vector<std::string> names3;
+    ValP arg = vUnit();
+    for (int dz = -k0; dz <= k0; ++dz) {
+      const Sx& plane = pattern.at(1 + dz + k0);
+      const int k1 = stencilWidth(plane) / 2;
+      ValP pv = vUnit();
+      for (int dy = -k1; dy <= k1; ++dy) {
+        const Sx& row = plane.at(1 + dy + k1);
+        if (row.head().compare(0, 4, "unit") != 0) throw Error("stencil3d: pattern is not of rank 3");
+        const int k2 = stencilWidth(row) / 2;
+        ValP rv = vUnit();
+        for (int dx = -k2; dx <= k2; ++dx) {
+          ValP t = bindLeaf(elt->st, "w.r[" + std::to_string(halo[0] + dz) + "][b + " + std::to_string(halo[1] + dy) + "].e[k + " +
+                                         std::to_string(halo[2] + dx) + "]", em);
+          names3.push_back(t->ex);
+          rv = vPair(rv, t);
+        }
+        pv = vPair(pv, rv);
+      }
+      arg = vPair(arg, pv);
+    }
+    const size_t bound = em.code.size();
+    ValP r = applyFun(f, {arg}, {}, em);
+    if (!typeEq(valType(r), outElt)) throw Error("stencil: function result does not match the declared element type");
+    const std::string code = returnElt(r, em), used = code.substr(bound);
+    // (names are v and a number: one occurrence that no further digit follows is enough)
+    taps = 0;
+    for (const std::string& nm : names3)
+      for (size_t at = used.find(nm); at != std::string::npos; at = used.find(nm, at + 1))
+        if (at + nm.size() >= used.size() || !std::isdigit((unsigned char)used[at + nm.size()])) {
+          ++taps;
+          break;
+        }
+    body += "  template <class W>\n" + fnHead("Elt", "apply_win", "const Env& env, const W& w, const int b, const int k") + code + "  }\n";
+  }
+  KernelSource ks = finish(body, outElt, typeLeaves(outElt), "stencil3d_rows.hpp", v);
+  ks.group = rows;
+  return ks;
+}
+
 // Rank-3 stencils: tiles of ACC_ST_H x ACC_ST_W results in (y, x) that march along z with a
 // ring of 2*HZ+1 staged planes in LDS (stencil3d.hpp).  Same generated members as for rank 2,
 // with a z coordinate; apply() receives the LDS offsets of the planes z-HZ .. z+HZ.

@@ -113,6 +113,9 @@ class Codegen {
   // stencilSweepable holds
   KernelSource stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& boundary, const Operand& src);
   static bool stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const ArrayR& src);
+  // rank 3 from registers (stencil3d_rows.hpp); only where stencilRowsable holds.  taps: how many the function reads
+  KernelSource stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src, int& taps);
+  static bool stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource scalarKernel(const Sx& exp);  // evaluates a closed Exp with one thread
 
   // type of a closed scalar expression / result of a function, without emitting code

@@ -785,8 +785,24 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
       plan.k = ctx_.kernel(cg.stencil2d(pats[0], outElt, *f, bnds[0], srcs[0]));
       plan.mode = "lds2d";
     } else if (!two && srcs[0].r.rank == 3 && !ctx_.knobs.stencil_no3d) {
-      plan.k = ctx_.kernel(cg.stencil3d(pats[0], outElt, *f, bnds[0], srcs[0]));
+      KernelSource lds = cg.stencil3d(pats[0], outElt, *f, bnds[0], srcs[0]);
       plan.mode = "lds3d";
+      if (ctx_.knobs.stencil_rows3d && Codegen::stencilRowsable(pats[0], outElt, *f, bnds[0], srcs[0])) {
+        Codegen cgr(aenvOf(tenv));
+        Plan scratch;
+        Operand src = operandOf(n.at(5), cgr, tenv, scratch);
+        int taps = 0;
+        KernelSource rows = cgr.stencil3dRows(pats[0], outElt, *f, bnds[0], src, taps);
+        // Through LDS the time grows with the taps (7 / 27 of them, 401 x 387 x 393: Float32 138 / 211 us, Float64
+        // 250 / 346), from registers it hardly does (152 / 162, 301 / 317): the lines lie where the two meet.
+        const long long least = ctx_.knobs.stencil_rows3d > 1 ? 1 : stSize(srcs[0].r.elt->st) == 4 ? 16 : 25;
+        if (taps >= least) {
+          plan.k = ctx_.kernel(rows);
+          plan.wide = std::make_shared<KernelSource>(std::move(lds));
+          plan.mode = "rows3d";
+        }
+      }
+      if (!plan.k) plan.k = ctx_.kernel(lds);
     } else {
       plan.k = ctx_.kernel(cg.stencil(pats, outElt, *f, bnds, srcs));
     }
@@ -1790,9 +1806,34 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       ctx_.launch(plan.k, "acc_stencil2d", (uint64_t)(tilesX * chunksY), 256, args);
       return avArr(out);
     }
-    if (plan.mode == "lds3d") {
+    const bool wide3d = plan.mode == "rows3d" && (ext[0] >= (1 << 30) || ext[1] >= (1 << 30) || ext[2] >= (1 << 30));
+    if (plan.mode == "rows3d" && !wide3d) {
       if (out->size() == 0) return avArr(out);
-      const int64_t th = plan.k->meta.group, tw = plan.k->meta.words;
+      const int64_t v = plan.k->meta.vec, hx = stencilHaloOf(n.at(1))[2];
+      const int64_t cols = 64 * v - 2 * ((hx + v - 1) / v * v);  // kCols
+      const int64_t strips = (ext[2] + cols - 1) / cols, r = plan.k->meta.group;
+      const int64_t bands = ((ext[1] + r - 1) / r + 3) / 4 * 4, groups = strips * bands / 4;
+      const int64_t resident = std::max<int64_t>(256, ctx_.residentGroups(plan.k, "acc_stencil3d_rows", 256));
+      // chunks of planes so that the launch fills the device once (twice for 8-byte elements: 512^3 816 -> 586 us)
+      const int64_t gens = ctx_.knobs.stencil_chain > 0 ? ctx_.knobs.stencil_chain : r >= 4 ? 1 : 2;
+      int64_t chunks = std::max<int64_t>(1, std::min(gens * resident / groups, (ext[0] + 3) / 4));
+      const int64_t planes = (ext[0] + chunks - 1) / chunks;
+      chunks = (ext[0] + planes - 1) / planes;
+      if (groups * chunks > 0x7fffffffLL) throw Error("stencil: too many tiles for one launch");
+      std::vector<uint64_t> args = packArgs(plan.k->meta, aenv, temps, ext);
+      packOut(args, *out);
+      for (int64_t a : {ext[0], ext[1], ext[2], strips, bands, chunks, planes}) args.push_back((uint64_t)a);
+      ctx_.launch(plan.k, "acc_stencil3d_rows", (uint64_t)(groups * chunks), 256, args);
+      return avArr(out);
+    }
+    if (plan.mode == "lds3d" || wide3d) {
+      if (out->size() == 0) return avArr(out);
+      KernelP k3d = plan.k;
+      if (wide3d) {
+        k3d = ctx_.kernel(*plan.wide);
+        ctx_.wait(k3d);
+      }
+      const int64_t th = k3d->meta.group, tw = k3d->meta.words;
       const int64_t tilesY = (ext[1] + th - 1) / th, tilesX = (ext[2] + tw - 1) / tw;
       // planes per workgroup: long enough to amortise the 2*HZ planes staged before the first
       // result, short enough that the grid fills the device
@@ -1802,13 +1843,13 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       chain = std::max<int64_t>(1, std::min(chain, ext[0]));
       const int64_t chunksZ = (ext[0] + chain - 1) / chain;
       if (tilesX * tilesY * chunksZ > 0x7fffffffLL) throw Error("stencil: too many tiles for one launch");
-      std::vector<uint64_t> args = packArgs(plan.k->meta, aenv, temps, ext);
+      std::vector<uint64_t> args = packArgs(k3d->meta, aenv, temps, ext);
       packOut(args, *out);
       for (int k = 0; k < 3; ++k) args.push_back((uint64_t)ext[k]);
       args.push_back((uint64_t)tilesX);
       args.push_back((uint64_t)tilesY);
       args.push_back((uint64_t)chain);
-      ctx_.launch(plan.k, "acc_stencil3d", (uint64_t)(tilesX * tilesY * chunksZ), 256, args);
+      ctx_.launch(k3d, "acc_stencil3d", (uint64_t)(tilesX * tilesY * chunksZ), 256, args);
       return avArr(out);
     }
     launchMap(plan.k, aenv, temps, *out);

@@ -1,0 +1,63 @@
+"""Rank-3 stencils of many taps computed from registers (stencil3d_rows.hpp) against the kernel that goes
+through LDS, which the oracle tests cover: the function fixes the order of its operations, so results
+are equal bit for bit."""
+import numpy as np
+import pytest
+
+from accelerate_amd import ir as A
+
+from . import progs as Q
+
+pytestmark = pytest.mark.gpu
+
+# extents at the edges of a strip (124 columns of the 128 its lanes hold), of the four bands of 4 or 2 rows of a
+# workgroup and of the loop's three planes; the smallest
+SHAPES = [(2, 2, 2), (3, 3, 5), (1, 4, 7), (5, 1, 64), (4, 9, 123), (6, 8, 124), (7, 31, 125), (9, 16, 128), (3, 5, 249),
+          (33, 17, 126), (12, 100, 130), (5, 33, 248)]
+
+
+def _weighted(ty, nx, boundary):
+    """all taps of 3 x 3 x nx, distinct weights"""
+    return Q.stencil_weighted(ty, (3, 3, nx), boundary) if nx > 1 else _column(ty, boundary)
+
+
+def _column(ty, boundary):
+    """the 9 taps of 3 x 3 x 1, to a result of another type"""
+    row = A.sunit(1, ty)
+    sr = A.stup(*[A.stup(row, row, row)] * 3)
+
+    def f(st):
+        acc = A.const(A.i64, 1)
+        for p in A.untup(st):
+            for r in A.untup(p):
+                for t in A.untup(r):
+                    acc = A.add(A.i64, A.mul(A.i64, acc, A.constI(3)), A.fromintegral(ty, A.i64, t))
+        return acc
+
+    return A.alam([A.tarray(3, ty)], lambda g: A.stencil(sr, A.i64, A.lam([A.stencil_type(sr)], f), boundary, g))
+
+
+@pytest.mark.parametrize("chain", [0, 7])
+@pytest.mark.parametrize("kind", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ty,npty,nx", [(A.f32, np.float32, 3), (A.f64, np.float64, 3), (A.i32, np.int32, 3), (A.i64, np.int64, 3),
+                                        (A.i32, np.int32, 1)], ids=str)
+def test_equal_to_the_lds_kernel(gpu_ctx, knobs, ty, npty, nx, kind, chain):
+    prog = _weighted(ty, nx, A.constant(ty, 3) if kind == "constant" else kind)
+    knobs("stencil_rows3d", 0)
+    lds = gpu_ctx.compile(prog)
+    knobs("stencil_rows3d", 2)
+    rows = gpu_ctx.compile(prog)
+    assert lds.kernel_keys != rows.kernel_keys
+    rng = np.random.default_rng(6)
+    for shape in SHAPES:
+        if kind == "mirror" and min(shape[:2] + (shape[2:] if nx > 1 else ())) < 2:
+            continue  # refused: shorter than the taps reach
+        g = rng.integers(-999, 999, shape).astype(npty)
+        if np.dtype(npty).kind == "f":
+            g *= npty(0.37)
+        d = gpu_ctx.to_device(g, A.tarray(3, ty))
+        want = lds.execute(d).to_host()
+        knobs("stencil_chain", chain)
+        got = rows.execute(d).to_host()
+        knobs("stencil_chain", 0)
+        assert np.array_equal(got, want), shape
