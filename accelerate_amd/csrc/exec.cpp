@@ -915,14 +915,7 @@ void Program::materialize(DArray& a) {
   if (!a.hostKnown || a.onDevice) return;
   if (noAlloc_) throw Error("an argument of acchip_execute_into has not been written to the device yet");
   auto leaves = typeLeaves(a.r.elt);
-  Buffer& b = *a.bufs.at(0);
-  if (!b.p) {  // (shared with the array's reshapes, which then find it)
-    b.p = ctx_.malloc(b.bytes);
-    if (!b.p) throw Error("Remote memory exhausted");  // Array/Remote/LRU.hs:250-341
-    b.ctx = ctx_.shared_from_this();
-    b.owned = true;
-  }
-  void* p = b.p;
+  void* p = a.bufs.at(0)->p;
   const uint64_t v = (uint64_t)a.hostValue;
   hipStream_t st = ctx_.stream();
   switch (stSize(leaves.at(0))) {
@@ -1337,18 +1330,13 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
   auto seeded = [&](const Sx& s) { return !s.isAtom("nothing"); };
 
   if (h == "unit") {
+    DArrayP out = alloc(plan.ty->r, {});
     // the host follows integral scalars made of index arithmetic and other such scalars; the
-    // device copy is made and written only if something reads it there (materialize): an iteration
-    // of a loop that counts on the host then asks the pool for nothing
+    // device copy is written only if something reads it there (materialize)
     if (plan.ty->r.elt->k == Type::Scalar && !stIsFloat(plan.ty->r.elt->st) && hostSupported(n.at(2), true)) {
       try {
         HValP v = hostEval(n.at(2), {}, aenv);
         if (v->k == HVal::Leaf) {
-          auto out = std::make_shared<DArray>();
-          out->r = plan.ty->r;
-          auto b = std::make_shared<Buffer>();
-          b->bytes = (size_t)stSize(plan.ty->r.elt->st);
-          out->bufs.push_back(b);
           out->hostKnown = true;
           out->hostValue = wrapTo(plan.ty->r.elt->st, v->i);
           out->onDevice = false;
@@ -1357,7 +1345,6 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       } catch (const HostUnknown&) {
       }
     }
-    DArrayP out = alloc(plan.ty->r, {});
     launchMap(plan.k, aenv, {}, *out);
     return avArr(out);
   }
