@@ -2123,27 +2123,46 @@ KernelSource Codegen::stencil2d(const Sx& pattern, const TypeP& outElt, const Sx
   return ks;
 }
 
-// Can several sweeps be computed in one pass?  The kernel computes lanes and margins whose taps
-// are no values of the array, so the function has to be total on any bits: it may not index an
-// array with what it computes, nor loop until a value says so.  A boundary `function` has its
-// values depend on the position, which the marching wave would have to carry: left out.
-static bool pureScalar(const Sx& e) {
+// Has a scalar expression over its own variables a value whatever bits they hold?  The kernels that
+// march with windows in registers evaluate a stencil's function on lanes and margins whose taps
+// are no values of the array, so it may neither index an array with what it computes nor loop until a
+// value says so, and no operation may be undefined for some operands: the compiler takes it that such
+// operands never occur, and may drop all that leads there (a kernel that divided by a tap came out empty).
+// Integer division is therefore allowed by a positive constant only, rotr (which negates its amount) by a
+// constant, and conversions from floating point to integers, which are undefined beyond the integers' range, are not.
+static bool totalScalar(const Sx& e) {
   if (e.atom) return true;
-  if (e.is("while") || e.is("index") || e.is("linearindex") || e.is("shape") || e.is("foreign")) return false;
+  for (const char* h : {"while", "index", "linearindex", "shape", "foreign", "fromindex"})
+    if (e.is(h)) return false;
+  if (e.is("case") && e.at(3).isAtom("none")) return false;
+  if (e.is("prim")) {
+    const std::string& op = e.at(1).s;
+    for (const char* h : {"truncate", "round", "floor", "ceiling"})
+      if (op == h) return false;
+    for (const char* h : {"quot", "rem", "quotrem", "idiv", "mod", "divmod", "rotr"})
+      if (op == h) {
+        const Sx& arg = e.at(3);
+        if (!arg.is("pair") || !arg.at(2).is("const") || !arg.at(2).at(2).atom) return false;
+        const std::string& lit = arg.at(2).at(2).s;
+        if (lit[0] == '-' || std::strtoull(lit.c_str(), nullptr, 10) == 0) return false;
+      }
+  }
   for (size_t k = 0; k < e.size(); ++k)
-    if (!pureScalar(e.at(k))) return false;
+    if (!totalScalar(e.at(k))) return false;
   return true;
 }
 
+// Can several sweeps be computed in one pass?  (A boundary `function` has its values depend on the
+// position, which the marching wave would have to carry: left out.)
 bool Codegen::stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const ArrayR& src) {
   if (src.rank != 2 || !typeEq(src.elt, outElt) || outElt->k != Type::Scalar) return false;
   const ST st = outElt->st;
   if (stIsVec(st) || (stSize(st) != 4 && stSize(st) != 8)) return false;
   const std::string kind = bnd.atom ? bnd.s : bnd.head();
   if (kind != "clamp" && kind != "mirror" && kind != "wrap" && kind != "constant") return false;
-  if (kind == "constant" && !pureScalar(bnd.at(1))) return false;
+  if (kind == "constant" && !totalScalar(bnd.at(1))) return false;
   const std::vector<int> halo = stencilHaloOf(pattern);
-  return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && pureScalar(f);
+  return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && totalScalar(f);
 }
 
 KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& bnd, const Operand& src) {
@@ -2202,10 +2221,10 @@ bool Codegen::stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& 
   if (stIsVec(st) || stIsVec(outElt->st) || (stSize(st) != 4 && stSize(st) != 8)) return false;
   const std::string kind = bnd.atom ? bnd.s : bnd.head();
   if (kind != "clamp" && kind != "mirror" && kind != "wrap" && kind != "constant") return false;
-  if (kind == "constant" && !pureScalar(bnd.at(1))) return false;
+  if (kind == "constant" && !totalScalar(bnd.at(1))) return false;
   const std::vector<int> halo = stencilHaloOf(pattern);
   // (the window has to fit the registers: 3 planes x 6 rows of 4 values are 72 of them, 3 x 4 of twice the size 96)
-  return halo.size() == 3 && halo[0] == 1 && halo[1] == 1 && halo[2] <= 1 && pureScalar(f);
+  return halo.size() == 3 && halo[0] == 1 && halo[1] == 1 && halo[2] <= 1 && totalScalar(f);
 }
 
 KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src, int& taps) {

@@ -18,8 +18,9 @@
 // Boundary conditions hold in every sweep: a tap outside the array is replaced from the same
 // sweep's rows and columns (clamp, mirror), by the constant, or, for wrap, by continuing the array
 // periodically, which is the same numbers computed twice.  Lanes whose position lies outside the
-// array, and the margins of a strip, compute values nobody uses: the code generator takes this
-// path only for functions of the taps that are pure arithmetic.
+// array, and the margins of a strip, compute values nobody uses, on taps that no element has (zeros
+// among them): the code generator takes this path only for functions of the taps that are defined
+// for all of them, which a division by a tap is not.
 
 // results of one lane and row: S::V values of type S::E, with HX neighbours on either side
 #define ACC_SW_P (2 * Spec::HY + 1)

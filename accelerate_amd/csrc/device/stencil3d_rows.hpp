@@ -13,8 +13,8 @@
 //
 // Outside the array a tap is replaced as `bounded` says (Interpreter.hs:797-839): columns and rows
 // in the registers, planes by the index of the plane that is loaded, or the constant.  As in
-// the kernel for several sweeps, margins compute values nobody uses, so the function must be pure
-// arithmetic.
+// the kernel for several sweeps, margins compute values nobody uses on taps that no element has, so the
+// function must be defined for all of them.
 
 #define ACC_SR_ROWS (Spec::R + 2 * Spec::HY)
 #define ACC_SR_PZ (2 * Spec::HZ + 1)

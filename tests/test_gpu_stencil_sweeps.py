@@ -138,3 +138,91 @@ def test_loops_that_read_the_grid_are_left_alone(cc_ctx):
         finally:
             cc_ctx.set_knob("stencil_sweeps", old)
         assert len(on) - len(off) == (1 if fused else 0)
+
+
+def _nine(ty, fn, boundary="clamp"):
+    """a step over the nine taps of a 3 x 3 pattern, row by row"""
+    row = A.sunit(3, ty)
+    sr = A.stup(row, row, row)
+    f = A.lam([A.stencil_type(sr)], lambda st: fn([t for r in A.untup(st) for t in A.untup(r)]))
+    return A.alam([A.tarray(2, ty)], lambda g: A.stencil(sr, ty, f, boundary, g))
+
+
+def _kernels(ctx, prog, knob, on):
+    """keys of the program with the knob at `on`, and with it off"""
+    old = ctx.set_knob(knob, on)
+    try:
+        with_it = ctx.compile(prog).kernel_keys
+        ctx.set_knob(knob, 0)
+        return with_it, ctx.compile(prog).kernel_keys
+    finally:
+        ctx.set_knob(knob, old)
+
+
+# Lanes in the margins of a strip compute on combinations of values that the array does not hold, so no
+# operation of the function may be undefined for any of them (a division by what happens to be zero is, and the compiler
+# may drop all that leads there).
+_FLOOR = lambda t: A.fromintegral(A.i32, A.f32, A.floor(A.f32, A.i32, t))
+PARTIAL = {
+    "rem": (A.i32, lambda t: A.rem(A.i32, A.const(A.i32, 1000003), t[4])),
+    "quot": (A.i32, lambda t: A.add(A.i32, A.quot(A.i32, t[4], t[5]), t[1])),
+    "idiv": (A.i64, lambda t: A.idiv(A.i64, t[4], t[5])),
+    "mod": (A.i64, lambda t: A.mod(A.i64, t[4], A.bor(A.i64, t[5], A.const(A.i64, 1)))),
+    "quotrem": (A.u32, lambda t: A.let(A.tpair(A.u32, A.u32), A.quotrem(A.u32, t[0], t[8]), lambda v: A.add(A.u32, v[0], v[1]))),
+    "divmod": (A.i32, lambda t: A.let(A.tpair(A.i32, A.i32), A.divmod_(A.i32, t[0], t[8]), lambda v: A.add(A.i32, v[0], v[1]))),
+    "by zero": (A.i32, lambda t: A.quot(A.i32, t[4], A.const(A.i32, 0))),
+    "by minus one": (A.i32, lambda t: A.quot(A.i32, t[4], A.const(A.i32, -1))),
+    "guarded": (A.i32, lambda t: A.cond(A.eq(A.i32, t[5], A.const(A.i32, 0)), t[4], A.quot(A.i32, t[4], t[5]))),
+    "floor": (A.f32, lambda t: _FLOOR(A.add(A.f32, t[4], t[5]))),
+    "rotr": (A.i64, lambda t: A.rotr(A.i64, t[4], t[5])),
+    "fromindex": (A.i64, lambda t: A.let(A.tshape(2), A.fromindex(2, A.sh(t[1], t[3]), t[4]), lambda ix: ix[1])),
+    "no alternative": (A.i32, lambda t: A.case(A.fromintegral(A.i32, A.u8, t[4]), [(0, t[1]), (1, t[3])])),
+}
+TOTAL = {
+    "by a constant": (A.i32, lambda t: A.add(A.i32, A.quot(A.i32, t[4], A.const(A.i32, 3)), A.mod(A.i32, t[5], A.const(A.i32, 7)))),
+    "shifts": (A.i32, lambda t: A.bxor(A.i32, A.shl(A.i32, t[4], A.constI(3)), A.shr(A.i32, t[5], A.fromintegral(A.i32, A.Int, t[3])))),
+    "rotates": (A.i64, lambda t: A.bxor(A.i64, A.rotl(A.i64, t[4], t[5]), A.rotr(A.i64, t[3], A.constI(5)))),
+    "fdiv": (A.f32, lambda t: A.fdiv(A.f32, t[4], t[5])),
+    "alternatives": (A.i32, lambda t: A.case(A.fromintegral(A.i32, A.u8, t[4]), [(0, t[1]), (1, t[3])], t[7])),
+}
+
+
+def test_functions_undefined_for_some_values_are_left_alone(cc_ctx):
+    for name, (ty, fn) in list(PARTIAL.items()) + list(TOTAL.items()):
+        on, off = _kernels(cc_ctx, fixed_sweeps(lambda: _nine(ty, fn, "wrap"), ty, 9), "stencil_sweeps", 1)
+        assert len(on) - len(off) == (1 if name in TOTAL else 0), name
+
+
+def _window(g, kind):
+    """the nine taps of every element"""
+    p = np.pad(g, 1, **({"mode": "constant", "constant_values": 3} if kind == "constant" else
+                        {"mode": {"clamp": "edge", "mirror": "reflect", "wrap": "wrap"}[kind]}))
+    return [p[y:y + g.shape[0], x:x + g.shape[1]] for y in range(3) for x in range(3)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", BOUNDARIES)
+def test_division_by_a_tap(gpu_ctx, kind):
+    # 2 + 1000003 rem (centre + up): never zero
+    step = lambda t: A.add(A.i32, A.const(A.i32, 2), A.rem(A.i32, A.const(A.i32, 1000003), A.add(A.i32, t[4], t[1])))
+    run = gpu_ctx.compile(fixed_sweeps(lambda: _nine(A.i32, step, _boundary(kind, A.i32)), A.i32, 5))
+    for shape in SHAPES:
+        g = np.random.default_rng(2).integers(1, 5000, shape).astype(np.int32)
+        want = g
+        for _ in range(5):
+            w = _window(want, kind)
+            want = (2 + 1000003 % (w[4] + w[1])).astype(np.int32)
+        assert np.array_equal(run.execute(gpu_ctx.to_device(g, A.tarray(2, A.i32))).to_host(), want), shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(TOTAL))
+def test_total_functions_equal_single_launches(gpu_ctx, knobs, name):
+    ty, fn = TOTAL[name]
+    npty = {A.i32: np.int32, A.i64: np.int64, A.f32: np.float32}[ty]
+    for kind in BOUNDARIES:
+        fused, single = _both(gpu_ctx, knobs, fixed_sweeps(lambda: _nine(ty, fn, _boundary(kind, ty)), ty, 11))
+        for k, shape in enumerate(SHAPES):
+            g = gpu_ctx.to_device(_grid(shape, npty, k), A.tarray(2, ty))
+            got, want = fused.execute(g).to_host(), single.execute(g).to_host()
+            assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (kind, shape)
