@@ -1237,8 +1237,9 @@ DArrayP Program::launchSweeps(const Sweep& sw, DArrayP g, int64_t count) {
     const int64_t target = ctx_.knobs.stencil_sweeps > 1 ? ctx_.knobs.stencil_sweeps
                                                          : std::max<int64_t>(1024, 4 * ctx_.residentGroups(sw.k, fn, 256));
     // at least as many rows as a wave's margins have, unless that leaves SIMDs without a wave (8 rows / as few
-    // as it takes: 100 x 100 14.9 / 11.9 us, 1000 x 1000 15.7 / 14.3, 500 x 3000 17.1 / 15.8)
-    const int64_t most = std::max((h + T * hy - 1) / (T * hy), 4 * ctx_.computeUnits() / strips);
+    // as it takes: 100 x 100 14.9 / 11.9 us, 1000 x 1000 15.7 / 14.3, 500 x 3000 17.1 / 15.8).  A pattern of one row has no such margins.
+    const int64_t margin = std::max<int64_t>(1, T * hy);
+    const int64_t most = std::max((h + margin - 1) / margin, 4 * ctx_.computeUnits() / strips);
     int64_t chunks = std::max<int64_t>(1, std::min({target / strips, most, (h + 1) / 2}));
     const int64_t rows = (h + chunks - 1) / chunks;
     chunks = (h + rows - 1) / rows;

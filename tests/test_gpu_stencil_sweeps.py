@@ -226,3 +226,42 @@ def test_total_functions_equal_single_launches(gpu_ctx, knobs, name):
             g = gpu_ctx.to_device(_grid(shape, npty, k), A.tarray(2, ty))
             got, want = fused.execute(g).to_host(), single.execute(g).to_host()
             assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (kind, shape)
+
+
+def _sum(ty, widths, boundary):
+    """the sum of the taps of a pattern that may be one row, one column or one element"""
+    row = A.sunit(widths[1], ty)
+    sr = A.stup(*[row] * widths[0])
+
+    def f(st):
+        acc = A.const(ty, 1)
+        for r in A.untup(st):
+            for t in A.untup(r):
+                acc = A.add(ty, A.mul(ty, A.const(ty, 0.5 if ty in (A.f32, A.f64) else 3), acc), t)
+        return acc
+
+    return A.alam([A.tarray(2, ty)], lambda g: A.stencil(sr, ty, A.lam([A.stencil_type(sr)], f), boundary, g))
+
+
+FLAT = [(1, 3), (3, 1), (1, 5), (5, 1), (1, 1)]
+
+
+def test_patterns_of_one_row_or_column_get_the_kernel(cc_ctx):
+    for widths in FLAT + [(3, 3), (5, 5), (3, 7), (7, 1)]:
+        prog = fixed_sweeps(lambda: _sum(A.i32, widths, "clamp"), A.i32, 9)
+        on, off = _kernels(cc_ctx, prog, "stencil_sweeps", 1)
+        assert len(on) - len(off) == (1 if max(widths) <= 5 else 0), widths
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", BOUNDARIES)
+@pytest.mark.parametrize("widths", FLAT, ids=str)
+@pytest.mark.parametrize("ty,npty", [(A.f32, np.float32), (A.i64, np.int64)], ids=["f32", "i64"])
+def test_patterns_of_one_row_or_column(gpu_ctx, knobs, ty, npty, widths, kind):
+    fused, single = _both(gpu_ctx, knobs, sweeps(lambda: _sum(ty, widths, _boundary(kind, ty)), ty))
+    for k, shape in enumerate(SHAPES):
+        g = gpu_ctx.to_device(_grid(shape, npty, k), A.tarray(2, ty))
+        for n in (1, 2, 7, 8, 13) if k < 3 else (8 + k,):
+            cnt = gpu_ctx.to_device(np.array(n, np.int64), A.tarray(0, Int))
+            got, want = fused.execute(g, cnt).to_host(), single.execute(g, cnt).to_host()
+            assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (shape, n)
