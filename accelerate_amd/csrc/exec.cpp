@@ -1203,10 +1203,10 @@ AValP Program::evalSweeps(const Sx& n, const Sweep& sw, AEnv& aenv, AValP x) {
     int64_t count = 0;
     {
       struct Defer {  // left again however an iteration ends
-        Program& p;
-        ~Defer() { p.deferred_ = nullptr; }
-      } defer{*this};
-      deferred_ = sw.node;
+        AEnv& env;
+        ~Defer() { env.deferred = nullptr; }
+      } defer{aenv};
+      aenv.deferred = sw.node;
       while (count < sw.k->meta.group && (more = awhileTest(cond, aenv, x))) {
         x = evalFun(body, aenv, {x});
         ++count;
@@ -1753,7 +1753,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     ctx_.launch(plan.k, "acc_permute", (uint64_t)grid, 256, args);
     return avArr(out);
   }
-  if (deferred_ == &n) return eval(n.at(5), aenv);
+  if (aenv.deferred == &n) return eval(n.at(5), aenv);
   if (h == "stencil" || h == "stencil2") {
     const bool two = h == "stencil2";
     std::vector<DArrayP> temps = evalTemps(plan.temps, aenv);

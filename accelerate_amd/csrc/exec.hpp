@@ -113,7 +113,6 @@ class Program {
   std::vector<const Sx*> lams_;
   std::map<const Sx*, Plan> plans_;
   std::map<const Sx*, Sweep> sweeps_;   // by awhile node
-  const Sx* deferred_ = nullptr;        // a stencil whose sweeps are being counted: yields its operand unchanged
   const std::vector<DArrayP>* uses_ = nullptr;
   // runInto: alloc() hands out the caller's arrays, in the order the node asks for its results,
   // and fails once they are used up
@@ -122,7 +121,10 @@ class Program {
   size_t destNext_ = 0;
 
   using TEnv = std::vector<ArrayR>;     // back() has de Bruijn index 0
-  using AEnv = std::vector<DArrayP>;
+  struct AEnv : std::vector<DArrayP> {  // of one execution
+    using std::vector<DArrayP>::vector;
+    const Sx* deferred = nullptr;       // a stencil whose sweeps are being counted: yields its operand unchanged
+  };
 
   // preparation
   ATyP prepare(const Sx& n, TEnv& tenv);
