@@ -2152,6 +2152,56 @@ static bool totalScalar(const Sx& e) {
   return true;
 }
 
+// About how many vector instructions one evaluation of a scalar function takes, equal subterms counted once;
+// past `most` the count is not finished.  What functions of nine taps added to a pass of eight sweeps, in units of
+// an addition: a division 12 (8-byte elements 15), a square root 15 (20), exp and log 13 (18), pow 140 (190); sin 33 (54) in
+// time, but its code for large arguments makes kernels of half a megabyte, like that of the others.
+static double scalarWeight(const Sx& e, double most, std::set<std::string>& seen) {
+  if (e.atom) return 0;
+  double w = 0;
+  if (e.is("prim")) {
+    if (!seen.insert(e.str()).second) return 0;
+    const std::string& op = e.at(1).s;
+    const bool typed = e.at(2).atom && op != "land" && op != "lor" && op != "lnot";
+    const ST t = typed ? parseST(e.at(2)) : ST::U8;
+    const bool wide = stSize(t) == 8;
+    auto any = [&](std::initializer_list<const char*> names) {
+      for (const char* n : names)
+        if (op == n) return true;
+      return false;
+    };
+    const Sx& arg = e.at(e.size() - 1);
+    const bool byConst = arg.is("pair") && (arg.at(1).is("const") || arg.at(2).is("const"));
+    w = 1;
+    if (any({"fdiv", "recip"})) w = wide ? 15 : 12;
+    else if (op == "sqrt") w = wide ? 20 : 15;
+    else if (any({"exp", "log"})) w = wide ? 18 : 13;
+    else if (op == "logbase") w = wide ? 51 : 38;
+    else if (any({"fpow", "sin", "cos", "tan", "asin", "acos", "atan", "sinh", "cosh", "tanh", "asinh", "acosh", "atanh", "atan2"})) w = 150;
+    else if (any({"quot", "rem", "idiv", "mod", "quotrem", "divmod"})) w = wide ? 20 : 6;
+    else if (op == "mul" && stIsInt(t)) w = byConst ? (wide ? 1.5 : 1) : wide ? 8 : 4;
+    else if (op == "tofloating" && wide) w = 10;
+  }
+  if (e.is("cond") || e.is("case")) w = 1;
+  for (size_t k = 0; k < e.size() && w <= most; ++k) w += scalarWeight(e.at(k), most - w, seen);
+  return w;
+}
+
+// Several sweeps a pass save memory traffic and launches, and pay with margins computed twice and with few waves, each
+// doing everything in turn: the heavier the function, the less is left.  Single launches / passes, us a sweep over
+// 100^2, 2000^2 and 8000^2: Float32 of 17 operations 5.4 / 3.0, 10.0 / 7.4, 104 / 42; of 30 5.2 / 3.3, 10.3 / 9.1, 102 / 63; of 40
+// 5.2 / 5.6, 11.4 / 15.2, 120 / 86; of 49 (25 taps) 6.5 / 7.5, 13.5 / 16.0, 123 / 104; four exp 5.2 / 9.0, 14.0 / 21.9,
+// 135 / 126; two pow 9 / 45, 34 / 100, 415 / 602.  Float64 of 49 6.9 / 6.6, 19.5 / 19.3, 216 / 176; of 136 6.2 / 10.1, 29.6 /
+// 39.6, 352 / 330 (a kernel that takes 7 s to compile).  So: up to `sweepLight` always; up to `sweepMost` where a
+// sweep's operand and result are more than the last-level cache holds (4000^2 Float32, 64 MB, is level, 5600^2 gains 1.04 - 1.26,
+// 2800^2 Float64, 63 MB, 0.91 - 1.35, 4000^2 1.0 - 1.8); no kernel beyond.
+static double sweepLight(const TypeP& elt) { return stSize(elt->st) == 4 ? 32 : 50; }
+static double sweepMost(const TypeP& elt) { return stSize(elt->st) == 4 ? 56 : 64; }
+static double sweepWeight(const TypeP& elt, const Sx& f) {
+  std::set<std::string> seen;
+  return scalarWeight(f, sweepMost(elt), seen);
+}
+
 // Can several sweeps be computed in one pass?  (A boundary `function` has its values depend on the
 // position, which the marching wave would have to carry: left out.)
 bool Codegen::stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const ArrayR& src) {
@@ -2162,7 +2212,7 @@ bool Codegen::stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx&
   if (kind != "clamp" && kind != "mirror" && kind != "wrap" && kind != "constant") return false;
   if (kind == "constant" && !totalScalar(bnd.at(1))) return false;
   const std::vector<int> halo = stencilHaloOf(pattern);
-  return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && totalScalar(f);
+  return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && totalScalar(f) && sweepWeight(outElt, f) <= sweepMost(outElt);
 }
 
 KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& bnd, const Operand& src) {
@@ -2212,6 +2262,7 @@ KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const S
   KernelSource ks = finish(body, elt, typeLeaves(elt), "stencil2d_sweeps.hpp", v, true);
   ks.group = most;
   ks.words = hx * 16 + hy;
+  ks.sweepLeast = sweepWeight(elt, f) <= sweepLight(elt) ? 0 : (int64_t)96 << 20;
   return ks;
 }
 

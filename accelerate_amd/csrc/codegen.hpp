@@ -69,6 +69,7 @@ struct KernelSource {
   std::string pipeSlot;               // pipelined scan only: name of the array slot its loads move
   int rowsGroup = 1;                  // scan only: groups per wave of acc_scan_rows (small-tile variant)
   int allGroup = 0;                   // scan only: groups per wave of acc_scan_all (twice as many in acc_scan_all2); small-tile variant
+  int64_t sweepLeast = 0;             // several sweeps only: bytes an array has to have for them to be taken together
   std::string permuteMode;            // permute only: "atomic", "cas", "lock", "store"
   bool permuteCount = false;          // permute only: has acc_permute_count (sum of a constant per source)
   bool permuteCountSet = false;       // permute only: has count_set (defaults of one constant, written with the counts)

@@ -1194,8 +1194,10 @@ static AValP withComponent(const AValP& x, const std::string& path, const DArray
 AValP Program::evalSweeps(const Sx& n, const Sweep& sw, AEnv& aenv, AValP x) {
   const Sx &cond = n.at(1), &body = n.at(2);
   const std::vector<int64_t>& ext = componentAt(x, sw.path)->shape;
-  // the kernel's index arithmetic is 32 bits wide, and a strip's margins fold back once at most
-  if (ext[0] < 32 || ext[1] < 32 || ext[0] > (1 << 30) || ext[1] > (1 << 30)) {
+  // the kernel's index arithmetic is 32 bits wide, and a strip's margins fold back once at most; a heavy function
+  // gains on large arrays only (a knob that sets the number of waves asks for the kernel all the same)
+  const bool small = ctx_.knobs.stencil_sweeps <= 1 && arrayBytes(*componentAt(x, sw.path)) < sw.k->meta.sweepLeast;
+  if (small || ext[0] < 32 || ext[1] < 32 || ext[0] > (1 << 30) || ext[1] > (1 << 30)) {
     while (awhileTest(cond, aenv, x)) x = evalFun(body, aenv, {x});
     return x;
   }

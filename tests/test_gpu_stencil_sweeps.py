@@ -265,3 +265,57 @@ def test_patterns_of_one_row_or_column(gpu_ctx, knobs, ty, npty, widths, kind):
             cnt = gpu_ctx.to_device(np.array(n, np.int64), A.tarray(0, Int))
             got, want = fused.execute(g, cnt).to_host(), single.execute(g, cnt).to_host()
             assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (shape, n)
+
+
+def _chain(ty, name, n):
+    """`n` calls, one of the other's result, after the sum of the nine taps"""
+    def fn(t):
+        acc = t[0]
+        for x in t[1:]:
+            acc = A.add(ty, acc, x)
+        for k in range(n):
+            acc = A.prim(name, ty, A.pair(acc, t[k]) if name in ("fpow", "atan2") else acc)
+        return acc
+    return fn
+
+
+def test_heavy_functions_are_left_alone(cc_ctx):
+    for ty in (A.f32, A.f64):
+        for fn, kernel in [(_chain(ty, "abs", 16), True), (_chain(ty, "exp", 1), True), (_chain(ty, "sqrt", 2), True), (_chain(ty, "exp", 4), False),
+                           (_chain(ty, "fpow", 1), False), (_chain(ty, "sin", 1), False), (_chain(ty, "recip", 7), False)]:
+            on, off = _kernels(cc_ctx, fixed_sweeps(lambda: _nine(ty, fn), ty, 9), "stencil_sweeps", 1)
+            assert len(on) - len(off) == (1 if kernel else 0)
+    # equal subterms count once
+    fn = lambda t: A.add(A.f32, *[A.mul(A.f32, *[_chain(A.f32, "exp", 1)(t)] * 2)] * 2)
+    on, off = _kernels(cc_ctx, fixed_sweeps(lambda: _nine(A.f32, fn), A.f32, 9), "stencil_sweeps", 1)
+    assert len(on) == len(off) + 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", BOUNDARIES)
+@pytest.mark.parametrize("ty,npty", [(A.f32, np.float32), (A.i64, np.int64)], ids=["f32", "i64"])
+def test_functions_of_25_taps_on_small_arrays(gpu_ctx, knobs, ty, npty, kind):
+    # one launch a sweep on arrays of this size; a number of waves asks for the kernel all the same
+    step = lambda: Q.stencil_weighted(ty, (5, 5), _boundary(kind, ty))
+    fused, single = _both(gpu_ctx, knobs, fixed_sweeps(step, ty, 13))
+    for k, shape in enumerate(SHAPES):
+        g = gpu_ctx.to_device(_grid(shape, npty, k), A.tarray(2, ty))
+        want = single.execute(g).to_host()
+        for waves, launches in [(1, 13), (3072, 4)]:          # 4 + 4 + 4 + 1
+            knobs("stencil_sweeps", waves)
+            before = gpu_ctx.stat("launches")
+            got = fused.execute(g).to_host()
+            assert gpu_ctx.stat("launches") - before == launches
+            assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (shape, waves)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,launches", [(5000, 9), (5040, 3)])
+def test_functions_of_25_taps_on_large_arrays(gpu_ctx, knobs, rows, launches):
+    # 96 MiB are 5033.2 rows of 5000 Float32
+    fused, single = _both(gpu_ctx, knobs, fixed_sweeps(lambda: Q.stencil_weighted(A.f32, (5, 5), A.clamp), A.f32, 9))
+    g = gpu_ctx.to_device(np.random.default_rng(8).uniform(-1, 1, (rows, 5000)).astype(np.float32), A.tarray(2, A.f32))
+    before = gpu_ctx.stat("launches")
+    got = fused.execute(g)
+    assert gpu_ctx.stat("launches") - before == launches
+    assert np.array_equal(got.to_host(), single.execute(g).to_host())
