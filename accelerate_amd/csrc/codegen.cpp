@@ -2278,19 +2278,20 @@ bool Codegen::stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& 
   return halo.size() == 3 && halo[0] == 1 && halo[1] == 1 && halo[2] <= 1 && totalScalar(f);
 }
 
-KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src, int& taps) {
+KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src) {
   const std::vector<int> halo = stencilHaloOf(pattern);
   const std::string kind = bnd.atom ? bnd.s : bnd.head();
   const TypeP elt = src.r.elt;
   const std::string E = stName(elt->st);
   // Two columns a lane, four rows of 4-byte elements, two of 8-byte ones.  (columns, rows), smoothing with 27
   // taps, 401 x 387 x 393 / 512^3 / 200^3 in us: Float32 (2, 4) 162 / 323 / 24, (4, 4) 200 / 584 / 32, (4, 2) 206 / 563 / 30,
-  // (2, 2) 196 / 375 / 23, (2, 6) 261 / 496 / 33, through LDS 211 / 332 / 35; Float64, launches of two generations of workgroups,
-  // (2, 2) 317 / 586 / 33, (1, 4) 323 / 692 / 31, (2, 4) 323 / 637 / 46, through LDS 346 / 600 / 54.
+  // (2, 2) 196 / 375 / 23, (2, 6) 261 / 496 / 33, through LDS 194 / 332 / 37; Float64, launches of two generations of workgroups,
+  // (2, 2) 318 / 592 / 33, (1, 4) 323 / 692 / 31, (2, 4) 323 / 637 / 46, through LDS 333 / 611 / 57.
   const int v = 2;
   const int rows = stSize(elt->st) == 4 ? 4 : 2;
   const ArraySlot& slot = slotByName(src.slot);
   std::string body;
+  int taps = 0;
   body += "  typedef " + E + " E;\n  static constexpr int R = " + std::to_string(rows) + ";\n";
   const char* names[3] = {"HZ", "HY", "HX"};
   for (int k = 0; k < 3; ++k) body += std::string("  static constexpr int ") + names[k] + " = " + std::to_string(halo[k]) + ";\n";
@@ -2336,7 +2337,6 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
     if (!typeEq(valType(r), outElt)) throw Error("stencil: function result does not match the declared element type");
     const std::string code = returnElt(r, em), used = code.substr(bound);
     // (names are v and a number: one occurrence that no further digit follows is enough)
-    taps = 0;
     for (const std::string& nm : names3)
       for (size_t at = used.find(nm); at != std::string::npos; at = used.find(nm, at + 1))
         if (at + nm.size() >= used.size() || !std::isdigit((unsigned char)used[at + nm.size()])) {
@@ -2347,6 +2347,9 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
   }
   KernelSource ks = finish(body, outElt, typeLeaves(outElt), "stencil3d_rows.hpp", v);
   ks.group = rows;
+  ks.words = halo[2];
+  ks.taps = taps;
+  ks.moved = stSize(elt->st) + stSize(outElt->st);
   return ks;
 }
 

@@ -70,6 +70,7 @@ struct KernelSource {
   int rowsGroup = 1;                  // scan only: groups per wave of acc_scan_rows (small-tile variant)
   int allGroup = 0;                   // scan only: groups per wave of acc_scan_all (twice as many in acc_scan_all2); small-tile variant
   int64_t sweepLeast = 0;             // several sweeps only: bytes an array has to have for them to be taken together
+  int taps = 0, moved = 0;            // rank-3 stencils from registers only: taps the function reads, bytes of an element and its result
   std::string permuteMode;            // permute only: "atomic", "cas", "lock", "store"
   bool permuteCount = false;          // permute only: has acc_permute_count (sum of a constant per source)
   bool permuteCountSet = false;       // permute only: has count_set (defaults of one constant, written with the counts)
@@ -114,8 +115,8 @@ class Codegen {
   // stencilSweepable holds
   KernelSource stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& boundary, const Operand& src);
   static bool stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const ArrayR& src);
-  // rank 3 from registers (stencil3d_rows.hpp); only where stencilRowsable holds.  taps: how many the function reads
-  KernelSource stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src, int& taps);
+  // rank 3 from registers (stencil3d_rows.hpp); only where stencilRowsable holds
+  KernelSource stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   static bool stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource scalarKernel(const Sx& exp);  // evaluates a closed Exp with one thread
 

@@ -1,14 +1,14 @@
 // Rank-3 stencils of many taps (stencilOp, Interpreter.hs:637-649), from registers.
 //
 // Through LDS (stencil3d.hpp) every tap of every result is a read of its own, and its product
-// with a weight is computed anew: 27 taps on 401 x 387 x 393 Float32 take 211 us, bound by the vector
-// units and LDS, where the traffic needs 76 us.  Here a wave owns a strip of 64 * V columns and a
+// with a weight is computed anew: smoothing with 27 taps, 401 x 387 x 393 Float32, takes 194 us, where the traffic needs
+// 76, and 7 taps take 141.  Here a wave owns a strip of 64 * V columns and a
 // band of R rows and marches through the planes with the window of three planes by R + 2 * HY rows in
 // registers: a row is loaded V values a lane, its left and right neighbours come from the
 // next lanes by wave shifts, and what two results share (a loaded value, a product) is computed once, within
-// the band and within the three planes one turn of the loop covers.  162 us, half the time on small volumes
-// (200^3 35 -> 24); few taps are better off through LDS, which moves the data at 4.7 TB/s where the bands, which
-// each load their neighbours' border rows again, reach 3.2.  (A wave that marches down the rows of one plane
+// the band and within the three planes one turn of the loop covers.  162 us (7 taps 174), 24 instead of 37 on 200^3,
+// 323 instead of 332 on 512^3: bound by loads, of which the bands' border rows come again for every neighbour, so
+// it wins most where they come from the cache (the host chooses, see there).  (A wave that marches down the rows of one plane
 // with the planes around it loads everything three times: 198 - 317 us.)
 //
 // Outside the array a tap is replaced as `bounded` says (Interpreter.hs:797-839): columns and rows

@@ -785,24 +785,18 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
       plan.k = ctx_.kernel(cg.stencil2d(pats[0], outElt, *f, bnds[0], srcs[0]));
       plan.mode = "lds2d";
     } else if (!two && srcs[0].r.rank == 3 && !ctx_.knobs.stencil_no3d) {
-      KernelSource lds = cg.stencil3d(pats[0], outElt, *f, bnds[0], srcs[0]);
+      plan.k = ctx_.kernel(cg.stencil3d(pats[0], outElt, *f, bnds[0], srcs[0]));
       plan.mode = "lds3d";
       if (ctx_.knobs.stencil_rows3d && Codegen::stencilRowsable(pats[0], outElt, *f, bnds[0], srcs[0])) {
         Codegen cgr(aenvOf(tenv));
         Plan scratch;
         Operand src = operandOf(n.at(5), cgr, tenv, scratch);
-        int taps = 0;
-        KernelSource rows = cgr.stencil3dRows(pats[0], outElt, *f, bnds[0], src, taps);
-        // Through LDS the time grows with the taps (7 / 27 of them, 401 x 387 x 393: Float32 138 / 211 us, Float64
-        // 250 / 346), from registers it hardly does (152 / 162, 301 / 317): the lines lie where the two meet.
+        KernelSource rows = cgr.stencil3dRows(pats[0], outElt, *f, bnds[0], src);
+        // From registers where many taps are read: 200^3, 7 / 13 / 17 / 27 taps, Float32 1.02 / 1.17 / 1.27 / 1.37 times as fast
+        // as through LDS, Float64 1.22 / 1.49 / 1.52 / 1.56.  At a launch rowsPay chooses between the two by the extents.
         const long long least = ctx_.knobs.stencil_rows3d > 1 ? 1 : stSize(srcs[0].r.elt->st) == 4 ? 16 : 25;
-        if (taps >= least) {
-          plan.k = ctx_.kernel(rows);
-          plan.wide = std::make_shared<KernelSource>(std::move(lds));
-          plan.mode = "rows3d";
-        }
+        if (rows.taps >= least) plan.k2 = ctx_.kernel(rows);
       }
-      if (!plan.k) plan.k = ctx_.kernel(lds);
     } else {
       plan.k = ctx_.kernel(cg.stencil(pats, outElt, *f, bnds, srcs));
     }
@@ -1254,6 +1248,27 @@ DArrayP Program::launchSweeps(const Sweep& sw, DArrayP g, int64_t count) {
     count -= T;
   }
   return g;
+}
+
+// Does a rank-3 stencil of many taps go faster from registers (acc_stencil3d_rows) than through LDS on these extents?
+// From registers the time hardly depends on the taps, but every band loads its neighbours' border rows again: while operand
+// and result stay in the last-level cache it wins for every shape (16 million Float32 of 256 x 250 .. 1024 columns, 17 taps, 1.12 -
+// 1.78 times as fast, 27 taps 1.15 - 1.91; 200^3 1.27 / 1.37).  From memory LDS moves the data faster, and wins
+// for few taps (Float32 512^3, 17 / 19 / 23 / 25 / 27 taps 0.79 / 0.81 / 0.89 / 0.91 / 0.95 times as fast from registers,
+// 128 x 1024 x 1024 0.72 .. 0.85, 401 x 387 x 393 0.89 / 0.93 / 1.00 / 1.03 / 1.09) unless its tiles of 128 columns are
+// badly filled (640 x 512 x 300 1.14 .. 1.30, 1000 x 1000 x 100 1.51 .. 1.68).  In between, 33 to 67 million Float32, twice that for 8-byte elements,
+// which are bound less by the vector units: 23 taps 0.97 - 1.37 where the strips are filled to 0.7 and more (17 taps 0.82 - 1.25), 0.82 - 0.95 in 250
+// and 256 columns, of whose strips a third is empty; Float64 400^3, 25 / 27 taps 1.12 / 1.20, 500^3 0.90 / 0.98.
+static bool rowsPay(const KernelSource& rows, long long knob, const std::vector<int64_t>& ext) {
+  // (the kernel's index arithmetic is 32 bits wide)
+  if (knob == 0 || ext[0] >= (1 << 30) || ext[1] >= (1 << 30) || ext[2] >= (1 << 30)) return false;
+  if (knob > 1) return true;
+  const int64_t w = ext[2], hx = rows.words, v = rows.vec, cols = 64 * v - 2 * ((hx + v - 1) / v * v);  // kCols
+  auto fill = [&](int64_t own, int64_t of) { return (double)w / (double)((w + own - 1) / own * of); };
+  const int64_t mib = ext[0] * ext[1] * w * rows.moved >> 20;  // operand and result
+  if (mib <= 192) return true;
+  if (mib <= (rows.moved < 16 ? 512 : 1024)) return rows.taps >= 23 && fill(cols, 64 * v) >= 0.7;
+  return rows.taps >= 25 && fill(128, 128) < 0.8;
 }
 
 AValP Program::eval(const Sx& n, AEnv& aenv) {
@@ -1810,34 +1825,28 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       ctx_.launch(plan.k, "acc_stencil2d", (uint64_t)(tilesX * chunksY), 256, args);
       return avArr(out);
     }
-    const bool wide3d = plan.mode == "rows3d" && (ext[0] >= (1 << 30) || ext[1] >= (1 << 30) || ext[2] >= (1 << 30));
-    if (plan.mode == "rows3d" && !wide3d) {
+    if (plan.mode == "lds3d" && plan.k2 && rowsPay(plan.k2->meta, ctx_.knobs.stencil_rows3d, ext)) {
       if (out->size() == 0) return avArr(out);
-      const int64_t v = plan.k->meta.vec, hx = stencilHaloOf(n.at(1))[2];
+      const int64_t v = plan.k2->meta.vec, hx = plan.k2->meta.words;
       const int64_t cols = 64 * v - 2 * ((hx + v - 1) / v * v);  // kCols
-      const int64_t strips = (ext[2] + cols - 1) / cols, r = plan.k->meta.group;
+      const int64_t strips = (ext[2] + cols - 1) / cols, r = plan.k2->meta.group;
       const int64_t bands = ((ext[1] + r - 1) / r + 3) / 4 * 4, groups = strips * bands / 4;
-      const int64_t resident = std::max<int64_t>(256, ctx_.residentGroups(plan.k, "acc_stencil3d_rows", 256));
+      const int64_t resident = std::max<int64_t>(256, ctx_.residentGroups(plan.k2, "acc_stencil3d_rows", 256));
       // chunks of planes so that the launch fills the device once (twice for 8-byte elements: 512^3 816 -> 586 us)
       const int64_t gens = ctx_.knobs.stencil_chain > 0 ? ctx_.knobs.stencil_chain : r >= 4 ? 1 : 2;
       int64_t chunks = std::max<int64_t>(1, std::min(gens * resident / groups, (ext[0] + 3) / 4));
       const int64_t planes = (ext[0] + chunks - 1) / chunks;
       chunks = (ext[0] + planes - 1) / planes;
       if (groups * chunks > 0x7fffffffLL) throw Error("stencil: too many tiles for one launch");
-      std::vector<uint64_t> args = packArgs(plan.k->meta, aenv, temps, ext);
+      std::vector<uint64_t> args = packArgs(plan.k2->meta, aenv, temps, ext);
       packOut(args, *out);
       for (int64_t a : {ext[0], ext[1], ext[2], strips, bands, chunks, planes}) args.push_back((uint64_t)a);
-      ctx_.launch(plan.k, "acc_stencil3d_rows", (uint64_t)(groups * chunks), 256, args);
+      ctx_.launch(plan.k2, "acc_stencil3d_rows", (uint64_t)(groups * chunks), 256, args);
       return avArr(out);
     }
-    if (plan.mode == "lds3d" || wide3d) {
+    if (plan.mode == "lds3d") {
       if (out->size() == 0) return avArr(out);
-      KernelP k3d = plan.k;
-      if (wide3d) {
-        k3d = ctx_.kernel(*plan.wide);
-        ctx_.wait(k3d);
-      }
-      const int64_t th = k3d->meta.group, tw = k3d->meta.words;
+      const int64_t th = plan.k->meta.group, tw = plan.k->meta.words;
       const int64_t tilesY = (ext[1] + th - 1) / th, tilesX = (ext[2] + tw - 1) / tw;
       // planes per workgroup: long enough to amortise the 2*HZ planes staged before the first
       // result, short enough that the grid fills the device
@@ -1847,13 +1856,13 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       chain = std::max<int64_t>(1, std::min(chain, ext[0]));
       const int64_t chunksZ = (ext[0] + chain - 1) / chain;
       if (tilesX * tilesY * chunksZ > 0x7fffffffLL) throw Error("stencil: too many tiles for one launch");
-      std::vector<uint64_t> args = packArgs(k3d->meta, aenv, temps, ext);
+      std::vector<uint64_t> args = packArgs(plan.k->meta, aenv, temps, ext);
       packOut(args, *out);
       for (int k = 0; k < 3; ++k) args.push_back((uint64_t)ext[k]);
       args.push_back((uint64_t)tilesX);
       args.push_back((uint64_t)tilesY);
       args.push_back((uint64_t)chain);
-      ctx_.launch(k3d, "acc_stencil3d", (uint64_t)(tilesX * tilesY * chunksZ), 256, args);
+      ctx_.launch(plan.k, "acc_stencil3d", (uint64_t)(tilesX * tilesY * chunksZ), 256, args);
       return avArr(out);
     }
     launchMap(plan.k, aenv, temps, *out);

@@ -77,7 +77,6 @@ struct Plan {
   std::map<const Sx*, KernelP> scalarKernels;    // expressions evaluated by a one-thread kernel
   std::map<const Sx*, std::vector<const Sx*>> scalarTemps;
   std::string mode;
-  std::shared_ptr<KernelSource> wide;            // stencils from registers: the kernel for extents beyond 32-bit arithmetic, compiled when one comes
   ATyP ty;                                       // result type of the node
 };
 

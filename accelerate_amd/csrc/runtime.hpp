@@ -65,7 +65,7 @@ struct Knobs {
   long long permute_fresh = 1;      // 0: constant defaults are materialised also where the counting kernels could write them
   long long stencil_chain = 0;      // 0: decide per launch; tiles (rank 2) or planes (rank 3) per workgroup
   long long stencil_sweeps = 1;     // 0: a loop of stencil sweeps computes one at a time; > 1: waves a launch of several sweeps aims at
-  long long stencil_rows3d = 1;     // 1: rank-3 stencils of many taps are computed from registers, 0: never, 2: whatever the taps
+  long long stencil_rows3d = 1;     // 1: rank-3 stencils of many taps are computed from registers where that is faster, 0: never, 2: whatever the taps and extents
   long long stencil_no2d = 0, stencil_no3d = 0;  // 1: rank-2 / rank-3 stencils through the generic skeleton
   long long pool_async = 1;         // 1: device blocks come from the stream-ordered allocator (hipMallocAsync), 0: hipMalloc
   long long scan_tiles = 0;         // 0: decide per launch, 1 large, 2 small, 3 rows, 4 pipelined (where the operand allows), 5 / 6 acc_scan_all / acc_scan_all2

@@ -61,3 +61,36 @@ def test_equal_to_the_lds_kernel(gpu_ctx, knobs, ty, npty, nx, kind, chain):
         got = rows.execute(d).to_host()
         knobs("stencil_chain", 0)
         assert np.array_equal(got, want), shape
+
+
+# Both kernels are compiled; a launch takes the one that is faster on its extents.  Below 192 MiB of operand and
+# result from registers; up to 512 MiB (of 4-byte elements) where strips of 124 columns are filled to 0.7 of 128; beyond, where tiles of 128
+# columns are filled to less than 0.8.
+@pytest.mark.parametrize("shape,taps,rows", [
+    ((6, 8, 124), 27, True), ((200, 200, 200), 19, True), ((290, 295, 300), 19, False), ((290, 295, 300), 27, True),
+    ((500, 256, 256), 27, False), ((512, 512, 512), 27, False), ((640, 400, 300), 27, True)], ids=str)
+def test_the_kernel_a_launch_takes(gpu_ctx, knobs, capfd, shape, taps, rows):
+    row = A.sunit(3, A.f32)
+    sr = A.stup(*[A.stup(row, row, row)] * 3)
+
+    def f(st):
+        ts = [t for p in A.untup(st) for r in A.untup(p) for t in A.untup(r)]
+        acc = ts[13]
+        for k, t in enumerate(ts[:taps - 1]):
+            acc = A.add(A.f32, acc, A.mul(A.f32, A.const(A.f32, 0.01 * (k + 1)), t))
+        return acc if taps < 27 else A.add(A.f32, acc, ts[26])
+
+    prog = gpu_ctx.compile(A.alam([A.tarray(3, A.f32)], lambda g: A.stencil(sr, A.f32, A.lam([A.stencil_type(sr)], f), A.clamp, g)))
+    g = gpu_ctx.to_device(np.random.default_rng(9).random(shape, dtype=np.float32), A.tarray(3, A.f32))
+    got, before = {}, gpu_ctx.flags
+    for knob in (1, 0, 2):
+        knobs("stencil_rows3d", knob)
+        gpu_ctx.flags = before | gpu_ctx.FLAG_DUMP_EXEC
+        capfd.readouterr()
+        try:
+            out = prog.execute(g)
+        finally:
+            gpu_ctx.flags = before
+        assert ("acc_stencil3d_rows" in capfd.readouterr().err) == (knob == 2 or knob == 1 and rows)
+        got[knob] = out.to_host()
+    assert np.array_equal(got[0], got[2]) and np.array_equal(got[0], got[1])
