@@ -1062,7 +1062,20 @@ static int scanBlock() {
   return (v == 256 || v == 512 || v == 1024) ? v : 1024;
 }
 
-KernelSource Codegen::foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType) {
+bool Codegen::foldSegHalves(const Operand& src) {
+  if (!src.delayed || std::getenv("ACCHIP_FOLDSEG_BYTES")) return false;
+  struct R {
+    static bool reads(const Sx& e) {
+      if (e.is("index") || e.is("linearindex")) return true;
+      for (size_t k = 0; !e.atom && k < e.size(); ++k)
+        if (reads(e.at(k))) return true;
+      return false;
+    }
+  };
+  return R::reads(src.linearD);
+}
+
+KernelSource Codegen::foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType, bool half) {
   const TypeP elt = src.r.elt;
   std::string body;
   body += std::string("  static constexpr bool kSeeded = ") + (seed ? "true" : "false") + ";\n";
@@ -1117,11 +1130,7 @@ KernelSource Codegen::foldSeg(const Sx& f, const Sx* seed, const Operand& src, c
   const char* vm = std::getenv("ACCHIP_FOLDSEG_VECMUL");
   vec *= vm ? std::max(1, std::min(4, std::atoi(vm))) : 2;
   const char* fe = std::getenv("ACCHIP_FOLDSEG_BYTES");
-  // A fused producer reads more than the element (indices, what they point at) and waits for one
-  // load behind another: its tiles are half as long, which puts twice as many workgroups under way.
-  // Sparse matrix times vector, 256 / 128 / 64 B: 6.3 million non-zeros Float32 31.1 / 28.3 / 28.1 us, Float64
-  // 37.8 / 33.7 / 34.7, 25 million with columns anywhere 189 / 185 / 187, 0.6 million 19.9 / 18.2 / 18.3.
-  const int dflt = src.delayed ? 128 : 256;
+  const int dflt = half ? 128 : 256;  // (a launch takes the one that is faster for its values)
   int fbytes = fe ? std::atoi(fe) : dflt;
   if (fbytes < 16 || fbytes > 512) fbytes = dflt;
   int g = std::max(1, std::min(8, fbytes / std::max(1, vec * eltBytes)));

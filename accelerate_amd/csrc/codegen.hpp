@@ -102,7 +102,9 @@ class Codegen {
   KernelSource scan(const Sx& f, const Sx* seed, const Operand& src, bool right, int kind, int variant = 0,
                     const Sx* post = nullptr, const TypeP& postElt = nullptr);
   static bool scanPipeable(const Operand& src, bool right);
-  KernelSource foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType);
+  // half: tiles of half the length, for fused producers that read arrays (foldSegHalves) and not too many values
+  KernelSource foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType, bool half);
+  static bool foldSegHalves(const Operand& src);
   // freshInit: the literal every element of the defaults holds when they are `generate sh (\_ -> c)`
   // (the counting variant can then write defaults and counts together), else null
   KernelSource permute(const Sx& f, const ArrayR& dst, const Sx& p, const Operand& src, const Sx* freshInit = nullptr);

@@ -811,7 +811,13 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
     Operand src = operandOf(n.at(4), cg, tenv, plan);
     Operand seg = operandOf(n.at(5), cg, tenv, plan);
     if (src.r.rank < 1 || seg.r.rank != 1) throw Error("foldSeg: operands have the wrong rank");
-    plan.k = ctx_.kernel(cg.foldSeg(n.at(2), seedOf(n.at(3)), src, seg, ity));
+    plan.k = ctx_.kernel(cg.foldSeg(n.at(2), seedOf(n.at(3)), src, seg, ity, false));
+    if (Codegen::foldSegHalves(src)) {
+      Codegen cgh(aenvOf(tenv));
+      Plan scratch;
+      Operand srcH = operandOf(n.at(4), cgh, tenv, scratch), segH = operandOf(n.at(5), cgh, tenv, scratch);
+      plan.k2 = ctx_.kernel(cgh.foldSeg(n.at(2), seedOf(n.at(3)), srcH, segH, ity, true));
+    }
     return done(src.r);
   }
   if (h == "scan" || h == "scan'") return prepareScan(n, tenv, plan, nullptr, nullptr);
@@ -1269,6 +1275,18 @@ static bool rowsPay(const KernelSource& rows, long long knob, const std::vector<
   if (mib <= 192) return true;
   if (mib <= (rows.moved < 16 ? 512 : 1024)) return rows.taps >= 23 && fill(cols, 64 * v) >= 0.7;
   return rows.taps >= 25 && fill(128, 128) < 0.8;
+}
+
+// Segmented folds over a fused producer that reads arrays: are tiles of half the length (128 B of values and flags a lane) faster?
+// Twice as many workgroups wait for loads behind loads, and a last tile that is not full, whose elements are loaded one by one while the
+// others have finished, holds half as many.  256 B / 128 B, us, segments of 100: a function of one Float32 array 8.29 million
+// 20.8 / 19.5, of two 23.0 / 20.8, sparse matrix times vector 6.3 million 31.1 / 28.3; Float64 8.29 million 28.3 / 25.6.  From 50 million on,
+// both cost: 2^26 Float32 66.7 / 69.9, Float64 132 / 137, 2^27 115 / 128 and 235 / 250 (28 million are at 1.02 - 1.05).
+// Where all tiles of full length are full: 2^22 1.02 - 1.04, 2^23 Float32 16.7 / 18.2, 2^24 0.97 (Float64 2^23 28.3 / 25.5, but 25.6 / 25.5 at a whole
+// number of its tiles).  A producer that reads nothing does not gain (2^23 0.92).
+static bool foldSegHalf(const KernelSource& full, int64_t total) {
+  const int64_t tile = (int64_t)full.block * full.group * full.vec;
+  return total <= (int64_t)3 << 23 && (total < (int64_t)3 << 21 || total % tile != 0);
 }
 
 AValP Program::eval(const Sx& n, AEnv& aenv) {
@@ -1881,9 +1899,10 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     oshape.push_back(nseg);
     DArrayP out = alloc(plan.ty->r, oshape);
     if (rows == 0 || nseg == 0) return avArr(out);
-    const KernelSource& m = plan.k->meta;
-    const int64_t tile = (int64_t)m.block * m.group * m.vec;
     const int64_t total = rows * len;
+    const KernelP& kern = plan.k2 && foldSegHalf(plan.k->meta, total) ? plan.k2 : plan.k;
+    const KernelSource& m = kern->meta;
+    const int64_t tile = (int64_t)m.block * m.group * m.vec;
     const int64_t tiles = std::max<int64_t>(1, (total + tile - 1) / tile);
     if (tiles > 0x7f000000LL) throw Error("foldSeg: too many tiles for one launch");
     ArrayR pr;
@@ -1907,14 +1926,14 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
     const int64_t boundaries = rows * (nseg + 1);
     if ((boundaries + 255) / 256 > 0x7fffffffLL) throw Error("foldSeg: too many segments for one launch");
-    ctx_.launch(plan.k, "acc_foldseg_partition", (uint64_t)((boundaries + 255) / 256), 256, args);
+    ctx_.launch(kern, "acc_foldseg_partition", (uint64_t)((boundaries + 255) / 256), 256, args);
     // behind the tiles, the workgroups that complete the segment ends reaching across tile borders
     const uint64_t fixGroups = (uint64_t)((tiles + m.block - 1) / m.block);
     if (ctx_.knobs.foldseg_one_launch != 0) {
-      ctx_.launch(plan.k, "acc_foldseg", (uint64_t)tiles + fixGroups, (unsigned)m.block, args);
+      ctx_.launch(kern, "acc_foldseg", (uint64_t)tiles + fixGroups, (unsigned)m.block, args);
     } else {
-      ctx_.launch(plan.k, "acc_foldseg", (uint64_t)tiles, (unsigned)m.block, args);
-      ctx_.launch(plan.k, "acc_foldseg_fixup", fixGroups, (unsigned)m.block, args);
+      ctx_.launch(kern, "acc_foldseg", (uint64_t)tiles, (unsigned)m.block, args);
+      ctx_.launch(kern, "acc_foldseg_fixup", fixGroups, (unsigned)m.block, args);
     }
     return avArr(out);
   }
