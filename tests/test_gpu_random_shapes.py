@@ -45,7 +45,7 @@ def _shape(rng, most=MOST):
 
 
 _last = A.lam([I64, I64], lambda p, q: A.cond(A.neq(I64, q, A.constI(0)), q, p))
-KNOBS = {"scan_tiles": [0, 0, 0, 1, 2, 3, 4], "fold_rows": [-1, -1, -1, 0, 1, 2], "scan_ticketless": [1, 1, 0],
+KNOBS = {"scan_tiles": [0, 0, 0, 1, 2, 3, 4, 5, 6], "fold_rows": [-1, -1, -1, 0, 1, 2], "scan_ticketless": [1, 1, 0],
          "fold_staged": [1, 1, 0], "fold_one_launch": [1, 1, 0], "fold_target": [2048, 2048, 64, 7]}
 
 

@@ -76,3 +76,25 @@ def test_wide_elements(gpu_ctx, knobs):
             got = run.execute(gpu_ctx.to_device(a, A.tarray(1, A.i32)), gpu_ctx.to_device(b, A.tarray(1, A.i64))).to_host()
             for g, w in zip(got, (np.cumsum(a, dtype=np.int32), np.cumsum(b))):
                 assert np.array_equal(np.asarray(g), w), (which, n)
+
+
+@pytest.mark.parametrize("which", [5, 6])
+@pytest.mark.parametrize("d", ["l", "r"])
+@pytest.mark.parametrize("ty,npty,size", [(A.i32, np.int32, 4), (A.i64, np.int64, 8)], ids=["i32", "i64"])
+def test_every_kind_over_rows(gpu_ctx, knobs, ty, npty, size, d, which):
+    # a tile belongs to one row; rows that end in, just before and just after a tile's last value
+    tile = 256 * 64 // size * (which - 4)
+    progs = [gpu_ctx.compile(p) for p in (P.scan1_sum(d, ty, 2), P.scan_sum(d, ty, 2, 5), P.scan_prime_sum(d, ty, 2, 3))]
+    knobs("scan_tiles", which)
+    rng = np.random.default_rng(12)
+    for rows, n in [(2, tile // 2 + 3), (5, tile - 1), (3, tile), (4, tile + 1), (7, 2 * tile + 5), (2, 65 * tile + 1), (3, 66 * tile - 3)]:
+        x = rng.integers(-1000, 1000, (rows, n)).astype(npty)
+        inc = _running(x, d == "r")
+        none = np.zeros((rows, 1), npty)
+        with_seed = np.concatenate([inc, none] if d == "r" else [none, inc], axis=1)
+        dx = gpu_ctx.to_device(x, A.tarray(2, ty))
+        assert np.array_equal(progs[0].execute(dx).to_host(), inc), (rows, n)
+        assert np.array_equal(progs[1].execute(dx).to_host(), 5 + with_seed), (rows, n)
+        body, total = [p.to_host() for p in progs[2].execute(dx).parts()]
+        assert np.array_equal(body, 3 + (with_seed[:, 1:] if d == "r" else with_seed[:, :-1])), (rows, n)
+        assert np.array_equal(total, 3 + inc[:, 0 if d == "r" else -1]), (rows, n)
