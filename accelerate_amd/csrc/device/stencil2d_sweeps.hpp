@@ -10,9 +10,10 @@
 // wave shifts.  What a wave lacks beyond its strip it recomputes: a strip gives 64 * V - 2 * T * HX
 // (rounded to V) columns, a chunk of rows starts and ends T * HY rows early and late.
 //
-// Measured (Jacobi, 8192 x 8192): Float32 90 us a sweep with a launch for each, 15.6 us in passes of 8
-// (125 us a pass: 4.3 TB/s, and 60 % of what the vector units can issue); a pass of 4 takes 131 us, so 8 it is where
-// registers allow (146 of them, 3 waves a SIMD; halos of 2 take 4).  Float64 30 us a sweep.  All waves
+// Measured (Jacobi, 8192 x 8192): Float32 90 us a sweep with a launch for each, 15.6 us in passes of 8.  A pass of
+// 8 takes 118 - 125 us: its 61 million vector instructions are issued in 92 % of the busy cycles.  A pass of 4 has half as many
+// and takes 118 - 123 us, for which 572 MiB (operand and result 512) come and go at 5.1 TB/s, so 8 it is where registers
+// allow (146 of them, 3 waves a SIMD; halos of 2 take 4).  Float64 30 us a sweep.  All waves
 // of a launch are resident at once: with 3072 of them 15.7 us a sweep, 2048 16.0, 1024 22.3, 4096, a second generation, 18.0.
 //
 // Boundary conditions hold in every sweep: a tap outside the array is replaced from the same

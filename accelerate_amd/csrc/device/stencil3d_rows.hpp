@@ -1,7 +1,7 @@
 // Rank-3 stencils of many taps (stencilOp, Interpreter.hs:637-649), from registers.
 //
 // Through LDS (stencil3d.hpp) every tap of every result is a read of its own, and its product
-// with a weight is computed anew: smoothing with 27 taps, 401 x 387 x 393 Float32, takes 194 us, where the traffic needs
+// with a weight is computed anew: smoothing with 27 taps, 401 x 387 x 393 Float32, keeps the vector units busy for 91 % of 194 us, where the traffic needs
 // 76, and 7 taps take 141.  Here a wave owns a strip of 64 * V columns and a
 // band of R rows and marches through the planes with the window of three planes by R + 2 * HY rows in
 // registers: a row is loaded V values a lane, its left and right neighbours come from the

@@ -127,7 +127,10 @@ int acchip_set_clean_hook(acchip_ctx* ctx, acchip_clean_fn fn, void* user);
  * ...: the name in capitals), and changed afterwards only here.  Names: stream_bytes,
  * map_max_blocks, map_tiled, fold_rows, fold_target, fold_max_blocks, permute_parts, permute_count, permute_groups,
  * permute_partials, permute_fresh, stencil_chain, stencil_no2d, stencil_no3d (these two take effect for programs
- * compiled afterwards), scan_tiles (0 automatic, 1 large, 2 small, 3 rows, 4 pipelined), scan_spin_limit,
+ * compiled afterwards), stencil_sweeps (0: a loop of stencil sweeps computes one at a time, for programs compiled afterwards;
+ * above 1: waves a launch of several sweeps aims at), stencil_rows3d (rank-3 stencils from registers, 0: never, 1: where that is
+ * faster, 2: whatever the taps and extents; for programs compiled afterwards, and at a launch where a program holds both kernels),
+ * scan_tiles (0 automatic, 1 large, 2 small, 3 rows, 4 pipelined, 5 / 6 small tiles of 64 / 128 bytes a lane), scan_spin_limit,
  * scan_test_skew, scan_ticketless (0: the tiles of a scan always take their numbers from the counter),
  * scan_post (0: the function of a map around a scan is never applied by the scan itself; read by acchip_compile),
  * fold_staged (0: folds under operators that are not commutative never stage blocks of tiles in LDS),
