@@ -2224,16 +2224,37 @@ bool Codegen::stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx&
   return halo.size() == 2 && halo[0] <= 2 && halo[1] <= 2 && totalScalar(f) && sweepWeight(outElt, f) <= sweepMost(outElt);
 }
 
+// does generated code mention a name?  (names are v and a number: one occurrence that no further digit follows is enough)
+static bool mentions(const std::string& code, const std::string& name) {
+  for (size_t at = code.find(name); at != std::string::npos; at = code.find(name, at + 1))
+    if (at + name.size() >= code.size() || !std::isdigit((unsigned char)code[at + name.size()])) return true;
+  return false;
+}
+
+// a function whose only operations are additions, subtractions, multiplications and negations of Float32 or Float64
+static bool plainFloat(const Sx& e) {
+  if (e.atom) return true;
+  if (e.is("cond") || e.is("case") || e.is("coerce")) return false;
+  if (e.is("prim")) {
+    const std::string& op = e.at(1).s;
+    if (op != "add" && op != "sub" && op != "mul" && op != "neg") return false;
+    const ST t = parseST(e.at(2));
+    if (t != ST::F32 && t != ST::F64) return false;
+  }
+  for (size_t k = 0; k < e.size(); ++k)
+    if (!plainFloat(e.at(k))) return false;
+  return true;
+}
+
 KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const Sx& f, const Sx& bnd, const Operand& src) {
   const std::vector<int> halo = stencilHaloOf(pattern);
   const int hy = halo[0], hx = halo[1];
   const std::string kind = bnd.atom ? bnd.s : bnd.head();
   const std::string E = stName(elt->st);
   const int v = 16 / stSize(elt->st);  // a lane moves 16 bytes of a row
-  const int most = hy <= 1 && hx <= 1 ? 8 : 4;
   const ArraySlot& slot = slotByName(src.slot);
   std::string body;
-  body += "#define ACC_SW_MAX " + std::to_string(most) + "\n";
+  int most;
   body += "  typedef " + E + " E;\n";
   body += "  static constexpr int HY = " + std::to_string(hy) + ";\n  static constexpr int HX = " + std::to_string(hx) + ";\n";
   body += "  static constexpr int BOUNDARY = " + std::string(kind == "clamp" ? "0" : kind == "mirror" ? "1" : kind == "wrap" ? "2" : "3") + ";\n";
@@ -2254,19 +2275,32 @@ KernelSource Codegen::stencilSweeps(const Sx& pattern, const TypeP& elt, const S
     Emit em;
     em.ind = 4;
     const int k0 = stencilWidth(pattern) / 2;
+    std::vector<std::pair<std::string, int>> sides;  // taps beside the focus' column, and their rows
     ValP arg = vUnit();
     for (int dy = -k0; dy <= k0; ++dy) {
       const Sx& row = pattern.at(1 + dy + k0);
       if (row.head().compare(0, 4, "unit") != 0) throw Error("stencil2d: pattern is not of rank 2");
       const int k1 = stencilWidth(row) / 2;
       ValP rv = vUnit();
-      for (int dx = -k1; dx <= k1; ++dx)
-        rv = vPair(rv, bindLeaf(elt->st, "w[" + std::to_string(hy + dy) + "].e[k + " + std::to_string(hx + dx) + "]", em));
+      for (int dx = -k1; dx <= k1; ++dx) {
+        ValP t = bindLeaf(elt->st, "w[" + std::to_string(hy + dy) + "].e[k + " + std::to_string(hx + dx) + "]", em);
+        if (dx != 0) sides.push_back({t->ex, dy});
+        rv = vPair(rv, t);
+      }
       arg = vPair(arg, rv);
     }
+    const size_t bound = em.code.size();
     ValP r = applyFun(f, {arg}, {}, em);
     if (!typeEq(valType(r), elt)) throw Error("stencil: function result does not match the declared element type");
-    body += "  template <class W>\n" + fnHead("Elt", "apply_win", "const Env& env, const W& w, const int k") + returnElt(r, em) + "  }\n";
+    const std::string code = returnElt(r, em), used = code.substr(bound);
+    std::set<int> sideRows;
+    for (const auto& s : sides)
+      if (mentions(used, s.first)) sideRows.insert(s.second);
+    const bool late = sideRows.size() <= 1 && plainFloat(f);
+    most = hy > 1 || hx > 1 ? 4 : late ? 10 : 8;
+    body += "#define ACC_SW_MAX " + std::to_string(most) + "\n";
+    body += "  static constexpr bool LATE = " + std::string(late ? "true" : "false") + ";\n";
+    body += "  template <class W>\n" + fnHead("Elt", "apply_win", "const Env& env, const W& w, const int k") + code + "  }\n";
   }
   KernelSource ks = finish(body, elt, typeLeaves(elt), "stencil2d_sweeps.hpp", v, true);
   ks.group = most;
@@ -2345,13 +2379,7 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
     ValP r = applyFun(f, {arg}, {}, em);
     if (!typeEq(valType(r), outElt)) throw Error("stencil: function result does not match the declared element type");
     const std::string code = returnElt(r, em), used = code.substr(bound);
-    // (names are v and a number: one occurrence that no further digit follows is enough)
-    for (const std::string& nm : names3)
-      for (size_t at = used.find(nm); at != std::string::npos; at = used.find(nm, at + 1))
-        if (at + nm.size() >= used.size() || !std::isdigit((unsigned char)used[at + nm.size()])) {
-          ++taps;
-          break;
-        }
+    for (const std::string& nm : names3) taps += mentions(used, nm);
     body += "  template <class W>\n" + fnHead("Elt", "apply_win", "const Env& env, const W& w, const int b, const int k") + code + "  }\n";
   }
   KernelSource ks = finish(body, outElt, typeLeaves(outElt), "stencil3d_rows.hpp", v);

@@ -10,11 +10,15 @@
 // wave shifts.  What a wave lacks beyond its strip it recomputes: a strip gives 64 * V - 2 * T * HX
 // (rounded to V) columns, a chunk of rows starts and ends T * HY rows early and late.
 //
-// Measured (Jacobi, 8192 x 8192): Float32 90 us a sweep with a launch for each, 15.6 us in passes of 8.  A pass of
-// 8 takes 118 - 125 us: its 61 million vector instructions are issued in 92 % of the busy cycles.  A pass of 4 has half as many
-// and takes 118 - 123 us, for which 572 MiB (operand and result 512) come and go at 5.1 TB/s, so 8 it is where registers
-// allow (146 of them, 3 waves a SIMD; halos of 2 take 4).  Float64 30 us a sweep.  All waves
-// of a launch are resident at once: with 3072 of them 15.7 us a sweep, 2048 16.0, 1024 22.3, 4096, a second generation, 18.0.
+// Measured (Jacobi, 8192 x 8192): Float32 90 us a sweep with a launch for each, 16.3 us in passes of 8 that fetched the neighbours
+// when a row was made, 12.8 us in passes of 10 that fetch them late: 17 vector instructions a sweep and row of which 16 are the
+// function's, 63 million a pass of 126 us at 2.3 GHz, 81 % of what can be issued.  10 is what 3 waves a SIMD hold
+// (154 registers; us for 100 sweeps, plain stores: passes of 8 1626, 10 1315, 12 1450, 16 1415, the last two with 2 waves; 12 held
+// to 168 registers spills, 2160).  Results stored past the caches 1315 -> 1280, where operand and result exceed them (4000^2
+// 464 -> 493).  Leaving out the sweeps whose rows a chunk does not need yet: 5 x 3 taps 56.9 -> 52.3 us a sweep, 2000^2 10.2 -> 8.7.  Rows
+// fetched 6 or 9 instead of 3 ahead 1820 / 1840 us, strips that start at whole cache lines 1370 (their margins are wider).
+// Float64 30 us a sweep, 6000^2 17.8 -> 13.9.  All waves of a launch are resident at once: with 3072 of them passes of 8 took 15.7 us
+// a sweep, 2048 16.0, 1024 22.3, 4096, a second generation, 18.0.
 //
 // Boundary conditions hold in every sweep: a tap outside the array is replaced from the same
 // sweep's rows and columns (clamp, mirror), by the constant, or, for wrap, by continuing the array
@@ -32,14 +36,31 @@ struct SweepParams {
   i64 strips;     // strips of columns
   i64 items;      // strips * chunks of rows
   i64 rows;       // rows per chunk
+  i64 fewer;      // not 0: one sweep less than the kernel's number (LATE only: 4 instructions a row)
 };
 
 template <int N> struct AccConst { static constexpr int value = N; };
 
+// The value of the lane to the left (wave_shr:1 = 0x138) or right (wave_shl:1 = 0x130), as acc_dpp gives it, but 0 instead of their
+// own in the outermost lanes, which lie in the margins.  Without an old value to keep the compiler makes the move a modifier of
+// the addition that uses it.  For Spec::LATE only, that is for functions of floating-point additions and multiplications: a
+// subtraction with the modifier whose other operand a 64-bit integer multiply-add had written two wait states before
+// came out wrong (Int32, l + 3 c - r), as if it had read that register too early.
+template <int CTRL, class T> ACC_DEV T acc_shift(const T& v) {
+  if constexpr (!Spec::LATE) return acc_dpp<CTRL, 0xf>(v);
+  u32 w[AccWords<T>::N];
+  acc_to_words(v, w);
+#pragma unroll
+  for (int k = 0; k < AccWords<T>::N; ++k) w[k] = (u32)__builtin_amdgcn_update_dpp(0, (int)w[k], CTRL, 0xf, 0xf, true);
+  return acc_from_words<T>(w);
+}
+
 struct SweepRow { Spec::E e[ACC_SW_E]; };
 
-// v with its neighbours; XE: the strip reaches beyond the first or last column
-template <bool XE> ACC_DEV SweepRow acc_sweep_expand(const Spec::Env& env, const Spec::E (&v)[Spec::V], int gx, int w) {
+// v with its neighbours; XE: the strip reaches beyond the first or last column; OWN: the lane's own columns may lie outside
+// too (they do not once acc_sweep_keep has been over them)
+template <bool XE, bool OWN> ACC_DEV SweepRow acc_sweep_expand(const Spec::Env& env, const Spec::E (&v)[Spec::V], int gx,
+                                                              int w) {
   typedef Spec S;
   const int V = S::V, HX = S::HX;
   SweepRow r;
@@ -47,32 +68,57 @@ template <bool XE> ACC_DEV SweepRow acc_sweep_expand(const Spec::Env& env, const
   for (int k = 0; k < V; ++k) r.e[HX + k] = v[k];
 #pragma unroll
   for (int j = 1; j <= HX; ++j) {
-    r.e[HX - j] = acc_dpp<0x138, 0xf>(v[V - j]);          // from the lane to the left
-    r.e[HX + V - 1 + j] = acc_dpp<0x130, 0xf>(v[j - 1]);  // from the lane to the right
+    r.e[HX - j] = acc_shift<0x138>(v[V - j]);          // from the lane to the left
+    r.e[HX + V - 1 + j] = acc_shift<0x130>(v[j - 1]);  // from the lane to the right
   }
   if constexpr (XE && S::BOUNDARY != 2) {
     // a lane starts at column 0 or at a multiple of V from it, so only the last column can lie
     // inside a lane
+    const int first = OWN ? 1 : V;
     if constexpr (S::BOUNDARY == 0) {
 #pragma unroll
       for (int i = -1; i >= -HX; --i) r.e[HX + i] = gx + i < 0 ? r.e[HX + i + 1] : r.e[HX + i];
 #pragma unroll
-      for (int i = 1; i < V + HX; ++i) r.e[HX + i] = gx + i >= w ? r.e[HX + i - 1] : r.e[HX + i];
+      for (int i = first; i < V + HX; ++i) r.e[HX + i] = gx + i >= w ? r.e[HX + i - 1] : r.e[HX + i];
     } else if constexpr (S::BOUNDARY == 1) {
 #pragma unroll
       for (int j = 1; j <= HX; ++j) r.e[HX - j] = gx == 0 ? r.e[HX + j] : r.e[HX - j];
 #pragma unroll
-      for (int i = 1; i < V + HX; ++i)
+      for (int i = first; i < V + HX; ++i)
 #pragma unroll
         for (int j = 1; j <= HX; ++j)
           if (i - 2 * j >= -HX) r.e[HX + i] = gx + i == w - 1 + j ? r.e[HX + i - 2 * j] : r.e[HX + i];
     } else {
       const S::E c = S::outside(env);
 #pragma unroll
-      for (int i = -HX; i < V + HX; ++i) r.e[HX + i] = (gx + i < 0 || gx + i >= w) ? c : r.e[HX + i];
+      for (int i = -HX; i < V + HX; ++i)
+        if (OWN || i < 0 || i >= V) r.e[HX + i] = (gx + i < 0 || gx + i >= w) ? c : r.e[HX + i];
     }
   }
   return r;
+}
+
+// A row of a sweep as the wave keeps it until the last sweep that taps it.  Where the function taps neighbours in one row of
+// its window only (LATE), they are fetched when they are used: an operand that comes from the next lane then costs no instruction
+// of its own, and no registers in between.  Otherwise they are fetched once, when the row is made.
+template <bool LATE> struct SweepKept { Spec::E e[Spec::V]; };
+template <> struct SweepKept<false> { SweepRow row; };
+
+template <bool XE, bool LATE = Spec::LATE>
+ACC_DEV SweepKept<LATE> acc_sweep_keep(const Spec::Env& env, const Spec::E (&v)[Spec::V], int gx, int w) {
+  SweepKept<LATE> k;
+  const SweepRow r = acc_sweep_expand<XE, true>(env, v, gx, w);
+  if constexpr (LATE) {
+#pragma unroll
+    for (int i = 0; i < Spec::V; ++i) k.e[i] = r.e[Spec::HX + i];
+  } else {
+    k.row = r;
+  }
+  return k;
+}
+template <bool XE, bool LATE> ACC_DEV SweepRow acc_sweep_row(const Spec::Env& env, const SweepKept<LATE>& k, int gx, int w) {
+  if constexpr (LATE) return acc_sweep_expand<XE, false>(env, k.e, gx, w);
+  else return k.row;
 }
 
 // the window around row y of h; YE: the window may reach beyond the first or last row
@@ -119,7 +165,7 @@ template <int T> struct SweepGeo {
   static constexpr int U = ACC_WAVE * Spec::V - 2 * HXT;                        // columns a strip gives
 };
 
-template <int T, bool XE> ACC_DEV void acc_sweep_strip(const Spec::Env& env, const Spec::Out& out, const SweepParams& p,
+template <int T, bool XE, bool NT> ACC_DEV void acc_sweep_strip(const Spec::Env& env, const Spec::Out& out, const SweepParams& p,
                                                        int strip, int y0, int y1) {
   typedef Spec S;
   typedef S::E E;
@@ -165,74 +211,79 @@ template <int T, bool XE> ACC_DEV void acc_sweep_strip(const Spec::Env& env, con
   E pre[ACC_SW_P][S::V];            // the next rows, on their way
 #pragma unroll
   for (int u = 0; u < NP; ++u) load(ys + u, pre[u]);
-  SweepRow win[T][ACC_SW_P];        // win[t][u]: the newest rows of sweep t; row r lies in slot (r - ys + t * HY) % NP
+  SweepKept<S::LATE> win[T][ACC_SW_P];  // win[t][u]: the newest rows of sweep t; row r lies in slot (r - ys + t * HY) % NP
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int u = 0; u < NP; ++u)
-#pragma unroll
-      for (int e = 0; e < ACC_SW_E; ++e) win[t][u].e[e] = (E)0;
+    for (int u = 0; u < NP; ++u) win[t][u] = SweepKept<S::LATE>{};
 
-  auto step = [&](auto ye_, auto u_, int yin) __attribute__((always_inline)) {
+  // Sweep t has its first row that is computed from nothing but loaded ones 2 * t * HY steps in: until then it is left out, two sweeps
+  // at a time.
+  constexpr int GROUP = 2;
+  auto level = [&](auto ye_, auto u_, auto t_, int yin) __attribute__((always_inline)) {
     constexpr bool YE = decltype(ye_)::value != 0;
-    constexpr int u = decltype(u_)::value;
-    win[0][u] = acc_sweep_expand<XE>(env, pre[u], gx, w);
-    load(yin + NP, pre[u]);
+    constexpr int u = decltype(u_)::value, t = decltype(t_)::value;
+    const int y = yin - t * HY;
+    SweepRow wv[ACC_SW_P];
 #pragma unroll
-    for (int t = 1; t <= T; ++t) {
-      const int y = yin - t * HY;
-      SweepRow wv[ACC_SW_P];
+    for (int q = 0; q < NP; ++q) wv[q] = acc_sweep_row<XE>(env, win[t - 1][(u + 1 + q) % NP], gx, w);
+    acc_sweep_window<YE>(env, wv, y, h);
+    E r[S::V];
 #pragma unroll
-      for (int q = 0; q < NP; ++q) wv[q] = win[t - 1][(u + 1 + q) % NP];
-      acc_sweep_window<YE>(env, wv, y, h);
-      E r[S::V];
+    for (int k = 0; k < V; ++k) r[k] = S::apply_win(env, wv, k).c0;
+    if constexpr (t == T && S::LATE) {
+      // one sweep less: the last one hands on what it finds
 #pragma unroll
-      for (int k = 0; k < V; ++k) r[k] = S::apply_win(env, wv, k).c0;
-      if (t < T) {
-        win[t < T ? t : 0][u] = acc_sweep_expand<XE>(env, r, gx, w);
-      } else if (y >= y0 && y < y1) {
-        E* row = dst + (i64)y * w;
-        if constexpr (XE) {
+      for (int k = 0; k < V; ++k) r[k] = p.fewer ? wv[HY].e[S::HX + k] : r[k];
+    }
+    if constexpr (t < T) {
+      win[t][u] = acc_sweep_keep<XE>(env, r, gx, w);
+    } else if (y >= y0 && y < y1) {
+      E* row = dst + (i64)y * w;
+      if constexpr (XE) {
 #pragma unroll
-          for (int k = 0; k < V; ++k)
-            if (gx + k >= lo && gx + k < hi) row[gx + k] = r[k];
-        } else if (gx >= lo && gx < hi) {
-          acc_run<E, S::V> o;
+        for (int k = 0; k < V; ++k)
+          if (gx + k >= lo && gx + k < hi) row[gx + k] = r[k];
+      } else if (gx >= lo && gx < hi) {
+        typedef E Run __attribute__((vector_size(16), aligned(sizeof(E))));
+        Run o;
 #pragma unroll
-          for (int k = 0; k < V; ++k) o.e[k] = r[k];
-          *(acc_run<E, S::V>*)(row + gx) = o;
-        }
+        for (int k = 0; k < V; ++k) o[k] = r[k];
+        if constexpr (NT) __builtin_nontemporal_store(o, (Run*)(row + gx));
+        else *(Run*)(row + gx) = o;
       }
+    }
+  };
+  auto levels = [&](auto self, auto ye_, auto u_, auto t_, int yin) __attribute__((always_inline)) {
+    constexpr int t = decltype(t_)::value;
+    if constexpr (t <= T) {
+      if (t > 1 && (t - 1) % GROUP == 0 && yin < ys + 2 * t * HY) return;
+      level(ye_, u_, t_, yin);
+      self(self, ye_, u_, AccConst<t + 1>(), yin);
+    }
+  };
+  auto step = [&](auto ye_, auto u_, int yin) __attribute__((always_inline)) {
+    constexpr int u = decltype(u_)::value;
+    win[0][u] = acc_sweep_keep<XE>(env, pre[u], gx, w);
+    load(yin + NP, pre[u]);
+    levels(levels, ye_, u_, AccConst<1>(), yin);
+  };
+  auto steps = [&](auto self, auto ye_, auto u_, int y) __attribute__((always_inline)) {
+    constexpr int u = decltype(u_)::value;
+    if constexpr (u < ACC_SW_P) {
+      step(ye_, u_, y + u);
+      self(self, ye_, AccConst<u + 1>(), y);
     }
   };
   for (int y = ys; y < ye; y += NP) {
     // a sweep of these steps computes rows y - T * HY .. y + NP - 1 - HY, and looks HY rows further
     const bool edge = S::BOUNDARY != 2 && (y - (T + 1) * HY < 0 || y + NP - 1 >= h);
-    if (edge) {
-      step(AccConst<1>(), AccConst<0>(), y);
-      if constexpr (ACC_SW_P > 1) {
-        step(AccConst<1>(), AccConst<1>(), y + 1);
-        step(AccConst<1>(), AccConst<2>(), y + 2);
-      }
-      if constexpr (ACC_SW_P > 3) {
-        step(AccConst<1>(), AccConst<3>(), y + 3);
-        step(AccConst<1>(), AccConst<4>(), y + 4);
-      }
-    } else {
-      step(AccConst<0>(), AccConst<0>(), y);
-      if constexpr (ACC_SW_P > 1) {
-        step(AccConst<0>(), AccConst<1>(), y + 1);
-        step(AccConst<0>(), AccConst<2>(), y + 2);
-      }
-      if constexpr (ACC_SW_P > 3) {
-        step(AccConst<0>(), AccConst<3>(), y + 3);
-        step(AccConst<0>(), AccConst<4>(), y + 4);
-      }
-    }
+    if (edge) steps(steps, AccConst<1>(), AccConst<0>(), y);
+    else steps(steps, AccConst<0>(), AccConst<0>(), y);
   }
 }
 
-template <int T> ACC_DEV void acc_sweep(const Spec::Env& env, const Spec::Out& out, const SweepParams& p) {
+template <int T, bool NT = false> ACC_DEV void acc_sweep(const Spec::Env& env, const Spec::Out& out, const SweepParams& p) {
   typedef Spec S;
   // neighbouring strips share their margins: neighbours run on the same XCD
   const i64 b = acc_xcd_contiguous((i64)blockIdx.x, (i64)gridDim.x);
@@ -242,10 +293,18 @@ template <int T> ACC_DEV void acc_sweep(const Spec::Env& env, const Spec::Out& o
   const int y0 = chunk * (int)p.rows;
   const int y1 = y0 + p.rows < p.h ? y0 + (int)p.rows : (int)p.h;
   const int x0 = strip * SweepGeo<T>::U - SweepGeo<T>::HXT;
-  if (x0 >= 0 && x0 + ACC_WAVE * S::V <= p.w) acc_sweep_strip<T, false>(env, out, p, strip, y0, y1);
-  else acc_sweep_strip<T, true>(env, out, p, strip, y0, y1);
+  if (x0 >= 0 && x0 + ACC_WAVE * S::V <= p.w) acc_sweep_strip<T, false, NT>(env, out, p, strip, y0, y1);
+  else acc_sweep_strip<T, true, NT>(env, out, p, strip, y0, y1);
 }
 
+#if ACC_SW_MAX >= 10
+extern "C" __global__ void __launch_bounds__(ACC_BLOCK) acc_sweeps10(Spec::Env env, Spec::Out out, SweepParams p) {
+  acc_sweep<10>(env, out, p);
+}
+extern "C" __global__ void __launch_bounds__(ACC_BLOCK) acc_sweeps10_stream(Spec::Env env, Spec::Out out, SweepParams p) {
+  acc_sweep<10, true>(env, out, p);
+}
+#endif
 #if ACC_SW_MAX >= 8
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK) acc_sweeps8(Spec::Env env, Spec::Out out, SweepParams p) {
   acc_sweep<8>(env, out, p);

@@ -11,7 +11,7 @@ from . import progs as Q
 
 Int = A.Int
 BOUNDARIES = ["clamp", "mirror", "wrap", "constant"]
-# extents at the edges of the kernel's strips (128 / 256 columns less 2 x 8, 4, 2 margins of 1 or 2) and chunks
+# extents at the edges of the kernel's strips (128 / 256 columns less 2 x 10, 8, 4, 2 margins of 1 or 2) and chunks
 SHAPES = [(32, 32), (33, 47), (37, 240), (64, 241), (40, 255), (95, 256), (41, 497), (257, 112), (130, 1003), (1001, 123)]
 
 
@@ -82,6 +82,34 @@ def test_sweeps_equal_single_launches(gpu_ctx, knobs, ty, npty, kind, widths):
             cnt = gpu_ctx.to_device(np.array(n, np.int64), A.tarray(0, Int))
             got, want = fused.execute(g, cnt).to_host(), single.execute(g, cnt).to_host()
             assert np.array_equal(got, want, equal_nan=np.dtype(npty).kind == "f"), (shape, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", BOUNDARIES)
+@pytest.mark.parametrize("ty,npty,taps", [(A.f32, np.float32, "cross"), (A.f64, np.float64, "cross"), (A.i32, np.int32, "row")], ids=str)
+def test_neighbours_of_one_row(gpu_ctx, knobs, ty, npty, kind, taps):
+    """Functions that tap neighbours in one row only fetch them late and take passes of 10; every number of sweeps up to
+    two passes, with results stored past the caches or not."""
+    def step():
+        sr = A.stup(*[A.sunit(3, ty)] * 3)
+
+        def f(st):
+            (_, t, _), (l, c, r), (_, b, _) = (A.untup(row) for row in A.untup(st))
+            if taps == "row":
+                return A.sub(ty, A.add(ty, l, A.mul(ty, A.const(ty, 3), c)), r)
+            return A.sub(ty, A.add(ty, t, A.mul(ty, A.const(ty, 3), l)), A.add(ty, A.add(ty, r, r), b))
+        return A.alam([A.tarray(2, ty)], lambda g: A.stencil(sr, ty, A.lam([A.stencil_type(sr)], f), _boundary(kind, ty), g))
+
+    fused, single = _both(gpu_ctx, knobs, sweeps(step, ty))
+    for k, (shape, counts) in enumerate([((32, 33), range(1, 12)), ((61, 109), (10, 19)), ((47, 233), (9, 10, 20)),
+                                         ((130, 465), (10, 13)), ((300, 240), (3, 7, 10))]):
+        g = gpu_ctx.to_device(_grid(shape, npty, 2 + k), A.tarray(2, ty))
+        for n in counts:
+            cnt = gpu_ctx.to_device(np.array(n, np.int64), A.tarray(0, Int))
+            want = single.execute(g, cnt).to_host()
+            for stream in (1 << 40, 1):
+                knobs("stream_bytes", stream)
+                assert np.array_equal(fused.execute(g, cnt).to_host(), want, equal_nan=np.dtype(npty).kind == "f"), (shape, n, stream)
 
 
 @pytest.mark.gpu
