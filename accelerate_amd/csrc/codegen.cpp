@@ -1158,9 +1158,10 @@ bool Codegen::scanPipeable(const Operand& src, bool right) {
 }
 
 KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool right, int kind, int variant,
-                           const Sx* post, const TypeP& postElt) {
-  const TypeP elt = src.r.elt;
+                           const Sx* post, const TypeP& postElt, const Scanned* also) {
+  const TypeP elt = also ? tPair(src.r.elt, also->src.r.elt) : src.r.elt;
   const bool small = variant == 1, pipe = variant == 2;
+  if (also && (pipe || post)) throw Error("scan: this variant takes no second scan");
   if (pipe && !scanPipeable(src, right)) throw Error("scan: this operand cannot take the pipelined kernel");
   if (post && (pipe || kind == 2)) throw Error("scan: this variant applies no function to its results");
   std::string pipeSlot;  // the array the pipelined kernel moves
@@ -1179,7 +1180,9 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
     Emit em;
     em.ind = 4;
     ValP a = eltVal(elt, "x"), b = eltVal(elt, "y");
-    ValP r = right ? applyFun(f, {b, a}, {}, em) : applyFun(f, {a, b}, {}, em);
+    if (right) std::swap(a, b);
+    ValP r = also ? applyFun(f, {a->a, b->a}, {}, em) : applyFun(f, {a, b}, {}, em);
+    if (also) r = vPair(r, applyFun(also->f, {a->b, b->b}, {}, em));
     if (!typeEq(valType(r), elt)) throw Error("scan: combination function does not return the element type");
     body += fnHead("Elt", "combine", "const Env& env, const Elt& x, const Elt& y") + returnElt(r, em) + "  }\n";
   }
@@ -1188,6 +1191,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
     em.ind = 4;
     if (seed) {
       ValP z = exp(*seed, {}, em);
+      if (also) z = vPair(z, exp(*also->seed, {}, em));
       if (!typeEq(valType(z), elt)) throw Error("scan: seed does not have the element type");
       returnElt(z, em);
     } else {
@@ -1200,6 +1204,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
     Emit em;
     em.ind = 4;
     ValP v = operandLinear(src, "i", em);
+    if (also) v = vPair(v, operandLinear(also->src, "i", em));
     if (!typeEq(valType(v), elt)) throw Error("scan: fused producer does not return the element type");
     body += fnHead("Elt", "in_linear", "const Env& env, i64 i") + returnElt(v, em) + "  }\n";
   }
@@ -1287,7 +1292,9 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
     rowsG = std::max(1, std::min(g, 128 / std::max(1, vec * std::max(1, eltBytes))));
     if (small) body += "#define ACC_ROWS_G " + std::to_string(rowsG) + "\n";
     if (small) {
-      allG = std::max(1, std::min(8, 64 / std::max(1, vec * std::max(1, eltBytes))));
+      // (two scans at once hold a pair an element, of which one source may give both: twice the bytes; Int64 flags and their
+      // opposite, two million 41.5 -> 34.4 us a radix pass)
+      allG = std::max(1, std::min(8, (also ? 128 : 64) / std::max(1, vec * std::max(1, eltBytes))));
       body += "#define ACC_SCAN_ALL_G " + std::to_string(allG) + "\n";
     }
     if (small && rowsG > 1 && (long)(block / 64) * (64 * (rowsG + 1) + 1) * sz <= 64 * 1024 && !(re && re[0] == '0'))

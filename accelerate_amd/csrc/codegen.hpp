@@ -99,8 +99,15 @@ class Codegen {
   // (only where scanPipeable holds)
   // post (with its result type): a function applied to every result on its way to memory -- the
   // `map g` of `map g (scan f z xs)`, which then costs neither a launch nor an array of its own
+  // also: a second scan of the same kind, direction and extents, computed together with the first (elements, results
+  // and totals are pairs); not the pipelined kernel, no post
+  struct Scanned {
+    const Sx& f;
+    const Sx* seed;
+    const Operand& src;
+  };
   KernelSource scan(const Sx& f, const Sx* seed, const Operand& src, bool right, int kind, int variant = 0,
-                    const Sx* post = nullptr, const TypeP& postElt = nullptr);
+                    const Sx* post = nullptr, const TypeP& postElt = nullptr, const Scanned* also = nullptr);
   static bool scanPipeable(const Operand& src, bool right);
   // half: tiles of half the length, for fused producers that read arrays (foldSegHalves) and not too many values
   KernelSource foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType, bool half);

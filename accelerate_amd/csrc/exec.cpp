@@ -519,6 +519,10 @@ Program::Program(Context& ctx, const char* text, size_t len) : ctx_(ctx) {
     for (auto& sk : kv.second.scalarKernels) ctx_.wait(sk.second);
   }
   for (auto& kv : sweeps_) ctx_.wait(kv.second.k);
+  for (auto& kv : joints_) {
+    ctx_.wait(kv.second.k);
+    ctx_.wait(kv.second.k2);
+  }
   // a program that is one scan can be run without allocating (runInto): its code objects are
   // loaded now, so that no launch of it has set-up work left
   if (ctx_.hasDevice() && (body_->is("scan") || body_->is("scan'"))) {
@@ -538,6 +542,8 @@ std::vector<std::string> Program::kernelKeys() const {
       if (sk.second) keys.push_back(sk.second->hash);
   }
   for (auto& kv : sweeps_) keys.push_back(kv.second.k->hash);
+  for (auto& kv : joints_)
+    for (const KernelP& k : {kv.second.k, kv.second.k2}) keys.push_back(k->hash);
   std::sort(keys.begin(), keys.end());
   keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
   return keys;
@@ -613,6 +619,7 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
     pushTypes(n.at(1), tenv);
     ATyP r = prepare(n.at(3), tenv);
     tenv.resize(mark);
+    prepareJoint(n, tenv);
     return r;
   }
   if (h == "apair") {
@@ -868,6 +875,50 @@ ATyP Program::prepareScan(const Sx& n, TEnv& tenv, Plan& plan, const Sx* post, c
   if (post) r.elt = postElt;
   plan.ty = atArr(r);
   return plan.ty;
+}
+
+// a term moved out of `by` innermost bindings of arrays; false where it mentions one of them
+static bool moveOut(Sx& e, long long by) {
+  if (e.atom) return true;
+  if (e.is("avar") || e.is("index") || e.is("linearindex") || e.is("shape")) {
+    const long long ix = e.at(1).asInt();
+    if (ix < by) return false;
+    e.kids[1].s = std::to_string(ix - by);
+  }
+  for (Sx& k : e.kids)
+    if (!moveOut(k, by)) return false;
+  return true;
+}
+
+void Program::prepareJoint(const Sx& n, TEnv& tenv) {
+  if (ctx_.knobs.scan_joint == 0 || !n.at(3).is("alet")) return;
+  const Sx &a = n.at(2), &b = n.at(3).at(2);
+  const bool prime = a.is("scan'");
+  if (!(prime ? b.is("scan'") : a.is("scan") && b.is("scan")) || a.at(1).s != b.at(1).s) return;
+  if (!prime && a.at(3).isAtom("nothing") != b.at(3).isAtom("nothing")) return;
+  TEnv inner;
+  pushTypes(n.at(1), inner);
+  Joint j;
+  j.second = b;
+  if (!moveOut(j.second, (long long)inner.size())) return;
+  const Plan &pa = plans_.at(&a), &pb = plans_.at(&b);
+  if (!pa.temps.empty() || !pb.temps.empty() || !pa.scalarKernels.empty() || !pb.scalarKernels.empty()) return;
+  j.first = pa.ty;
+  j.other = pb.ty;
+  const ArrayR &ra = prime ? pa.ty->a->r : pa.ty->r, &rb = prime ? pb.ty->a->r : pb.ty->r;
+  std::vector<ST> leaves = typeLeaves(ra.elt);
+  for (ST t : typeLeaves(rb.elt)) leaves.push_back(t);
+  if (ra.rank != rb.rank || leaves.size() != 2 || stIsVec(leaves[0]) || stIsVec(leaves[1])) return;
+  for (int small = 0; small < 2; ++small) {
+    Codegen cg(aenvOf(tenv));
+    Plan none;
+    Operand sa = operandOf(a.at(4), cg, tenv, none), sb = operandOf(j.second.at(4), cg, tenv, none);
+    auto seed = [&](const Sx& s) -> const Sx* { return prime ? &s.at(3) : s.at(3).is("just") ? &s.at(3).at(1) : nullptr; };
+    const Codegen::Scanned also{j.second.at(2), seed(j.second), sb};
+    const int kind = prime ? 2 : seed(a) ? 1 : 0;
+    (small ? j.k2 : j.k) = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, small, nullptr, nullptr, &also));
+  }
+  joints_.emplace(&n, std::move(j));
 }
 
 // ------------------------------------------------------------------------------------
@@ -1290,6 +1341,185 @@ static bool foldSegHalf(const KernelSource& full, int64_t total) {
   return total <= (int64_t)3 << 23 && (total < (int64_t)3 << 21 || total % tile != 0);
 }
 
+// Both scans of a joint pair in one launch; false: one after the other, as they stand.  A scan of a few million elements is
+// a chain of round trips that one launch makes once for both: 1000 elements 9.7 -> 6.7 us, one million Int64 14.5 -> 10.2, Float32 12.1 -> 7.3,
+// three million 27.7 -> 21.4, 18.8 -> 12.6; with one source for both (flags and their opposite) the elements are read once as well.
+// From 64 MiB of pairs on two of the kernels for long rows are as fast: Int64 4 million 35.3 / 31.7, scan' 37.8 / 38.6, 8 million 53 / 59;
+// Float32 8 million 37.6 / 24.1.
+bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other) {
+  auto it = joints_.find(&n);
+  if (it == joints_.end() || ctx_.knobs.scan_joint == 0) return false;
+  const Joint& j = it->second;
+  const Plan none;
+  size_t cur = 0;
+  const std::vector<int64_t> ext = operandExtent(n.at(2).at(4), aenv, none, {}, cur);
+  if (operandExtent(j.second.at(4), aenv, none, {}, cur) != ext) return false;
+  int64_t bytes = 0;
+  for (ST t : j.k->meta.outLeaves) bytes += stSize(t);
+  for (int64_t d : ext) bytes *= std::max<int64_t>(d, 0);
+  if (ctx_.knobs.scan_joint < 2 && bytes > (int64_t)64 << 20) return false;
+  const bool prime = n.at(2).is("scan'");
+  const int kind = prime ? 2 : n.at(2).at(3).isAtom("nothing") ? 0 : 1;
+  std::vector<int64_t> outer(ext.begin(), ext.end() - 1), oshape = outer;
+  oshape.push_back(std::max<int64_t>(ext.back(), 0) + (kind == 1));
+  std::vector<DArrayP> outs, tots;
+  for (const ATyP& t : {j.first, j.other}) outs.push_back(alloc(prime ? t->a->r : t->r, oshape));
+  tots = outs;
+  if (prime) tots = {alloc(j.first->b->r, outer), alloc(j.other->b->r, outer)};
+  launchScan(j.k, j.k2, nullptr, kind, ext, aenv, {}, outs, tots);
+  first = prime ? avPair(avArr(outs[0]), avArr(tots[0])) : avArr(outs[0]);
+  other = prime ? avPair(avArr(outs[1]), avArr(tots[1])) : avArr(outs[1]);
+  return true;
+}
+
+void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext,
+                         const AEnv& aenv, const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs,
+                         const std::vector<DArrayP>& tots) {
+  const int64_t len = std::max<int64_t>(ext.back(), 0);
+  int64_t rows = 1;
+  for (size_t d = 0; d + 1 < ext.size(); ++d) rows *= std::max<int64_t>(ext[d], 0);
+  if (rows == 0 || (kind == 0 && len == 0)) return;
+  // (an argument structure starts with a word of its own: the arrays of a joint scan share one)
+  auto packOuts = [&](std::vector<uint64_t>& args) {
+    for (const std::vector<DArrayP>* part : {&outs, &tots}) {
+      packOut(args, *part->at(0));
+      for (size_t i = 1; i < part->size(); ++i)
+        for (auto& b : part->at(i)->bufs) args.push_back((uint64_t)(uintptr_t)b->p);
+    }
+  };
+  // large tiles when they fill the device, small ones otherwise
+  const KernelSource& big = k->meta;
+  const int64_t bigTile = (int64_t)big.block * big.group * big.vec;
+  bool small = false;
+  if (k2) {
+    const KernelSource& sm = k2->meta;
+    const int64_t smallTile = (int64_t)sm.block * sm.group * sm.vec;
+    // (measured, large against small tiles: Float32 171 large tiles 26.7 / 21.9 us, 341 tiles 36.0 /
+    // 39.4; Int64 85 tiles 13.3 / 13.2, 171 tiles 18.0 / 21.7 -- elements of 4 bytes and fewer keep
+    // the small tiles for longer because a large tile's lanes hold twice as many of them)
+    const int64_t fewer = big.words <= 1 ? 256 : 100;
+    small = rows * ((len + bigTile - 1) / bigTile) < fewer || len <= 2 * smallTile;
+    // and as long as all small tiles are on the device at once, for then they need no tickets
+    // (Float32 2^24, 1024 tiles: 27.9 us against 36.1 with the large tiles and 37.2 pipelined;
+    // Int64 2^23: 25.4 against 32.1 and 27.0)
+    if (!small && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0)
+      small = rows * ((len + smallTile - 1) / smallTile) <= ctx_.residentGroups(k2, "acc_scan", (unsigned)sm.block);
+  }
+  const long long forcedTiles = ctx_.knobs.scan_tiles;  // 1 large / 2 small / 3 rows: override, for tests
+  if (forcedTiles == 1 || forcedTiles == 4) small = false;
+  if ((forcedTiles == 2 || forcedTiles >= 5) && k2) small = true;
+  if (k2 && len >= 1) {
+    // many short rows: several whole rows per workgroup (acc_scan_rows)
+    const KernelSource& sm = k2->meta;
+    const int64_t rowsTile = (int64_t)sm.block * sm.rowsGroup * sm.vec;
+    const bool forced = forcedTiles == 3;
+    // (up to a whole tile of it: a row alone in its workgroup still moves group by group, while
+    // a tile of acc_scan that its row does not fill goes through the code for ragged ends)
+    if ((forced && len <= rowsTile) || (forcedTiles == 0 && rows >= 2 && len <= rowsTile)) {
+      const int64_t rpt = rowsTile / len;
+      const int64_t groups = (rows + rpt - 1) / rpt;
+      if (groups > 0x7fffffffLL) throw Error("scan: too many rows for one launch");
+      std::vector<uint64_t> args = packArgs(sm, aenv, temps, {});
+      packOuts(args);
+      args.push_back((uint64_t)rows);
+      args.push_back((uint64_t)len);
+      args.push_back((uint64_t)rpt);
+      ctx_.launch(k2, "acc_scan_rows", (uint64_t)groups, (unsigned)sm.block, args);
+      return;
+    }
+  }
+  // Long rows of a plain array: the pipelined kernel (persistent workgroups, one per CU).  Its
+  // direct global -> LDS loads move 16 bytes per lane from 16-byte aligned addresses.
+  bool pipe = false;
+  if (k3 && !small) {
+    const KernelSource& pm = k3->meta;
+    const int64_t pipeTile = (int64_t)pm.block * pm.group * pm.vec;
+    const int64_t eltBytes = 16 / pm.vec;
+    // the array the kernel moves: the operand itself, or the one array a fused producer reads
+    DArrayP srcArr;
+    for (const ArraySlot& sl : pm.arrays)
+      if (sl.name == pm.pipeSlot) srcArr = sl.temp ? temps.at(sl.index) : aenv.at(aenv.size() - 1 - sl.index);
+    // (a right scan's tiles are counted from the end of each row; a producer must cover its array exactly)
+    const bool aligned = srcArr && !srcArr->bufs.empty() && ((uintptr_t)srcArr->bufs[0]->p & 15) == 0 &&
+                         srcArr->shape == ext && ((rows == 1 && !pm.scanRight) || (len * eltBytes) % 16 == 0);
+    const int64_t tprP = (len + pipeTile - 1) / pipeTile;
+    // measured on 2^28 elements: Float32 350 us against 395 us for a workgroup per tile, Int64 706
+    // against 742; from two tiles per CU on it is level or ahead (Int64 2^23, 512 tiles: 27 against
+    // 32 us; Float32 2^24, 585 tiles: 37 against 36; with 256 tiles 18.7 against 18.0)
+    pipe = aligned && (forcedTiles == 4 ? len >= pipeTile
+                                        : (forcedTiles == 0 && tprP >= 16 && rows * tprP >= 2 * ctx_.computeUnits()));
+  }
+  const KernelP& kern = pipe ? k3 : (small ? k2 : k);
+  const KernelSource& m = kern->meta;
+  // Of the small tiles, where all of them run at once: a quarter of their size for up to a tile per CU,
+  // half of it for up to three, and every tile reads all its predecessors' aggregates (acc_scan_all,
+  // acc_scan_all2).  Measured, acc_scan / all / all2 in us, scanl: Float32 2^18 7.0 / 4.6 / 5.1, 2^20 (256 tiles
+  // of acc_scan_all) 7.5 / 6.4 / 6.4, 2^21 9.2 / 8.3 / 7.7, 2^22 12.7 / 12.7 / 10.2, 6 million (733 tiles of
+  // acc_scan_all2) 16.9 / 17.9 / 14.0, 2^23 (1024) 17.7 / 26.0 / 18.6; Int64 2^17 7.2 / 4.7 / 5.6, 2^19 (256) 7.6 /
+  // 6.1 / 6.4, 2^20 9.3 / 7.9 / 7.2, 2^21 12.6 / 12.0 / 9.8, 3 million (733) 15.0 / 16.6 / 13.0, 2^22 (1024) 17.1 / 26.2 / 17.3.
+  const char* fn = "acc_scan";
+  int64_t group = m.group;
+  if (small && (forcedTiles == 0 || forcedTiles >= 5) && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0) {
+    for (int two = forcedTiles == 6 ? 1 : 0; two < 2; ++two) {
+      const char* f = two ? "acc_scan_all2" : "acc_scan_all";
+      const int64_t g = (int64_t)m.allGroup * (two + 1), t = (int64_t)m.block * g * m.vec, all = rows * ((len + t - 1) / t);
+      const int64_t most = forcedTiles >= 5 ? 4096 : (two ? 3 : 1) * ctx_.computeUnits();
+      // (every CU holds at least one workgroup of any kernel: the runtime need not be asked)
+      if (all <= most && (all <= ctx_.computeUnits() || all <= ctx_.residentGroups(kern, f, (unsigned)m.block))) {
+        fn = f;
+        group = g;
+        break;
+      }
+      if (forcedTiles == 5) break;
+    }
+  }
+  const int64_t tile = (int64_t)m.block * group * m.vec;
+  const int64_t tpr = std::max<int64_t>(1, (len + tile - 1) / tile);
+  const int64_t tiles = rows * tpr;
+  if (tiles > 0x7fffffffLL) throw Error("scan: too many tiles for one launch");
+  const size_t descBytes = (size_t)tiles * m.words * sizeof(uint64_t);
+  ScanState& st = noAlloc_ ? staticScanState(ctx_.device(), ctx_.stream(), descBytes) : ctx_.scanState(descBytes);
+  std::vector<uint64_t> args = packArgs(m, aenv, temps, {});
+  packOuts(args);
+  args.push_back((uint64_t)rows);
+  args.push_back((uint64_t)len);
+  args.push_back((uint64_t)tpr);
+  args.push_back((uint64_t)(uintptr_t)st.desc);
+  args.push_back((uint64_t)(uintptr_t)st.ticket);
+  const size_t ticketAt = args.size() - 1;
+  // fault injection for the test of the bounded look-back wait: a ticket base that lags the
+  // counter by `skew` gives every tile a number `skew` too high, so the first tiles wait for
+  // predecessors that never run, give up after `spin` polls and report
+  const uint64_t skew = (uint64_t)std::max<long long>(0, ctx_.knobs.scan_test_skew);
+  // a legitimate wait lasts microseconds; 2^22 polls are several seconds
+  const uint64_t spin = (uint64_t)std::max<long long>(1, ctx_.knobs.scan_spin_limit);
+  args.push_back((uint64_t)(st.ticketBase - skew));
+  args.push_back((uint64_t)st.epoch);
+  args.push_back(spin);
+  args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
+  const int64_t tprFull = len / tile;
+  args.push_back((uint64_t)tprFull);
+  if (pipe) {
+    // the full tiles of every row; every workgroup takes tickets until it meets the first one
+    // beyond them.  Then, with the same epoch, the rows' last tiles where they are partial.
+    const int64_t fullTiles = rows * tprFull;
+    const uint64_t groups = (uint64_t)std::min<int64_t>(fullTiles, ctx_.computeUnits());
+    ctx_.launch(kern, "acc_scan_pipe", groups, (unsigned)m.block, args);
+    // (a workgroup stops at the first ticket beyond the tiles: with the test's skew that is `skew` tickets earlier)
+    st.ticketBase += (uint64_t)std::max<int64_t>(0, fullTiles - (int64_t)skew) + groups;
+    if (tprFull < tpr) ctx_.launch(kern, "acc_scan_pipe_tail", (uint64_t)rows, (unsigned)m.block, args);
+    return;
+  }
+  // A launch whose tiles are all on the device at once needs no tickets: a tile's number is its
+  // workgroup's, nobody waits for a tile that cannot start, and every workgroup is spared the
+  // counter's round trip in front of its loads (one row of 2^20 Int32: 7.5 -> 6.5 us).
+  const bool ticketless = skew == 0 && ctx_.knobs.scan_ticketless != 0 &&
+                          (tiles <= ctx_.computeUnits() || tiles <= ctx_.residentGroups(kern, fn, (unsigned)m.block));
+  if (ticketless) args[ticketAt] = 0;
+  ctx_.launch(kern, fn, (uint64_t)tiles, (unsigned)m.block, args);
+  if (!ticketless) st.ticketBase += (uint64_t)tiles;
+}
+
 AValP Program::eval(const Sx& n, AEnv& aenv) {
   if (n.isAtom("anil")) return avUnit();
   const std::string& h = n.head();
@@ -1298,10 +1528,18 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     return avArr(aenv[aenv.size() - 1 - ix]);
   }
   if (h == "alet") {
-    AValP v = eval(n.at(2), aenv);
+    AValP v, other;
     size_t mark = aenv.size();
-    pushVals(n.at(1), v, aenv);
-    AValP r = eval(n.at(3), aenv);
+    const Sx* body = &n.at(3);
+    if (evalJoint(n, aenv, v, other)) {
+      pushVals(n.at(1), v, aenv);
+      pushVals(body->at(1), other, aenv);
+      body = &body->at(3);
+    } else {
+      v = eval(n.at(2), aenv);
+      pushVals(n.at(1), v, aenv);
+    }
+    AValP r = eval(*body, aenv);
     aenv.resize(mark);
     return r;
   }
@@ -1953,144 +2191,8 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     DArrayP out = alloc(ar, oshape);
     DArrayP tot = out;
     if (prime) tot = alloc(plan.ty->b->r, outer);
-    int64_t rows = 1;
-    for (int64_t d : outer) rows *= std::max<int64_t>(d, 0);
-    AValP result = prime ? avPair(avArr(out), avArr(tot)) : avArr(out);
-    if (rows == 0 || (kind == 0 && len == 0)) return result;
-    // large tiles when they fill the device, small ones otherwise
-    const KernelSource& big = plan.k->meta;
-    const int64_t bigTile = (int64_t)big.block * big.group * big.vec;
-    bool small = false;
-    if (plan.k2) {
-      const KernelSource& sm = plan.k2->meta;
-      const int64_t smallTile = (int64_t)sm.block * sm.group * sm.vec;
-      // (measured, large against small tiles: Float32 171 large tiles 26.7 / 21.9 us, 341 tiles 36.0 /
-      // 39.4; Int64 85 tiles 13.3 / 13.2, 171 tiles 18.0 / 21.7 -- elements of 4 bytes and fewer keep
-      // the small tiles for longer because a large tile's lanes hold twice as many of them)
-      const int64_t fewer = big.words <= 1 ? 256 : 100;
-      small = rows * ((len + bigTile - 1) / bigTile) < fewer || len <= 2 * smallTile;
-      // and as long as all small tiles are on the device at once, for then they need no tickets
-      // (Float32 2^24, 1024 tiles: 27.9 us against 36.1 with the large tiles and 37.2 pipelined;
-      // Int64 2^23: 25.4 against 32.1 and 27.0)
-      if (!small && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0)
-        small = rows * ((len + smallTile - 1) / smallTile) <= ctx_.residentGroups(plan.k2, "acc_scan", (unsigned)sm.block);
-    }
-    const long long forcedTiles = ctx_.knobs.scan_tiles;  // 1 large / 2 small / 3 rows: override, for tests
-    if (forcedTiles == 1 || forcedTiles == 4) small = false;
-    if ((forcedTiles == 2 || forcedTiles >= 5) && plan.k2) small = true;
-    if (plan.k2 && len >= 1) {
-      // many short rows: several whole rows per workgroup (acc_scan_rows)
-      const KernelSource& sm = plan.k2->meta;
-      const int64_t rowsTile = (int64_t)sm.block * sm.rowsGroup * sm.vec;
-      const bool forced = forcedTiles == 3;
-      // (up to a whole tile of it: a row alone in its workgroup still moves group by group, while
-      // a tile of acc_scan that its row does not fill goes through the code for ragged ends)
-      if ((forced && len <= rowsTile) || (forcedTiles == 0 && rows >= 2 && len <= rowsTile)) {
-        const int64_t rpt = rowsTile / len;
-        const int64_t groups = (rows + rpt - 1) / rpt;
-        if (groups > 0x7fffffffLL) throw Error("scan: too many rows for one launch");
-        std::vector<uint64_t> args = packArgs(sm, aenv, temps, {});
-        packOut(args, *out);
-        packOut(args, *tot);
-        args.push_back((uint64_t)rows);
-        args.push_back((uint64_t)len);
-        args.push_back((uint64_t)rpt);
-        ctx_.launch(plan.k2, "acc_scan_rows", (uint64_t)groups, (unsigned)sm.block, args);
-        return result;
-      }
-    }
-    // Long rows of a plain array: the pipelined kernel (persistent workgroups, one per CU).  Its
-    // direct global -> LDS loads move 16 bytes per lane from 16-byte aligned addresses.
-    bool pipe = false;
-    if (plan.k3 && !small) {
-      const KernelSource& pm = plan.k3->meta;
-      const int64_t pipeTile = (int64_t)pm.block * pm.group * pm.vec;
-      const int64_t eltBytes = 16 / pm.vec;
-      // the array the kernel moves: the operand itself, or the one array a fused producer reads
-      DArrayP srcArr;
-      for (const ArraySlot& sl : pm.arrays)
-        if (sl.name == pm.pipeSlot) srcArr = sl.temp ? temps.at(sl.index) : aenv.at(aenv.size() - 1 - sl.index);
-      // (a right scan's tiles are counted from the end of each row; a producer must cover its array exactly)
-      const bool aligned = srcArr && !srcArr->bufs.empty() && ((uintptr_t)srcArr->bufs[0]->p & 15) == 0 &&
-                           srcArr->shape == ext && ((rows == 1 && !pm.scanRight) || (len * eltBytes) % 16 == 0);
-      const int64_t tprP = (len + pipeTile - 1) / pipeTile;
-      // measured on 2^28 elements: Float32 350 us against 395 us for a workgroup per tile, Int64 706
-      // against 742; from two tiles per CU on it is level or ahead (Int64 2^23, 512 tiles: 27 against
-      // 32 us; Float32 2^24, 585 tiles: 37 against 36; with 256 tiles 18.7 against 18.0)
-      pipe = aligned && (forcedTiles == 4 ? len >= pipeTile
-                                          : (forcedTiles == 0 && tprP >= 16 && rows * tprP >= 2 * ctx_.computeUnits()));
-    }
-    const KernelP& kern = pipe ? plan.k3 : (small ? plan.k2 : plan.k);
-    const KernelSource& m = kern->meta;
-    // Of the small tiles, where all of them run at once: a quarter of their size for up to a tile per CU,
-    // half of it for up to three, and every tile reads all its predecessors' aggregates (acc_scan_all,
-    // acc_scan_all2).  Measured, acc_scan / all / all2 in us, scanl: Float32 2^18 7.0 / 4.6 / 5.1, 2^20 (256 tiles
-    // of acc_scan_all) 7.5 / 6.4 / 6.4, 2^21 9.2 / 8.3 / 7.7, 2^22 12.7 / 12.7 / 10.2, 6 million (733 tiles of
-    // acc_scan_all2) 16.9 / 17.9 / 14.0, 2^23 (1024) 17.7 / 26.0 / 18.6; Int64 2^17 7.2 / 4.7 / 5.6, 2^19 (256) 7.6 /
-    // 6.1 / 6.4, 2^20 9.3 / 7.9 / 7.2, 2^21 12.6 / 12.0 / 9.8, 3 million (733) 15.0 / 16.6 / 13.0, 2^22 (1024) 17.1 / 26.2 / 17.3.
-    const char* fn = "acc_scan";
-    int64_t group = m.group;
-    if (small && (forcedTiles == 0 || forcedTiles >= 5) && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0) {
-      for (int two = forcedTiles == 6 ? 1 : 0; two < 2; ++two) {
-        const char* f = two ? "acc_scan_all2" : "acc_scan_all";
-        const int64_t g = (int64_t)m.allGroup * (two + 1), t = (int64_t)m.block * g * m.vec, all = rows * ((len + t - 1) / t);
-        const int64_t most = forcedTiles >= 5 ? 4096 : (two ? 3 : 1) * ctx_.computeUnits();
-        // (every CU holds at least one workgroup of any kernel: the runtime need not be asked)
-        if (all <= most && (all <= ctx_.computeUnits() || all <= ctx_.residentGroups(kern, f, (unsigned)m.block))) {
-          fn = f;
-          group = g;
-          break;
-        }
-        if (forcedTiles == 5) break;
-      }
-    }
-    const int64_t tile = (int64_t)m.block * group * m.vec;
-    const int64_t tpr = std::max<int64_t>(1, (len + tile - 1) / tile);
-    const int64_t tiles = rows * tpr;
-    if (tiles > 0x7fffffffLL) throw Error("scan: too many tiles for one launch");
-    const size_t descBytes = (size_t)tiles * m.words * sizeof(uint64_t);
-    ScanState& st = noAlloc_ ? staticScanState(ctx_.device(), ctx_.stream(), descBytes) : ctx_.scanState(descBytes);
-    std::vector<uint64_t> args = packArgs(m, aenv, temps, {});
-    packOut(args, *out);
-    packOut(args, *tot);
-    args.push_back((uint64_t)rows);
-    args.push_back((uint64_t)len);
-    args.push_back((uint64_t)tpr);
-    args.push_back((uint64_t)(uintptr_t)st.desc);
-    args.push_back((uint64_t)(uintptr_t)st.ticket);
-    const size_t ticketAt = args.size() - 1;
-    // fault injection for the test of the bounded look-back wait: a ticket base that lags the
-    // counter by `skew` gives every tile a number `skew` too high, so the first tiles wait for
-    // predecessors that never run, give up after `spin` polls and report
-    const uint64_t skew = (uint64_t)std::max<long long>(0, ctx_.knobs.scan_test_skew);
-    // a legitimate wait lasts microseconds; 2^22 polls are several seconds
-    const uint64_t spin = (uint64_t)std::max<long long>(1, ctx_.knobs.scan_spin_limit);
-    args.push_back((uint64_t)(st.ticketBase - skew));
-    args.push_back((uint64_t)st.epoch);
-    args.push_back(spin);
-    args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
-    const int64_t tprFull = len / tile;
-    args.push_back((uint64_t)tprFull);
-    if (pipe) {
-      // the full tiles of every row; every workgroup takes tickets until it meets the first one
-      // beyond them.  Then, with the same epoch, the rows' last tiles where they are partial.
-      const int64_t fullTiles = rows * tprFull;
-      const uint64_t groups = (uint64_t)std::min<int64_t>(fullTiles, ctx_.computeUnits());
-      ctx_.launch(kern, "acc_scan_pipe", groups, (unsigned)m.block, args);
-      // (a workgroup stops at the first ticket beyond the tiles: with the test's skew that is `skew` tickets earlier)
-      st.ticketBase += (uint64_t)std::max<int64_t>(0, fullTiles - (int64_t)skew) + groups;
-      if (tprFull < tpr) ctx_.launch(kern, "acc_scan_pipe_tail", (uint64_t)rows, (unsigned)m.block, args);
-      return result;
-    }
-    // A launch whose tiles are all on the device at once needs no tickets: a tile's number is its
-    // workgroup's, nobody waits for a tile that cannot start, and every workgroup is spared the
-    // counter's round trip in front of its loads (one row of 2^20 Int32: 7.5 -> 6.5 us).
-    const bool ticketless = skew == 0 && ctx_.knobs.scan_ticketless != 0 &&
-                            (tiles <= ctx_.computeUnits() || tiles <= ctx_.residentGroups(kern, fn, (unsigned)m.block));
-    if (ticketless) args[ticketAt] = 0;
-    ctx_.launch(kern, fn, (uint64_t)tiles, (unsigned)m.block, args);
-    if (!ticketless) st.ticketBase += (uint64_t)tiles;
-    return result;
+    launchScan(plan.k, plan.k2, plan.k3, kind, ext, aenv, temps, {out}, {tot});
+    return prime ? avPair(avArr(out), avArr(tot)) : avArr(out);
   }
   throw Error("unsupported array term '" + h + "'");
 }

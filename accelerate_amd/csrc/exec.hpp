@@ -88,6 +88,14 @@ struct Sweep {
   std::string path;          // where the component lies in the state: 'l' / 'r' per pair
 };
 
+// Two scans in a row of the same kind, direction and extents, the second of which does not read what the first
+// gives (alet p S1 (alet q S2 body)): one launch can compute both.
+struct Joint {
+  Sx second;                 // S2 in the environment of S1
+  KernelP k, k2;             // large and small tiles, elements are pairs
+  ATyP first, other;         // result types
+};
+
 class Program {
  public:
   Program(Context& ctx, const char* text, size_t len);
@@ -112,6 +120,7 @@ class Program {
   std::vector<const Sx*> lams_;
   std::map<const Sx*, Plan> plans_;
   std::map<const Sx*, Sweep> sweeps_;   // by awhile node
+  std::map<const Sx*, Joint> joints_;   // by the outer alet node
   const std::vector<DArrayP>* uses_ = nullptr;
   // runInto: alloc() hands out the caller's arrays, in the order the node asks for its results,
   // and fails once they are used up
@@ -133,8 +142,14 @@ class Program {
   static std::vector<ArrayR> aenvOf(const TEnv& tenv);
   ATyP prepareScan(const Sx& n, TEnv& tenv, Plan& plan, const Sx* post, const TypeP& postElt);
 
+  void prepareJoint(const Sx& n, TEnv& tenv);
+
   // execution
   AValP eval(const Sx& n, AEnv& aenv);
+  bool evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other);
+  // the launch of a scan over ext into outs (and totals: scan' only, else the same arrays again): one array each, two of a joint scan
+  void launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext, const AEnv& aenv,
+                  const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs, const std::vector<DArrayP>& tots);
   AValP evalFun(const Sx& f, AEnv& aenv, const std::vector<AValP>& args);
   void prepareSweeps(const Sx& n, const TEnv& tenv);
   bool awhileTest(const Sx& cond, AEnv& aenv, const AValP& x);

@@ -61,6 +61,7 @@ const KnobName kKnobs[] = {
     {"stencil_sweeps", &Knobs::stencil_sweeps}, {"stencil_rows3d", &Knobs::stencil_rows3d},
     {"pool_async", &Knobs::pool_async}, {"fold_one_launch", &Knobs::fold_one_launch},
     {"foldseg_one_launch", &Knobs::foldseg_one_launch}, {"scan_ticketless", &Knobs::scan_ticketless}, {"scan_post", &Knobs::scan_post},
+    {"scan_joint", &Knobs::scan_joint},
     {"stencil_no2d", &Knobs::stencil_no2d},       {"stencil_no3d", &Knobs::stencil_no3d},
     {"scan_tiles", &Knobs::scan_tiles},           {"scan_spin_limit", &Knobs::scan_spin_limit},
     {"scan_test_skew", &Knobs::scan_test_skew},

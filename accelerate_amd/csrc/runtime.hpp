@@ -54,6 +54,7 @@ struct Knobs {
   long long fold_target = 2048;     // workgroups a fold aims at
   long long fold_staged = 1;        // 0: ordered folds never take the kernel that stages blocks of tiles in LDS
   long long scan_post = 1;          // 0: a map around a scan is always a launch of its own
+  long long scan_joint = 1;         // 0: two scans in a row that do not depend on one another are always two launches; 2: one, whatever their size
   long long scan_ticketless = 1;    // 0: the tiles of a scan always take their numbers from the ticket counter
   long long foldseg_one_launch = 1; // 0: the ends that reach across tile borders are completed by a launch of their own
   long long fold_one_launch = 1;    // 0: a single row cut into chunks always takes the second launch (acc_fold_final)

@@ -133,6 +133,7 @@ int acchip_set_clean_hook(acchip_ctx* ctx, acchip_clean_fn fn, void* user);
  * scan_tiles (0 automatic, 1 large, 2 small, 3 rows, 4 pipelined, 5 / 6 small tiles of 64 / 128 bytes a lane), scan_spin_limit,
  * scan_test_skew, scan_ticketless (0: the tiles of a scan always take their numbers from the counter),
  * scan_post (0: the function of a map around a scan is never applied by the scan itself; read by acchip_compile),
+ * scan_joint (0: two scans in a row that do not depend on one another are always two launches; 2: one, whatever their size),
  * fold_staged (0: folds under operators that are not commutative never stage blocks of tiles in LDS),
  * fold_one_launch and foldseg_one_launch (0: the work that rides behind the main launch
  * takes a launch of its own), pool_async (0: plain hipMalloc / hipFree under the pool).  Fails for a name
