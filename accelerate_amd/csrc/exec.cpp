@@ -620,6 +620,7 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
     ATyP r = prepare(n.at(3), tenv);
     tenv.resize(mark);
     prepareJoint(n, tenv);
+    prepareAhead(n);
     return r;
   }
   if (h == "apair") {
@@ -919,6 +920,52 @@ void Program::prepareJoint(const Sx& n, TEnv& tenv) {
     (small ? j.k2 : j.k) = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, small, nullptr, nullptr, &also));
   }
   joints_.emplace(&n, std::move(j));
+}
+
+// 8 bytes of an array that holds the literal (const T lit) everywhere; false for literals it does not know
+static bool constantWord(const Sx& c, uint64_t& word) {
+  if (!isST(c.at(1)) || !c.at(2).atom) return false;
+  const ST t = parseST(c.at(1));
+  const int size = stSize(t);
+  if (stIsVec(t) || t == ST::F16) return false;
+  uint64_t bits = 0;
+  if (stIsFloat(t)) {
+    char* end = nullptr;
+    const double d = std::strtod(c.at(2).s.c_str(), &end);
+    if (!end || *end || c.at(2).s.find("n") != std::string::npos) return false;  // (nan, inf: left to the kernel)
+    const float f = (float)d;
+    std::memcpy(&bits, t == ST::F64 ? (const void*)&d : (const void*)&f, (size_t)size);
+  } else {
+    bits = (uint64_t)hostEval(c, {}, {})->i;
+  }
+  if (size < 8) bits &= ((uint64_t)1 << (8 * size)) - 1;
+  word = 0;
+  for (int at = 0; at < 8; at += size) word |= bits << (8 * at);
+  return true;
+}
+
+void Program::prepareAhead(const Sx& n) {
+  if (!n.at(2).is("scan") && !n.at(2).is("scan'")) return;
+  TEnv inner;
+  pushTypes(n.at(1), inner);
+  const Sx* next = &n.at(3);
+  if (joints_.count(&n)) {
+    pushTypes(next->at(1), inner);
+    next = &next->at(3);
+  }
+  if (next->is("alet")) next = &next->at(2);
+  if (!next->is("permute") || !next->at(2).is("generate")) return;
+  const Sx& gen = next->at(2);
+  if (!gen.at(3).is("lam") || !gen.at(3).at(2).is("const") || !hostSupported(gen.at(2))) return;
+  // (defaults that the counting kernels write together with the counts are never filled)
+  if (plans_.at(next).k->meta.permuteCountSet) return;
+  Ahead a;
+  a.defaults = &gen;
+  a.r = plans_.at(&gen).ty->r;
+  a.extent = gen.at(2);
+  if (typeLeaves(a.r.elt).size() != 1 || !constantWord(gen.at(3).at(2), a.word)) return;
+  if (!moveOut(a.extent, (long long)inner.size())) return;
+  aheads_.emplace(&n, std::move(a));
 }
 
 // ------------------------------------------------------------------------------------
@@ -1346,7 +1393,7 @@ static bool foldSegHalf(const KernelSource& full, int64_t total) {
 // three million 27.7 -> 21.4, 18.8 -> 12.6; with one source for both (flags and their opposite) the elements are read once as well.
 // From 64 MiB of pairs on two of the kernels for long rows are as fast: Int64 4 million 35.3 / 31.7, scan' 37.8 / 38.6, 8 million 53 / 59;
 // Float32 8 million 37.6 / 24.1.
-bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other) {
+bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, const std::function<void()>& before) {
   auto it = joints_.find(&n);
   if (it == joints_.end() || ctx_.knobs.scan_joint == 0) return false;
   const Joint& j = it->second;
@@ -1366,6 +1413,7 @@ bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other) {
   for (const ATyP& t : {j.first, j.other}) outs.push_back(alloc(prime ? t->a->r : t->r, oshape));
   tots = outs;
   if (prime) tots = {alloc(j.first->b->r, outer), alloc(j.other->b->r, outer)};
+  before();
   launchScan(j.k, j.k2, nullptr, kind, ext, aenv, {}, outs, tots);
   first = prime ? avPair(avArr(outs[0]), avArr(tots[0])) : avArr(outs[0]);
   other = prime ? avPair(avArr(outs[1]), avArr(tots[1])) : avArr(outs[1]);
@@ -1373,7 +1421,7 @@ bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other) {
 }
 
 void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext,
-                         const AEnv& aenv, const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs,
+                         AEnv& aenv, const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs,
                          const std::vector<DArrayP>& tots) {
   const int64_t len = std::max<int64_t>(ext.back(), 0);
   int64_t rows = 1;
@@ -1499,6 +1547,18 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
   args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
   const int64_t tprFull = len / tile;
   args.push_back((uint64_t)tprFull);
+  // (the defaults of a permute that follows: up to 64 KiB a workgroup, 16 stores a thread; blocks of the pool are a multiple of 16 bytes)
+  int64_t fillWords = 0;
+  if (aenv.fill.of && !aenv.fill.done && (!std::strcmp(fn, "acc_scan_all") || !std::strcmp(fn, "acc_scan_all2"))) {
+    const int64_t bytes = arrayBytes(*aenv.fill.array);
+    if (bytes > 0 && bytes <= tiles << 16) {
+      fillWords = (bytes + 7) / 8;
+      aenv.fill.done = true;
+    }
+  }
+  args.push_back(fillWords ? (uint64_t)(uintptr_t)aenv.fill.array->bufs[0]->p : 0);
+  args.push_back((uint64_t)fillWords);
+  args.push_back(fillWords ? aenv.fill.of->word : 0);
   if (pipe) {
     // the full tiles of every row; every workgroup takes tickets until it meets the first one
     // beyond them.  Then, with the same epoch, the rows' last tiles where they are partial.
@@ -1531,14 +1591,26 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     AValP v, other;
     size_t mark = aenv.size();
     const Sx* body = &n.at(3);
-    if (evalJoint(n, aenv, v, other)) {
-      pushVals(n.at(1), v, aenv);
-      pushVals(body->at(1), other, aenv);
-      body = &body->at(3);
+    auto ahead = aheads_.find(&n);
+    auto fill = [&]() {  // offers the next permute's defaults to the scan
+      if (ahead == aheads_.end() || noAlloc_ || !ctx_.flag(Context::kInplace) || ctx_.knobs.permute_ahead == 0) return;
+      const Ahead& a = ahead->second;
+      aenv.fill = {&a, alloc(a.r, hostShape(a.extent, aenv, Plan(), a.r.rank)), false};
+    };
+    if (joints_.count(&n)) {
+      if (evalJoint(n, aenv, v, other, fill)) {
+        pushVals(n.at(1), v, aenv);
+        pushVals(body->at(1), other, aenv);
+        body = &body->at(3);
+      }
     } else {
+      fill();
+    }
+    if (!v) {
       v = eval(n.at(2), aenv);
       pushVals(n.at(1), v, aenv);
     }
+    if (!aenv.fill.done) aenv.fill = {};
     AValP r = eval(*body, aenv);
     aenv.resize(mark);
     return r;
@@ -1917,6 +1989,11 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
         out = alloc(gr, shp);
         freshDefaults = true;
       }
+    }
+    // the scan before this node has filled the defaults already
+    if (!out && aenv.fill.done && aenv.fill.of->defaults == &n.at(2)) {
+      out = aenv.fill.array;
+      aenv.fill = {};
     }
     if (!out) {
       AValP dv = eval(n.at(2), aenv);

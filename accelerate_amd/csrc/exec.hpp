@@ -3,6 +3,7 @@
 // A Program is prepared once (parse, type inference, code generation and hipRTC for every
 // node: what `runN f` does at partial application) and executed many times.
 #pragma once
+#include <functional>
 #include <map>
 #include <memory>
 #include <vector>
@@ -96,6 +97,15 @@ struct Joint {
   ATyP first, other;         // result types
 };
 
+// A scan, or two computed together, right before a permute whose defaults are one constant (alet p S (permute f (generate sh
+// (\_ -> c)) ..), or that as the next alet's bound term): the scan's launch can fill them.
+struct Ahead {
+  const Sx* defaults = nullptr;  // the generate
+  Sx extent;                     // of the defaults, in the environment of the scan
+  ArrayR r;
+  uint64_t word = 0;             // 8 bytes of them
+};
+
 class Program {
  public:
   Program(Context& ctx, const char* text, size_t len);
@@ -121,6 +131,7 @@ class Program {
   std::map<const Sx*, Plan> plans_;
   std::map<const Sx*, Sweep> sweeps_;   // by awhile node
   std::map<const Sx*, Joint> joints_;   // by the outer alet node
+  std::map<const Sx*, Ahead> aheads_;   // by the scan's alet node (the outer one of two)
   const std::vector<DArrayP>* uses_ = nullptr;
   // runInto: alloc() hands out the caller's arrays, in the order the node asks for its results,
   // and fails once they are used up
@@ -132,6 +143,12 @@ class Program {
   struct AEnv : std::vector<DArrayP> {  // of one execution
     using std::vector<DArrayP>::vector;
     const Sx* deferred = nullptr;       // a stencil whose sweeps are being counted: yields its operand unchanged
+    // defaults of the next permute, which the scan about to be launched may fill (launchScan says whether it does)
+    struct Fill {
+      const Ahead* of = nullptr;
+      DArrayP array;
+      bool done = false;
+    } fill;
   };
 
   // preparation
@@ -143,12 +160,13 @@ class Program {
   ATyP prepareScan(const Sx& n, TEnv& tenv, Plan& plan, const Sx* post, const TypeP& postElt);
 
   void prepareJoint(const Sx& n, TEnv& tenv);
+  void prepareAhead(const Sx& n);
 
   // execution
   AValP eval(const Sx& n, AEnv& aenv);
-  bool evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other);
+  bool evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, const std::function<void()>& before);
   // the launch of a scan over ext into outs (and totals: scan' only, else the same arrays again): one array each, two of a joint scan
-  void launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext, const AEnv& aenv,
+  void launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext, AEnv& aenv,
                   const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs, const std::vector<DArrayP>& tots);
   AValP evalFun(const Sx& f, AEnv& aenv, const std::vector<AValP>& args);
   void prepareSweeps(const Sx& n, const TEnv& tenv);

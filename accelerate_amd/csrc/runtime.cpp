@@ -57,7 +57,7 @@ const KnobName kKnobs[] = {
     {"map_tiled", &Knobs::map_tiled},             {"fold_rows", &Knobs::fold_rows},
     {"fold_target", &Knobs::fold_target},         {"fold_staged", &Knobs::fold_staged},         {"fold_max_blocks", &Knobs::fold_max_blocks},         {"permute_parts", &Knobs::permute_parts},
     {"permute_count", &Knobs::permute_count},     {"permute_groups", &Knobs::permute_groups},
-    {"permute_partials", &Knobs::permute_partials}, {"permute_fresh", &Knobs::permute_fresh}, {"stencil_chain", &Knobs::stencil_chain},
+    {"permute_partials", &Knobs::permute_partials}, {"permute_fresh", &Knobs::permute_fresh}, {"permute_ahead", &Knobs::permute_ahead}, {"stencil_chain", &Knobs::stencil_chain},
     {"stencil_sweeps", &Knobs::stencil_sweeps}, {"stencil_rows3d", &Knobs::stencil_rows3d},
     {"pool_async", &Knobs::pool_async}, {"fold_one_launch", &Knobs::fold_one_launch},
     {"foldseg_one_launch", &Knobs::foldseg_one_launch}, {"scan_ticketless", &Knobs::scan_ticketless}, {"scan_post", &Knobs::scan_post},

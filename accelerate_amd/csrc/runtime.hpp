@@ -63,6 +63,7 @@ struct Knobs {
   long long permute_count = 1;      // 0: never take the counting kernel
   long long permute_groups = 0;     // 0: decide per launch
   long long permute_partials = -1;  // -1 / 0 / 1: counters summed by a second launch
+  long long permute_ahead = 1;      // 0: constant defaults are always filled by a launch of their own, also where a scan before the permute could
   long long permute_fresh = 1;      // 0: constant defaults are materialised also where the counting kernels could write them
   long long stencil_chain = 0;      // 0: decide per launch; tiles (rank 2) or planes (rank 3) per workgroup
   long long stencil_sweeps = 1;     // 0: a loop of stencil sweeps computes one at a time; > 1: waves a launch of several sweeps aims at

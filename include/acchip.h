@@ -126,7 +126,7 @@ int acchip_set_clean_hook(acchip_ctx* ctx, acchip_clean_fn fn, void* user);
  * read from the environment once, when the context is made (ACCHIP_STREAM_BYTES, ACCHIP_SCAN_TILES,
  * ...: the name in capitals), and changed afterwards only here.  Names: stream_bytes,
  * map_max_blocks, map_tiled, fold_rows, fold_target, fold_max_blocks, permute_parts, permute_count, permute_groups,
- * permute_partials, permute_fresh, stencil_chain, stencil_no2d, stencil_no3d (these two take effect for programs
+ * permute_partials, permute_fresh, permute_ahead (0: a scan never fills the constant defaults of the permute behind it), stencil_chain, stencil_no2d, stencil_no3d (these two take effect for programs
  * compiled afterwards), stencil_sweeps (0: a loop of stencil sweeps computes one at a time, for programs compiled afterwards;
  * above 1: waves a launch of several sweeps aims at), stencil_rows3d (rank-3 stencils from registers, 0: never, 1: where that is
  * faster, 2: whatever the taps and extents; for programs compiled afterwards, and at a launch where a program holds both kernels),
