@@ -2328,6 +2328,27 @@ bool Codegen::stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& 
   return halo.size() == 3 && halo[0] == 1 && halo[1] == 1 && halo[2] <= 1 && totalScalar(f);
 }
 
+// what the kernels that hold rank-3 windows in registers share: halos, boundary condition, source
+std::string Codegen::registerStencilMembers(const std::vector<int>& halo, const Sx& bnd, const ArraySlot& slot, const TypeP& elt) {
+  const std::string kind = bnd.atom ? bnd.s : bnd.head(), E = stName(elt->st);
+  std::string body;
+  const char* names[3] = {"HZ", "HY", "HX"};
+  for (int k = 0; k < 3; ++k) body += std::string("  static constexpr int ") + names[k] + " = " + std::to_string(halo[k]) + ";\n";
+  body += "  static constexpr int BOUNDARY = " + std::string(kind == "clamp" ? "0" : kind == "mirror" ? "1" : kind == "wrap" ? "2" : "3") + ";\n";
+  body += "  ACC_DEV const E* source(const Env& env) { return env." + slot.name + "_0; }\n";
+  if (kind != "constant") {
+    body += "  ACC_DEV E outside(const Env&) { return (E)0; }\n";  // not asked for
+  } else {
+    Emit em;
+    em.ind = 4;
+    ValP c = exp(bnd.at(1), {}, em);
+    if (!typeEq(valType(c), elt)) throw Error("stencil: boundary value does not have the element type");
+    em.line("return " + c->ex + ";");
+    body += fnHead("E", "outside", "const Env& env") + em.code + "  }\n";
+  }
+  return body;
+}
+
 KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src) {
   const std::vector<int> halo = stencilHaloOf(pattern);
   const std::string kind = bnd.atom ? bnd.s : bnd.head();
@@ -2343,20 +2364,7 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
   std::string body;
   int taps = 0;
   body += "  typedef " + E + " E;\n  static constexpr int R = " + std::to_string(rows) + ";\n";
-  const char* names[3] = {"HZ", "HY", "HX"};
-  for (int k = 0; k < 3; ++k) body += std::string("  static constexpr int ") + names[k] + " = " + std::to_string(halo[k]) + ";\n";
-  body += "  static constexpr int BOUNDARY = " + std::string(kind == "clamp" ? "0" : kind == "mirror" ? "1" : kind == "wrap" ? "2" : "3") + ";\n";
-  body += "  ACC_DEV const E* source(const Env& env) { return env." + slot.name + "_0; }\n";
-  if (kind != "constant") {
-    body += "  ACC_DEV E outside(const Env&) { return (E)0; }\n";  // not asked for
-  } else {
-    Emit em;
-    em.ind = 4;
-    ValP c = exp(bnd.at(1), {}, em);
-    if (!typeEq(valType(c), elt)) throw Error("stencil: boundary value does not have the element type");
-    em.line("return " + c->ex + ";");
-    body += fnHead("E", "outside", "const Env& env") + em.code + "  }\n";
-  }
+  body += registerStencilMembers(halo, bnd, slot, elt);
   {
     Emit em;
     em.ind = 4;
@@ -2394,6 +2402,143 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
   ks.words = halo[2];
   ks.taps = taps;
   ks.moved = stSize(elt->st) + stSize(outElt->st);
+  return ks;
+}
+
+// The same plane by plane (stencil3d_planes.hpp): the function's operations, each a line of generated code that defines one name, go
+// to the first of three stages by which all the planes they depend on have come; what a later stage needs of an earlier one is handed
+// on.  Throws StencilNotStaged where the function branches or hands on more than three values.
+KernelSource Codegen::stencil3dPlanes(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& bnd, const Operand& src) {
+  const std::vector<int> halo = stencilHaloOf(pattern);
+  const TypeP elt = src.r.elt;
+  const std::string E = stName(elt->st);
+  // 16 bytes of columns a lane (wrap: 8, for where a row is no whole number of lanes they are loaded one by one), three rows.  (bytes,
+  // rows), smoothing with 27 taps in chunks of 6 planes, Float32 401 x 387 x 393 / 512^3 / 200^3 and Float64 401 x 387 x 393, us: (16, 2) 109 / 220 /
+  // 15.0 / 219, (16, 3) 110 / 219 / 15.5 / 210, (16, 4) 112 / 219 / 17.9 / 230, (8, 4) 115 / 233 / 16.1, (8, 6) 115 / 233 / 16.5.
+  const int v = (bnd.isAtom("wrap") ? 8 : 16) / stSize(elt->st);
+  const int rows = 3;
+  Emit em;
+  em.ind = 0;
+  std::map<std::string, int> stage;        // of a name
+  std::map<std::string, std::string> tap;  // a tap in the window of its plane
+  const int k0 = stencilWidth(pattern) / 2;
+  ValP arg = vUnit();
+  for (int dz = -k0; dz <= k0; ++dz) {
+    const Sx& plane = pattern.at(1 + dz + k0);
+    const int k1 = stencilWidth(plane) / 2;
+    ValP pv = vUnit();
+    for (int dy = -k1; dy <= k1; ++dy) {
+      const Sx& row = plane.at(1 + dy + k1);
+      if (row.head().compare(0, 4, "unit") != 0) throw Error("stencil3d: pattern is not of rank 3");
+      const int k2 = stencilWidth(row) / 2;
+      ValP rv = vUnit();
+      for (int dx = -k2; dx <= k2; ++dx) {
+        const std::string nm = fresh();
+        stage[nm] = dz + 1;
+        tap[nm] = "w.r[b + " + std::to_string(halo[1] + dy) + "].e[k + " + std::to_string(halo[2] + dx) + "]";
+        rv = vPair(rv, vLeaf(elt->st, nm));
+      }
+      pv = vPair(pv, rv);
+    }
+    arg = vPair(arg, pv);
+  }
+  ValP r = applyFun(f, {arg}, {}, em);
+  if (!typeEq(valType(r), outElt)) throw Error("stencil: function result does not match the declared element type");
+  const std::string result = bindLeaf(outElt->st, r->ex, em)->ex;
+  static const std::regex line("const (\\w+) (v[0-9]+) = (.*);"), name("\\bv[0-9]+\\b");
+  struct Op {
+    std::string name, type, text;
+    std::vector<std::string> uses;
+    int stage;
+  };
+  std::vector<Op> ops;
+  std::set<std::string> tapsRead;
+  std::map<std::string, std::string> typeOf;
+  for (auto& t : tap) typeOf[t.first] = E;
+  for (size_t at = 0; at < em.code.size();) {
+    const size_t end = em.code.find('\n', at);
+    std::string text = em.code.substr(at, end - at);
+    at = end + 1;
+    text.erase(0, text.find_first_not_of(' '));
+    std::smatch m;
+    if (!std::regex_match(text, m, line)) throw StencilNotStaged();
+    Op op;
+    op.type = m[1];
+    op.name = m[2];
+    op.text = text;
+    op.stage = -1;  // (of constants only: computed wherever it is used)
+    const std::string expr = m[3];
+    for (std::sregex_iterator it(expr.begin(), expr.end(), name), none; it != none; ++it) {
+      const std::string u = it->str();
+      if (!stage.count(u)) throw StencilNotStaged();
+      if (tap.count(u)) tapsRead.insert(u);
+      op.uses.push_back(u);
+      op.stage = std::max(op.stage, stage[u]);
+    }
+    stage[op.name] = op.stage;
+    typeOf[op.name] = op.type;
+    ops.push_back(op);
+  }
+  // the result's line belongs to the last stage, whatever it depends on
+  ops.back().stage = stage[result] = 2;
+  std::set<std::string> handed[2];  // by the first stage, by the second
+  for (const Op& op : ops)
+    for (const std::string& u : op.uses) {
+      const int of = stage[u];
+      if (of < 0) continue;
+      for (int k = of; k < op.stage; ++k) handed[k].insert(u);
+    }
+  if (handed[0].size() + handed[1].size() > 3) throw StencilNotStaged();
+  for (const auto& part : handed)
+    for (const std::string& h : part)
+      for (const char* t : {"u8", "i8", "u16", "i16", "f16"})
+        if (typeOf[h] == t) throw StencilNotStaged();
+  std::string body;
+  body += "  typedef " + E + " E;\n  typedef " + stName(outElt->st) + " T;\n  static constexpr int R = " + std::to_string(rows) + ";\n";
+  body += "  static constexpr bool FOLD = " + std::string(plainFloat(f) ? "true" : "false") + ";\n";
+  body += "  ACC_DEV T* target(const Out& o) { return o.o0; }\n";
+  body += registerStencilMembers(halo, bnd, slotByName(src.slot), elt);
+  const char* types[2] = {"First", "Second"};
+  for (int k = 0; k < 2; ++k) {
+    body += std::string("  struct ") + types[k] + " {\n";
+    for (const std::string& h : handed[k]) body += "    " + typeOf[h] + " " + h + ";\n";
+    body += "  };\n";
+    // (values that the compiler has to compute where they stand)
+    body += std::string("  ACC_DEV void pin(") + types[k] + "& x) {\n";
+    for (const std::string& h : handed[k]) body += "    asm volatile(\"\" : \"+v\"(x." + h + "));\n";
+    body += "  }\n";
+  }
+  body += std::string("  ACC_DEV void pin(T& x) { ") + (stSize(outElt->st) >= 4 ? "asm volatile(\"\" : \"+v\"(x)); " : "") + "}\n";
+  const char* fns[3] = {"first", "second", "third"};
+  for (int k = 0; k < 3; ++k) {
+    std::string code;
+    std::set<std::string> have;
+    if (k > 0)
+      for (const std::string& h : handed[k - 1]) {
+        code += "    const " + typeOf[h] + " " + h + " = in_." + h + ";\n";
+        have.insert(h);
+      }
+    for (auto& t : tap)
+      if (stage[t.first] == k) code += "    const " + E + " " + t.first + " = " + t.second + ";\n";
+    for (const Op& op : ops)
+      if (op.stage == k || op.stage < 0) code += "    " + op.text + "\n";
+    const std::string params = std::string("const Env& env, const W& w, ") + (k > 0 ? std::string("const ") + types[k - 1] + "& in_, " : "") +
+                               "const int b, const int k";
+    if (k < 2) {
+      code += std::string("    ") + types[k] + " r_;\n";
+      for (const std::string& h : handed[k]) code += "    r_." + h + " = " + h + ";\n";
+    } else {
+      code += "    Elt r_;\n    r_.c0 = " + result + ";\n";
+    }
+    code += "    return r_;\n";
+    body += "  template <class W>\n" + fnHead(k < 2 ? types[k] : "Elt", fns[k], params.c_str()) + code + "  }\n";
+  }
+  KernelSource ks = finish(body, outElt, typeLeaves(outElt), "stencil3d_planes.hpp", v);
+  ks.group = rows;
+  ks.words = halo[2];
+  ks.taps = (int)tapsRead.size();
+  ks.moved = stSize(elt->st) + stSize(outElt->st);
+  ks.byPlanes = true;
   return ks;
 }
 

@@ -53,6 +53,9 @@ struct ScanNotPipeable {};
 // thrown by Codegen::scan when the function to apply to the results reads arrays
 struct ScanPostNotFusable {};
 
+// thrown by Codegen::stencil3dPlanes when the function does not go through its planes one after the other
+struct StencilNotStaged {};
+
 // Everything the executor needs to launch a generated kernel.
 struct KernelSource {
   std::string source;                 // full translation unit
@@ -70,6 +73,7 @@ struct KernelSource {
   int rowsGroup = 1;                  // scan only: groups per wave of acc_scan_rows (small-tile variant)
   int allGroup = 0;                   // scan only: groups per wave of acc_scan_all (twice as many in acc_scan_all2); small-tile variant
   int64_t sweepLeast = 0;             // several sweeps only: bytes an array has to have for them to be taken together
+  bool byPlanes = false;              // rank-3 stencils from registers only: acc_stencil3d_planes
   int taps = 0, moved = 0;            // rank-3 stencils from registers only: taps the function reads, bytes of an element and its result
   std::string permuteMode;            // permute only: "atomic", "cas", "lock", "store"
   bool permuteCount = false;          // permute only: has acc_permute_count (sum of a constant per source)
@@ -126,6 +130,7 @@ class Codegen {
   static bool stencilSweepable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const ArrayR& src);
   // rank 3 from registers (stencil3d_rows.hpp); only where stencilRowsable holds
   KernelSource stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
+  KernelSource stencil3dPlanes(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   static bool stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource scalarKernel(const Sx& exp);  // evaluates a closed Exp with one thread
 
@@ -160,6 +165,7 @@ class Codegen {
   ValP fromIndex(int rank, const ValP& sh, const std::string& lin, Emit& em);
   // from_index / next_index over the result's extents, the index value (ix[0], ix[1], ..) and
   // the tail that marks a producer as taking the multi-dimensional index (map.hpp)
+  std::string registerStencilMembers(const std::vector<int>& halo, const Sx& boundary, const ArraySlot& slot, const TypeP& elt);
   std::string indexedFns(int rank, const ArraySlot& o);
   ValP indexedIx(int rank);
   std::string indexedTail(int rank);

@@ -799,11 +799,19 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
         Codegen cgr(aenvOf(tenv));
         Plan scratch;
         Operand src = operandOf(n.at(5), cgr, tenv, scratch);
-        KernelSource rows = cgr.stencil3dRows(pats[0], outElt, *f, bnds[0], src);
+        KernelSource rows;
+        try {
+          Codegen cgp(aenvOf(tenv));
+          Plan scratch2;
+          rows = cgp.stencil3dPlanes(pats[0], outElt, *f, bnds[0], operandOf(n.at(5), cgp, tenv, scratch2));
+        } catch (const StencilNotStaged&) {
+          rows = cgr.stencil3dRows(pats[0], outElt, *f, bnds[0], src);
+        }
         // From registers where many taps are read: 200^3, 7 / 13 / 17 / 27 taps, Float32 1.02 / 1.17 / 1.27 / 1.37 times as fast
         // as through LDS, Float64 1.22 / 1.49 / 1.52 / 1.56.  At a launch rowsPay chooses between the two by the extents.
         const long long least = ctx_.knobs.stencil_rows3d > 1 ? 1 : stSize(srcs[0].r.elt->st) == 4 ? 16 : 25;
-        if (rows.taps >= least) plan.k2 = ctx_.kernel(rows);
+        // (plane by plane: for any number of taps)
+        if (rows.byPlanes || rows.taps >= least) plan.k2 = ctx_.kernel(rows);
       }
     } else {
       plan.k = ctx_.kernel(cg.stencil(pats, outElt, *f, bnds, srcs));
@@ -1374,6 +1382,19 @@ static bool rowsPay(const KernelSource& rows, long long knob, const std::vector<
   if (mib <= 192) return true;
   if (mib <= (rows.moved < 16 ? 512 : 1024)) return rows.taps >= 23 && fill(cols, 64 * v) >= 0.7;
   return rows.taps >= 25 && fill(128, 128) < 0.8;
+}
+
+// Does acc_stencil3d_planes take these extents, and is it faster than LDS on them?  (LDS / planes, us: Float32, 7 / 13 / 27 taps, 200^3 20.4 / 11.2,
+// 25.9 / 12.0, 32.7 / 17.0; 401 x 387 x 393 139 / 106, 146 / 108, 188 / 120; 512^3 211 / 216, 229 / 212, 310 / 235; 64 x 1000 x 1001 125 / 112,
+// 131 / 118, 159 / 128; 300 x 300 x 64 34 / 8.6, 41 / 10, 49 / 15; 40 x 60 x 80 10.2 / 5.6, 11.7 / 5.7, 15.2 / 5.7; Float64 401 x 387 x 393 250 / 210,
+// 264 / 209, 349 / 212; 512^3 422 / 428, 442 / 419, 572 / 433; 64 x 1000 x 1001 230 / 237, 239 / 237, 303 / 236.)
+static bool planesPay(const KernelSource& m, long long knob, const std::vector<int64_t>& ext) {
+  // (offsets within a plane are 32 bits wide; a lane loads V columns of one row)
+  const int64_t plane = ext[1] * ext[2];
+  if (knob == 0 || ext[0] >= (1 << 30) || ext[1] >= (1 << 24) || ext[2] >= (1 << 24) || plane * 8 >= ((int64_t)1 << 31)) return false;
+  if (ext[2] < m.vec) return false;
+  // few taps and a gibibyte of operand and result: bound by memory either way
+  return knob > 1 || m.taps >= 13 || (ext[0] * plane * m.moved) >> 20 < 896;
 }
 
 // Segmented folds over a fused producer that reads arrays: are tiles of half the length (128 B of values and flags a lane) faster?
@@ -2159,7 +2180,34 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       ctx_.launch(plan.k, "acc_stencil2d", (uint64_t)(tilesX * chunksY), 256, args);
       return avArr(out);
     }
-    if (plan.mode == "lds3d" && plan.k2 && rowsPay(plan.k2->meta, ctx_.knobs.stencil_rows3d, ext)) {
+    if (plan.mode == "lds3d" && plan.k2 && plan.k2->meta.byPlanes && planesPay(plan.k2->meta, ctx_.knobs.stencil_rows3d, ext)) {
+      if (out->size() == 0) return avArr(out);
+      const KernelSource& m = plan.k2->meta;
+      const int64_t r = m.group, bands = (ext[1] + r - 1) / r;
+      const int64_t lanes = (ext[2] + m.vec - 1) / m.vec + (m.words > 0 && n.at(4).isAtom("wrap") ? 2 : 0);
+      const int64_t own = m.words > 0 ? 62 : 64, waves = (lanes * bands + own - 1) / own, groups = (waves + 3) / 4;
+      // Chunks of 6 planes: the waves that run at a time then work on neighbouring places (27 taps, 401 x 387 x 393 Float32, 3 / 4 / 5 / 6 / 7 / 8 /
+      // 10 / 20 planes 118 / 114 / 112 / 110 / 111 / 114 / 116 / 132 us; 512^3 244 / 226 / 224 / 219 / 218 / 217 / 223 / 226).  Where that gives
+      // a CU a few workgroups only, 2 to 8, by how many a CU has to run and what a chunk takes (200^3 6 planes 15.5, 5 18.8, 4 16.6).
+      int64_t planes = 6;
+      const int64_t cus = ctx_.computeUnits();
+      if (groups * ((ext[0] + 5) / 6) < 8 * cus) {
+        int64_t best = INT64_MAX;
+        for (int64_t t : {6, 7, 8, 5, 4, 3, 2}) {
+          const int64_t cost = (groups * ((ext[0] + t - 1) / t) + cus - 1) / cus * (4 * t + 5);
+          if (cost < best) best = cost, planes = t;
+        }
+      }
+      if (ctx_.knobs.stencil_chain > 0) planes = ctx_.knobs.stencil_chain;
+      const int64_t chunks = (ext[0] + planes - 1) / planes;
+      if (groups * chunks > 0x7fffffffLL) throw Error("stencil: too many tiles for one launch");
+      std::vector<uint64_t> args = packArgs(m, aenv, temps, ext);
+      packOut(args, *out);
+      for (int64_t a : {ext[0], ext[1], ext[2], lanes, bands, groups, planes}) args.push_back((uint64_t)a);
+      ctx_.launch(plan.k2, "acc_stencil3d_planes", (uint64_t)(groups * chunks), 256, args);
+      return avArr(out);
+    }
+    if (plan.mode == "lds3d" && plan.k2 && !plan.k2->meta.byPlanes && rowsPay(plan.k2->meta, ctx_.knobs.stencil_rows3d, ext)) {
       if (out->size() == 0) return avArr(out);
       const int64_t v = plan.k2->meta.vec, hx = plan.k2->meta.words;
       const int64_t cols = 64 * v - 2 * ((hx + v - 1) / v * v);  // kCols

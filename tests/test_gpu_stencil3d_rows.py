@@ -94,3 +94,45 @@ def test_the_kernel_a_launch_takes(gpu_ctx, knobs, capfd, shape, taps, rows):
         assert ("acc_stencil3d_rows" in capfd.readouterr().err) == (knob == 2 or knob == 1 and rows)
         got[knob] = out.to_host()
     assert np.array_equal(got[0], got[2]) and np.array_equal(got[0], got[1])
+
+
+# plane by plane (stencil3d_planes.hpp): extents at the edges of a lane's columns (4, 2 of 8 bytes, 2 under wrap), of a wave's 62 lanes, of bands of
+# three rows and of chunks; the taps a function reads, from one plane or all of them
+@pytest.mark.parametrize("kind", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ty,npty,taps", [(A.f32, np.float32, "all"), (A.f64, np.float64, "cross"), (A.i32, np.int32, "cross"),
+                                          (A.i64, np.int64, "ends"), (A.f32, np.float32, "middle")], ids=str)
+def test_plane_by_plane(gpu_ctx, knobs, ty, npty, taps, kind):
+    row = A.sunit(3, ty)
+    sr = A.stup(*[A.stup(row, row, row)] * 3)
+    read = {"all": range(27), "cross": (4, 10, 12, 13, 14, 16, 22), "ends": (0, 26), "middle": (9, 13, 17)}[taps]
+
+    def f(st):
+        ts = [t for p in A.untup(st) for r in A.untup(p) for t in A.untup(r)]
+        acc = None
+        for k in read:
+            v = A.mul(ty, A.const(ty, k + 1), ts[k])
+            acc = v if acc is None else A.sub(ty, acc, v)
+        return acc
+
+    prog = A.alam([A.tarray(3, ty)], lambda g: A.stencil(sr, ty, A.lam([A.stencil_type(sr)], f),
+                                                         A.constant(ty, 3) if kind == "constant" else kind, g))
+    knobs("stencil_rows3d", 0)
+    lds = gpu_ctx.compile(prog)
+    knobs("stencil_rows3d", 2)
+    planes = gpu_ctx.compile(prog)
+    assert lds.kernel_keys != planes.kernel_keys
+    rng = np.random.default_rng(8)
+    for shape in [(2, 2, 2), (1, 1, 4), (2, 3, 3), (3, 2, 5), (6, 3, 123), (7, 4, 124), (13, 5, 125), (5, 64, 61), (12, 7, 248), (4, 10, 249),
+                  (30, 40, 50), (19, 100, 31), (3, 301, 6), (100, 33, 130)]:
+        if kind == "mirror" and min(shape) < 2:
+            continue  # refused: shorter than the taps reach
+        g = rng.integers(-999, 999, shape).astype(npty)
+        if np.dtype(npty).kind == "f":
+            g *= npty(0.37)
+            g[-1, -1, -1], g[0, 0, 0] = np.inf, npty(-0.0)
+        d = gpu_ctx.to_device(g, A.tarray(3, ty))
+        want = lds.execute(d).to_host()
+        for chain in (0, 1, 2, 3, 5):
+            knobs("stencil_chain", chain)
+            assert np.array_equal(planes.execute(d).to_host(), want, equal_nan=np.dtype(npty).kind == "f"), (shape, chain)
+        knobs("stencil_chain", 0)
