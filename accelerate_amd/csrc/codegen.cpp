@@ -918,6 +918,12 @@ KernelSource Codegen::finish(const std::string& specBody, const TypeP& elt, cons
     for (size_t k = 0; k < el.size(); ++k)
       s += "    acc_st<kStream>(&o.o" + std::to_string(k) + "[i], v.c" + std::to_string(k) + ");\n";
     s += "  }\n";
+    // V consecutive results, leaf by leaf: stores side by side that become one request, which they do not with another
+    // leaf's in between
+    s += "  template <bool kStream = false>\n  ACC_DEV void store_all(const Out& o, i64 i, const Elt* v) {\n";
+    for (size_t k = 0; k < el.size(); ++k)
+      s += "#pragma unroll\n    for (int k_ = 0; k_ < V; ++k_) acc_st<kStream>(&o.o" + std::to_string(k) + "[i + k_], v[k_].c" + std::to_string(k) + ");\n";
+    s += "  }\n";
     // V consecutive results at once: one wide request per leaf whatever the compiler can
     // prove about the alignment of position i
     s += "  ACC_DEV void store_run(const Out& o, i64 i, const Elt* v) {\n";

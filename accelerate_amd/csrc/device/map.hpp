@@ -37,8 +37,7 @@ ACC_DEV void acc_map_body(const Spec::Env& env, const Spec::Out& out, const MapP
     S::Elt r[S::V];
 #pragma unroll
     for (int k = 0; k < V; ++k) r[k] = S::produce_in(env, i0 + k, ix, k);
-#pragma unroll
-    for (int k = 0; k < V; ++k) S::store(out, i0 + k, r[k]);
+    S::store_all(out, i0, r);
     return;
   }
 #endif
@@ -49,8 +48,7 @@ ACC_DEV void acc_map_body(const Spec::Env& env, const Spec::Out& out, const MapP
       r[k] = S::produce_at(env, i0 + k, ix);
       if (k + 1 < V) S::next_index(env, ix);
     }
-#pragma unroll
-    for (int k = 0; k < V; ++k) S::store(out, i0 + k, r[k]);
+    S::store_all(out, i0, r);
   } else {
     for (int k = 0; k < V && i0 + k < p.n; ++k) {
       S::store(out, i0 + k, S::produce_at(env, i0 + k, ix));
@@ -62,8 +60,7 @@ ACC_DEV void acc_map_body(const Spec::Env& env, const Spec::Out& out, const MapP
     S::Elt r[S::V];
 #pragma unroll
     for (int k = 0; k < V; ++k) r[k] = S::produce<NT>(env, i0 + k);
-#pragma unroll
-    for (int k = 0; k < V; ++k) S::store<NT>(out, i0 + k, r[k]);
+    S::template store_all<NT>(out, i0, r);
   } else {
     for (int k = 0; k < V; ++k)
       if (i0 + k < p.n) S::store(out, i0 + k, S::produce(env, i0 + k));
@@ -117,8 +114,7 @@ acc_map_tiled(Spec::Env env, Spec::Out out, MapTiledParams p) {
     S::Elt r[S::V];
 #pragma unroll
     for (int k = 0; k < V; ++k) r[k] = S::produce(env, i0 + k);
-#pragma unroll
-    for (int k = 0; k < V; ++k) S::store(out, i0 + k, r[k]);
+    S::store_all(out, i0, r);
   } else {
     for (int k = 0; k < V && x0 + k < p.w; ++k) S::store(out, i0 + k, S::produce(env, i0 + k));
   }
