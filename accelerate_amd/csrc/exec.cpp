@@ -189,7 +189,7 @@ static HValP hShape(const std::vector<int64_t>& d) {
   return v;
 }
 
-static HValP hostEval(const Sx& e, std::vector<HValP> env, const std::vector<DArrayP>& aenv) {
+static HValP hostEval(const Sx& e, std::vector<HValP>& env, const std::vector<DArrayP>& aenv) {
   if (e.isAtom("nil")) return hvUnit();
   const std::string& h = e.head();
   if (h == "var") {
@@ -219,8 +219,11 @@ static HValP hostEval(const Sx& e, std::vector<HValP> env, const std::vector<DAr
   }
   if (h == "let") {
     HValP v = hostEval(e.at(2), env, aenv);
+    const size_t mark = env.size();
     hPush(e.at(1), v, env);
-    return hostEval(e.at(3), env, aenv);
+    HValP r = hostEval(e.at(3), env, aenv);
+    env.resize(mark);
+    return r;
   }
   if (h == "pair") {
     HValP a = hostEval(e.at(1), env, aenv);
@@ -335,6 +338,11 @@ static HValP hostEval(const Sx& e, std::vector<HValP> env, const std::vector<DAr
     if (n == "mod") return hvInt(st, wrapTo(st, adj ? r + b : r));
   }
   throw Error("host evaluation: unsupported expression '" + h + "'");
+}
+// a closed one
+static HValP hostEval(const Sx& e, const std::vector<DArrayP>& aenv) {
+  std::vector<HValP> env;
+  return hostEval(e, env, aenv);
 }
 
 // ------------------------------------------------------------------------------------
@@ -944,7 +952,7 @@ static bool constantWord(const Sx& c, uint64_t& word) {
     const float f = (float)d;
     std::memcpy(&bits, t == ST::F64 ? (const void*)&d : (const void*)&f, (size_t)size);
   } else {
-    bits = (uint64_t)hostEval(c, {}, {})->i;
+    bits = (uint64_t)hostEval(c, std::vector<DArrayP>())->i;
   }
   if (size < 8) bits &= ((uint64_t)1 << (8 * size)) - 1;
   word = 0;
@@ -1109,10 +1117,10 @@ bool Program::streams(const KernelSource& ks, const AEnv& aenv, const std::vecto
 
 HValP Program::hostExp(const Sx& e, const AEnv& aenv, const Plan& plan) {
   auto it = plan.scalarKernels.find(&e);
-  if (it == plan.scalarKernels.end()) return hostEval(e, {}, aenv);
+  if (it == plan.scalarKernels.end()) return hostEval(e, aenv);
   if (hostSupported(e, true)) {
     try {
-      return hostEval(e, {}, aenv);  // only reads scalars the host knows
+      return hostEval(e, aenv);  // only reads scalars the host knows
     } catch (const HostUnknown&) {
     }
   }
@@ -1188,7 +1196,7 @@ std::vector<DArrayP> Program::evalTemps(const std::vector<const Sx*>& temps, AEn
 
 std::vector<int64_t> Program::operandExtent(const Sx& o, const AEnv& aenv, const Plan& plan,
                                             const std::vector<DArrayP>& temps, size_t& cursor) {
-  if (o.is("delayed")) return hostShape(o.at(2), aenv, plan, parseArrayR(o.at(1)).rank);
+  if (o.is("delayed")) return hostShape(o.at(2), aenv, plan, (int)o.at(1).at(1).asInt());  // (array RANK T)
   if (o.is("avar")) {
     size_t ix = (size_t)o.at(1).asInt();
     return aenv[aenv.size() - 1 - ix]->shape;
@@ -1704,7 +1712,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     // device copy is written only if something reads it there (materialize)
     if (plan.ty->r.elt->k == Type::Scalar && !stIsFloat(plan.ty->r.elt->st) && hostSupported(n.at(2), true)) {
       try {
-        HValP v = hostEval(n.at(2), {}, aenv);
+        HValP v = hostEval(n.at(2), aenv);
         if (v->k == HVal::Leaf) {
           out->hostKnown = true;
           out->hostValue = wrapTo(plan.ty->r.elt->st, v->i);
