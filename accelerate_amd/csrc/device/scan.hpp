@@ -46,9 +46,14 @@ struct ScanParams {
   u64 spin_limit;   // polls of one window after which a tile stops waiting for its predecessors
   u32* err;         // host-visible word: 3 = a tile gave up waiting, or took a ticket outside the launch
   i64 tpr_full;     // tiles per row that lie completely inside the row (the pipelined kernel's share)
-  u64* fill;        // acc_scan_all and acc_scan_all2: a buffer to fill along the way (fill_n words with fill_word),
-  i64 fill_n;       // the constant defaults of the permute that follows
-  u64 fill_word;
+};
+
+// acc_scan_all and acc_scan_all2: a buffer to fill along the way, the constant defaults of the permute that follows (a
+// parameter of its own: the other kernels, the pipelined one among them, stay as they are)
+struct ScanFill {
+  u64* at;
+  i64 n;            // words
+  u64 word;
 };
 
 #ifndef ACC_SCAN_BLOCK

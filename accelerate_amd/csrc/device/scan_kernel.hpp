@@ -51,15 +51,16 @@ template <class S, bool ALL> ACC_DEV void acc_scan_body(const Spec::Env& env, co
     if (S::kKind == 2 && n == 0) S::store(tot, row, z);
     else S::store(out, outBase + (S::kRight ? m - 1 : 0), z);
   }
-  if constexpr (ALL) {
-    // The launch is a chain of round trips with memory idle in between: the buffer of the next node's defaults is written by its
-    // last instructions instead of by a launch of 3 us (a radix pass of one million keys 23.4 -> 19.6 us, of 1000 keys 12.1 -> 9.1).
-    const i64 step = (i64)gridDim.x * ACC_SCAN_BLOCK * 2;
-    for (i64 i = ((i64)blockIdx.x * ACC_SCAN_BLOCK + threadIdx.x) * 2; i < p.fill_n; i += step) {
-      typedef u64 Two __attribute__((ext_vector_type(2)));
-      const Two w = {p.fill_word, p.fill_word};
-      *(Two*)(p.fill + i) = w;
-    }
+}
+
+// The launch is a chain of round trips with memory idle in between: the buffer of the next node's defaults is written by its
+// last instructions instead of by a launch of 3 us (a radix pass of one million keys 23.4 -> 19.6 us, of 1000 keys 12.1 -> 9.1).
+ACC_DEV void acc_scan_fill(const ScanFill& f) {
+  const i64 step = (i64)gridDim.x * ACC_SCAN_BLOCK * 2;
+  for (i64 i = ((i64)blockIdx.x * ACC_SCAN_BLOCK + threadIdx.x) * 2; i < f.n; i += step) {
+    typedef u64 Two __attribute__((ext_vector_type(2)));
+    const Two w = {f.word, f.word};
+    *(Two*)(f.at + i) = w;
   }
 }
 
@@ -78,15 +79,17 @@ struct AccAllSpec : Spec {
   static constexpr int G = ACC_SCAN_ALL_G;
 };
 extern "C" __global__ void __launch_bounds__(ACC_SCAN_BLOCK, ACC_SCAN_MINWAVES)
-acc_scan_all(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p) {
+acc_scan_all(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p, ScanFill f) {
   acc_scan_body<AccAllSpec, true>(env, out, tot, p);
+  acc_scan_fill(f);
 }
 struct AccAll2Spec : Spec {
   static constexpr int G = 2 * ACC_SCAN_ALL_G;
 };
 extern "C" __global__ void __launch_bounds__(ACC_SCAN_BLOCK, ACC_SCAN_MINWAVES)
-acc_scan_all2(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p) {
+acc_scan_all2(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p, ScanFill f) {
   acc_scan_body<AccAll2Spec, true>(env, out, tot, p);
+  acc_scan_fill(f);
 }
 #endif
 

@@ -527,10 +527,7 @@ Program::Program(Context& ctx, const char* text, size_t len) : ctx_(ctx) {
     for (auto& sk : kv.second.scalarKernels) ctx_.wait(sk.second);
   }
   for (auto& kv : sweeps_) ctx_.wait(kv.second.k);
-  for (auto& kv : joints_) {
-    ctx_.wait(kv.second.k);
-    ctx_.wait(kv.second.k2);
-  }
+  for (auto& kv : joints_) ctx_.wait(kv.second.k);
   // a program that is one scan can be run without allocating (runInto): its code objects are
   // loaded now, so that no launch of it has set-up work left
   if (ctx_.hasDevice() && (body_->is("scan") || body_->is("scan'"))) {
@@ -550,8 +547,7 @@ std::vector<std::string> Program::kernelKeys() const {
       if (sk.second) keys.push_back(sk.second->hash);
   }
   for (auto& kv : sweeps_) keys.push_back(kv.second.k->hash);
-  for (auto& kv : joints_)
-    for (const KernelP& k : {kv.second.k, kv.second.k2}) keys.push_back(k->hash);
+  for (auto& kv : joints_) keys.push_back(kv.second.k->hash);
   std::sort(keys.begin(), keys.end());
   keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
   return keys;
@@ -926,15 +922,14 @@ void Program::prepareJoint(const Sx& n, TEnv& tenv) {
   std::vector<ST> leaves = typeLeaves(ra.elt);
   for (ST t : typeLeaves(rb.elt)) leaves.push_back(t);
   if (ra.rank != rb.rank || leaves.size() != 2 || stIsVec(leaves[0]) || stIsVec(leaves[1])) return;
-  for (int small = 0; small < 2; ++small) {
-    Codegen cg(aenvOf(tenv));
-    Plan none;
-    Operand sa = operandOf(a.at(4), cg, tenv, none), sb = operandOf(j.second.at(4), cg, tenv, none);
-    auto seed = [&](const Sx& s) -> const Sx* { return prime ? &s.at(3) : s.at(3).is("just") ? &s.at(3).at(1) : nullptr; };
-    const Codegen::Scanned also{j.second.at(2), seed(j.second), sb};
-    const int kind = prime ? 2 : seed(a) ? 1 : 0;
-    (small ? j.k2 : j.k) = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, small, nullptr, nullptr, &also));
-  }
+  // (small tiles only: what is too long for them is not computed together)
+  Codegen cg(aenvOf(tenv));
+  Plan none;
+  Operand sa = operandOf(a.at(4), cg, tenv, none), sb = operandOf(j.second.at(4), cg, tenv, none);
+  auto seed = [&](const Sx& s) -> const Sx* { return prime ? &s.at(3) : s.at(3).is("just") ? &s.at(3).at(1) : nullptr; };
+  const Codegen::Scanned also{j.second.at(2), seed(j.second), sb};
+  const int kind = prime ? 2 : seed(a) ? 1 : 0;
+  j.k = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, 1, nullptr, nullptr, &also));
   joints_.emplace(&n, std::move(j));
 }
 
@@ -1443,7 +1438,7 @@ bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, con
   tots = outs;
   if (prime) tots = {alloc(j.first->b->r, outer), alloc(j.other->b->r, outer)};
   before();
-  launchScan(j.k, j.k2, nullptr, kind, ext, aenv, {}, outs, tots);
+  launchScan(j.k, j.k, nullptr, kind, ext, aenv, {}, outs, tots);
   first = prime ? avPair(avArr(outs[0]), avArr(tots[0])) : avArr(outs[0]);
   other = prime ? avPair(avArr(outs[1]), avArr(tots[1])) : avArr(outs[1]);
   return true;
@@ -1576,18 +1571,21 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
   args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
   const int64_t tprFull = len / tile;
   args.push_back((uint64_t)tprFull);
-  // (the defaults of a permute that follows: up to 64 KiB a workgroup, 16 stores a thread; blocks of the pool are a multiple of 16 bytes)
-  int64_t fillWords = 0;
-  if (aenv.fill.of && !aenv.fill.done && (!std::strcmp(fn, "acc_scan_all") || !std::strcmp(fn, "acc_scan_all2"))) {
-    const int64_t bytes = arrayBytes(*aenv.fill.array);
-    if (bytes > 0 && bytes <= tiles << 16) {
-      fillWords = (bytes + 7) / 8;
-      aenv.fill.done = true;
+  if (std::strcmp(fn, "acc_scan") != 0) {
+    // ScanFill: the defaults of a permute that follows, up to 64 KiB a workgroup, 16 stores a thread (blocks of the pool are a
+    // multiple of 16 bytes)
+    int64_t fillWords = 0;
+    if (aenv.fill.of && !aenv.fill.done) {
+      const int64_t bytes = arrayBytes(*aenv.fill.array);
+      if (bytes > 0 && bytes <= tiles << 16) {
+        fillWords = (bytes + 7) / 8;
+        aenv.fill.done = true;
+      }
     }
+    args.push_back(fillWords ? (uint64_t)(uintptr_t)aenv.fill.array->bufs[0]->p : 0);
+    args.push_back((uint64_t)fillWords);
+    args.push_back(fillWords ? aenv.fill.of->word : 0);
   }
-  args.push_back(fillWords ? (uint64_t)(uintptr_t)aenv.fill.array->bufs[0]->p : 0);
-  args.push_back((uint64_t)fillWords);
-  args.push_back(fillWords ? aenv.fill.of->word : 0);
   if (pipe) {
     // the full tiles of every row; every workgroup takes tickets until it meets the first one
     // beyond them.  Then, with the same epoch, the rows' last tiles where they are partial.

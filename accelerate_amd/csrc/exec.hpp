@@ -93,7 +93,7 @@ struct Sweep {
 // gives (alet p S1 (alet q S2 body)): one launch can compute both.
 struct Joint {
   Sx second;                 // S2 in the environment of S1
-  KernelP k, k2;             // large and small tiles, elements are pairs
+  KernelP k;                 // elements are pairs
   ATyP first, other;         // result types
 };
 

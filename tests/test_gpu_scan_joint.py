@@ -121,7 +121,7 @@ def test_which_pairs_are_computed_together(cc_ctx):
             cc_ctx.set_knob("scan_joint", old)
 
     together = _two("scan", "l", A.i64, A.i64)
-    assert kernels(together) == apart(together) + 2
+    assert kernels(together) == apart(together) + 1
     # the second reads the first's result
     for prog in (_two("scan1", "l", A.i64, A.i64, second=lambda r: r), _two("scan'", "r", A.i64, A.i64, second=lambda r: r[0])):
         assert kernels(prog) == apart(prog)
