@@ -1438,25 +1438,24 @@ bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, con
   tots = outs;
   if (prime) tots = {alloc(j.first->b->r, outer), alloc(j.other->b->r, outer)};
   before();
-  launchScan(j.k, j.k, nullptr, kind, ext, aenv, {}, outs, tots);
+  launchScan(j.k, j.k, nullptr, kind, ext, aenv, {}, outs.data(), tots.data(), (int)outs.size());
   first = prime ? avPair(avArr(outs[0]), avArr(tots[0])) : avArr(outs[0]);
   other = prime ? avPair(avArr(outs[1]), avArr(tots[1])) : avArr(outs[1]);
   return true;
 }
 
 void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext,
-                         AEnv& aenv, const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs,
-                         const std::vector<DArrayP>& tots) {
+                         AEnv& aenv, const std::vector<DArrayP>& temps, const DArrayP* outs, const DArrayP* tots, int count) {
   const int64_t len = std::max<int64_t>(ext.back(), 0);
   int64_t rows = 1;
   for (size_t d = 0; d + 1 < ext.size(); ++d) rows *= std::max<int64_t>(ext[d], 0);
   if (rows == 0 || (kind == 0 && len == 0)) return;
   // (an argument structure starts with a word of its own: the arrays of a joint scan share one)
   auto packOuts = [&](std::vector<uint64_t>& args) {
-    for (const std::vector<DArrayP>* part : {&outs, &tots}) {
-      packOut(args, *part->at(0));
-      for (size_t i = 1; i < part->size(); ++i)
-        for (auto& b : part->at(i)->bufs) args.push_back((uint64_t)(uintptr_t)b->p);
+    for (const DArrayP* part : {outs, tots}) {
+      packOut(args, *part[0]);
+      for (int i = 1; i < count; ++i)
+        for (auto& b : part[i]->bufs) args.push_back((uint64_t)(uintptr_t)b->p);
     }
   };
   // large tiles when they fill the device, small ones otherwise
@@ -2322,7 +2321,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     DArrayP out = alloc(ar, oshape);
     DArrayP tot = out;
     if (prime) tot = alloc(plan.ty->b->r, outer);
-    launchScan(plan.k, plan.k2, plan.k3, kind, ext, aenv, temps, {out}, {tot});
+    launchScan(plan.k, plan.k2, plan.k3, kind, ext, aenv, temps, &out, &tot, 1);
     return prime ? avPair(avArr(out), avArr(tot)) : avArr(out);
   }
   throw Error("unsupported array term '" + h + "'");

@@ -165,9 +165,9 @@ class Program {
   // execution
   AValP eval(const Sx& n, AEnv& aenv);
   bool evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, const std::function<void()>& before);
-  // the launch of a scan over ext into outs (and totals: scan' only, else the same arrays again): one array each, two of a joint scan
+  // the launch of a scan over ext into outs (and totals: scan' only, else the same arrays again): `count` arrays each, two of a joint scan
   void launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3, int kind, const std::vector<int64_t>& ext, AEnv& aenv,
-                  const std::vector<DArrayP>& temps, const std::vector<DArrayP>& outs, const std::vector<DArrayP>& tots);
+                  const std::vector<DArrayP>& temps, const DArrayP* outs, const DArrayP* tots, int count);
   AValP evalFun(const Sx& f, AEnv& aenv, const std::vector<AValP>& args);
   void prepareSweeps(const Sx& n, const TEnv& tenv);
   bool awhileTest(const Sx& cond, AEnv& aenv, const AValP& x);
