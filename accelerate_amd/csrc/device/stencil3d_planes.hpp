@@ -280,6 +280,8 @@ acc_stencil3d_planes(Spec::Env env, Spec::Out out, Stencil3dPlanesParams p) {
   if constexpr (S::BOUNDARY == 2 && S::HX > 0) {
     own = own && !edge;
     --pos;
+    // (a row's last lane of its own may reach beyond it, and may be its wave's outermost, with no lending lane in the wave)
+    edge = edge || (i64)(pos + 1) * S::V > p.w;
   }
   const i64 z0 = chunk * p.planes, z1 = z0 + p.planes < p.d ? z0 + p.planes : p.d;
   if ((S::BOUNDARY == 2 && p.w % S::V == 0) || __ballot(edge) == 0) acc_planes<false>(env, out, p, own, pos * S::V, band * S::R, (int)z0, (int)z1);
