@@ -751,7 +751,19 @@ static std::string leafDecls(const std::vector<ST>& leaves, const char* prefix, 
 }
 
 std::string Codegen::eltStruct(const TypeP& t, const std::string& name) {
-  return "struct " + name + " {\n" + leafDecls(typeLeaves(t), "c", false, false) + "};\n";
+  const std::vector<ST> leaves = typeLeaves(t);
+  std::string s = "struct " + name + " {\n" + leafDecls(leaves, "c", false, false);
+  if (copyLeaves_) {
+    std::string init, assign;
+    for (size_t k = 0; k < leaves.size(); ++k) {
+      const std::string c = "c" + std::to_string(k);
+      init += (k ? ", " : " : ") + c + "(o." + c + ")";
+      assign += " " + c + " = o." + c + ";";
+    }
+    s += "  " + name + "() = default;\n  __device__ " + name + "(const " + name + "& o)" + init + " {}\n  __device__ " + name + "& operator=(const " +
+         name + "& o) {" + assign + " return *this; }\n";
+  }
+  return s + "};\n";
 }
 
 std::string Codegen::outStruct(const std::vector<ST>& leaves) {
@@ -1180,6 +1192,17 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
   auto leaves = typeLeaves(elt);
   int eltBytes = 0;
   for (ST s : leaves) eltBytes += stSize(s);
+  int laidOut, align;
+  structLayout(leaves, laidOut, align);
+  // Pairs of a leaf of one or two bytes and one of eight are copied leaf by leaf: copied as 16 bytes the padding travelled through LDS
+  // and scratch memory too, in odd pieces (u8 and i64, one million
+  // 29.9 -> 8.8 us; apart 14.4).
+  copyLeaves_ = also && laidOut - eltBytes > 4;
+  // What a lane holds of a pair lies in registers, where a leaf takes four bytes and an element its alignment: counted by the leaves'
+  // own bytes, tiles of (u8, u8), (u8, i32) and (u8, i64) had 128, 48 and 28 elements a lane, of which the first two spilled
+  // (447 and 80 registers).  scanl, before / now / apart, us: (u8, u8) 8 million 56 / 19.4 / 33.8, (u8, i32) 4 million 22.3 / 12.5 / 19.4, Float64 log of sums
+  // of exponentials beside Float32 sums 4 million 127 / 86 / 100.
+  if (also) eltBytes = std::max(laidOut, 4);
   {
     // combine(earlier, later) in traversal order; right scans apply f with the input on the
     // left (Interpreter.hs:524-526, 547-549)

@@ -147,6 +147,7 @@ class Codegen {
  private:
   friend struct CodegenImpl;
   std::vector<ArrayR> aenv_;
+  bool copyLeaves_ = false;  // elements are copied leaf by leaf, without what lies between the leaves
   std::map<std::string, ArraySlot> used_;
   std::vector<ArraySlot> temps_;
   int next_ = 0;

@@ -1415,8 +1415,8 @@ static bool foldSegHalf(const KernelSource& full, int64_t total) {
 // Both scans of a joint pair in one launch; false: one after the other, as they stand.  A scan of a few million elements is
 // a chain of round trips that one launch makes once for both: 1000 elements 9.7 -> 6.7 us, one million Int64 14.5 -> 10.2, Float32 12.1 -> 7.3,
 // three million 27.7 -> 21.4, 18.8 -> 12.6; with one source for both (flags and their opposite) the elements are read once as well.
-// From 64 MiB of pairs on two of the kernels for long rows are as fast: Int64 4 million 35.3 / 31.7, scan' 37.8 / 38.6, 8 million 53 / 59;
-// Float32 8 million 37.6 / 24.1.
+// From 1024 tiles of 64 KiB on two of the kernels for long rows are as fast: Int64 4 million 35.3 / 31.7, scan' 37.8 / 38.6, 8 million 53 / 59;
+// Float32 8 million 37.6 / 24.1, (u8, u8) 16 million 53.5 / 32.2, (u8, i64) 4 million 25.9 / 24.6.
 bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, const std::function<void()>& before) {
   auto it = joints_.find(&n);
   if (it == joints_.end() || ctx_.knobs.scan_joint == 0) return false;
@@ -1425,10 +1425,10 @@ bool Program::evalJoint(const Sx& n, AEnv& aenv, AValP& first, AValP& other, con
   size_t cur = 0;
   const std::vector<int64_t> ext = operandExtent(n.at(2).at(4), aenv, none, {}, cur);
   if (operandExtent(j.second.at(4), aenv, none, {}, cur) != ext) return false;
-  int64_t bytes = 0;
-  for (ST t : j.k->meta.outLeaves) bytes += stSize(t);
-  for (int64_t d : ext) bytes *= std::max<int64_t>(d, 0);
-  if (ctx_.knobs.scan_joint < 2 && bytes > (int64_t)64 << 20) return false;
+  const KernelSource& m = j.k->meta;
+  int64_t size = 1;
+  for (int64_t d : ext) size *= std::max<int64_t>(d, 0);
+  if (ctx_.knobs.scan_joint < 2 && size > (int64_t)1024 * m.block * m.group * m.vec) return false;
   const bool prime = n.at(2).is("scan'");
   const int kind = prime ? 2 : n.at(2).at(3).isAtom("nothing") ? 0 : 1;
   std::vector<int64_t> outer(ext.begin(), ext.end() - 1), oshape = outer;

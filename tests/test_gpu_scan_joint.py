@@ -109,6 +109,58 @@ def test_extents_that_differ(gpu_ctx):
             assert np.array_equal(g, w), (n, m)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("t1,n1,t2,n2,tile", [(A.i64, np.int64, A.i64, np.int64, 4096), (A.f32, np.float32, A.i32, np.int32, 8192),
+                                              (A.u8, np.uint8, A.u8, np.uint8, 16384), (A.u8, np.uint8, A.i32, np.int32, 8192),
+                                              (A.i16, np.int16, A.i64, np.int64, 4096)], ids=["i64-i64", "f32-i32", "u8-u8", "u8-i32", "i16-i64"])
+def test_the_line(gpu_ctx, t1, n1, t2, n2, tile):
+    """up to 1024 tiles of what a lane holds of the pairs (a leaf takes four bytes, an element its alignment) in one launch"""
+    p = gpu_ctx.compile(_two("scan", "l", t1, t2))
+    rng = np.random.default_rng(11)
+    for n, launches in ((1024 * tile, 1), (1024 * tile + 1, 2), (700 * tile + 1, 1)):
+        x, y = rng.integers(0, 2, n).astype(n1), rng.integers(0, 80, n).astype(n2)
+        args = [gpu_ctx.to_device(x, A.tarray(1, t1)), gpu_ctx.to_device(y, A.tarray(1, t2))]
+        start = gpu_ctx.stat("launches")
+        got = _leaves(p.execute(*args))
+        assert gpu_ctx.stat("launches") == start + launches
+        want = _numpy("scan", "l", np.add, 5, x) + _numpy("scan", "l", np.maximum, np.array(-7).astype(n2), y * np.array(3, n2))
+        for g, w in zip(got, want):
+            assert np.array_equal(g, w), n
+
+
+@pytest.mark.gpu
+def test_three_in_a_row_and_in_a_loop(gpu_ctx):
+    """three scans share a launch two by two; a pair inside a loop reads each iteration's state"""
+    V, Int = A.tarray(1, A.i64), A.Int
+    add = A.lam([A.i64, A.i64], lambda x, y: A.add(A.i64, x, y))
+    most = A.lam([A.i64, A.i64], lambda x, y: A.max_(A.i64, x, y))
+    scan = lambda f, xs: A.scan("l", f, None, xs)
+    three = gpu_ctx.compile(A.alam([V, V, V], lambda a, b, c: A.alet(V, scan(add, a), lambda x: A.alet(
+        V, scan(most, b), lambda y: A.alet(V, scan(add, c), lambda z: A.apair(x, A.apair(y, z)))))))
+    state = A.tpair(A.tpair(V, V), A.tarray(0, Int))
+    loop = gpu_ctx.compile(A.alam([V, V], lambda a, b: A.awhile(
+        state, lambda st: A.unit_(A.u8, A.lt(Int, A.index(st[1], A.nil), A.constI(3))),
+        lambda st: A.alet(V, scan(add, st[0][0]), lambda x: A.alet(V, scan(most, st[0][1]), lambda y: A.apair(
+            A.apair(y, x), A.unit_(Int, A.add(Int, A.index(st[1], A.nil), A.constI(1)))))),
+        A.apair(A.apair(a, b), A.unit_(Int, A.constI(0))))))
+    rng = np.random.default_rng(12)
+    for n in (3, 5000, 300001):
+        host = [rng.integers(-100, 100, n) for _ in range(3)]
+        dev = [gpu_ctx.to_device(x, V) for x in host]
+        start = gpu_ctx.stat("launches")
+        got = _leaves(three.execute(*dev))
+        assert gpu_ctx.stat("launches") == start + 2
+        for g, w in zip(got, (np.cumsum(host[0]), np.maximum.accumulate(host[1]), np.cumsum(host[2]))):
+            assert np.array_equal(g, w), n
+        a, b = host[:2]
+        for _ in range(3):
+            a, b = np.maximum.accumulate(b), np.cumsum(a)
+        start = gpu_ctx.stat("launches")
+        x, y, _ = _leaves(loop.execute(*dev[:2]))
+        assert gpu_ctx.stat("launches") == start + 3
+        assert np.array_equal(x, a) and np.array_equal(y, b), n
+
+
 def test_which_pairs_are_computed_together(cc_ctx):
     def kernels(prog):
         return len(cc_ctx.compile(prog).kernel_keys)
@@ -124,4 +176,11 @@ def test_which_pairs_are_computed_together(cc_ctx):
     assert kernels(together) == apart(together) + 1
     # the second reads the first's result
     for prog in (_two("scan1", "l", A.i64, A.i64, second=lambda r: r), _two("scan'", "r", A.i64, A.i64, second=lambda r: r[0])):
+        assert kernels(prog) == apart(prog)
+    # two directions, or only one of the two with a seed
+    V = A.tarray(1, A.i64)
+    add = A.lam([A.i64, A.i64], lambda x, y: A.add(A.i64, x, y))
+    for one, other in ((("l", None), ("r", None)), (("l", 0), ("l", None)), (("r", None), ("r", 0))):
+        scan = lambda k, xs: A.scan(k[0], add, None if k[1] is None else A.const(A.i64, k[1]), xs)
+        prog = A.alam([V, V], lambda a, b: A.alet(V, scan(one, a), lambda x: A.alet(V, scan(other, b), lambda y: A.apair(x, y))))
         assert kernels(prog) == apart(prog)
