@@ -219,7 +219,9 @@ template <int T, bool XE, bool NT> ACC_DEV void acc_sweep_strip(const Spec::Env&
 
   // Sweep t has its first row that is computed from nothing but loaded ones 2 * t * HY steps in: until then it is left out, two sweeps
   // at a time.
-  constexpr int GROUP = 2;
+  // (not where the rows kept fill the registers: 5 x 5 taps of 8 bytes, 240 of them, Float64 6000^2 112 -> 103 us a sweep, 4096^2 54.4 -> 51.1,
+  // 500 x 700 6.5 -> 7.4; Int64 6000^2 134 -> 131)
+  constexpr int GROUP = T * NP * (int)sizeof(SweepKept<S::LATE>) / 4 > 192 ? T : 2;
   auto level = [&](auto ye_, auto u_, auto t_, int yin) __attribute__((always_inline)) {
     constexpr bool YE = decltype(ye_)::value != 0;
     constexpr int u = decltype(u_)::value, t = decltype(t_)::value;

@@ -71,7 +71,7 @@ def _both(ctx, knobs, prog):
 @pytest.mark.parametrize("kind", BOUNDARIES)
 @pytest.mark.parametrize("ty,npty,widths", [
     (A.f32, np.float32, (3, 3)), (A.f32, np.float32, (5, 5)), (A.f32, np.float32, (3, 5)), (A.f32, np.float32, (5, 3)),
-    (A.f64, np.float64, (3, 3)), (A.f64, np.float64, (3, 5)), (A.i32, np.int32, (3, 3)), (A.i64, np.int64, (5, 5))], ids=str)
+    (A.f64, np.float64, (3, 3)), (A.f64, np.float64, (3, 5)), (A.f64, np.float64, (5, 5)), (A.i32, np.int32, (3, 3)), (A.i64, np.int64, (5, 5))], ids=str)
 def test_sweeps_equal_single_launches(gpu_ctx, knobs, ty, npty, kind, widths):
     step = lambda: Q.stencil_weighted(ty, widths, _boundary(kind, ty))
     fused, single = _both(gpu_ctx, knobs, sweeps(step, ty))
