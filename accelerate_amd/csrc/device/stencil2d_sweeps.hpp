@@ -36,7 +36,8 @@ struct SweepParams {
   i64 strips;     // strips of columns
   i64 items;      // strips * chunks of rows
   i64 rows;       // rows per chunk
-  i64 fewer;      // not 0: one sweep less than the kernel's number (LATE only: 4 instructions a row)
+  int fewer;      // not 0: one sweep less than the kernel's number (LATE only: 4 instructions a row)
+  int stream;     // not 0: results go past the caches (acc_sweeps10)
 };
 
 template <int N> struct AccConst { static constexpr int value = N; };
@@ -285,7 +286,7 @@ template <int T, bool XE, bool NT> ACC_DEV void acc_sweep_strip(const Spec::Env&
   }
 }
 
-template <int T, bool NT = false> ACC_DEV void acc_sweep(const Spec::Env& env, const Spec::Out& out, const SweepParams& p) {
+template <int T> ACC_DEV void acc_sweep(const Spec::Env& env, const Spec::Out& out, const SweepParams& p) {
   typedef Spec S;
   // neighbouring strips share their margins: neighbours run on the same XCD
   const i64 b = acc_xcd_contiguous((i64)blockIdx.x, (i64)gridDim.x);
@@ -295,16 +296,17 @@ template <int T, bool NT = false> ACC_DEV void acc_sweep(const Spec::Env& env, c
   const int y0 = chunk * (int)p.rows;
   const int y1 = y0 + p.rows < p.h ? y0 + (int)p.rows : (int)p.h;
   const int x0 = strip * SweepGeo<T>::U - SweepGeo<T>::HXT;
-  if (x0 >= 0 && x0 + ACC_WAVE * S::V <= p.w) acc_sweep_strip<T, false, NT>(env, out, p, strip, y0, y1);
-  else acc_sweep_strip<T, true, NT>(env, out, p, strip, y0, y1);
+  const bool inside = x0 >= 0 && x0 + ACC_WAVE * S::V <= p.w;
+  // (two copies of the sweeps' code: a choice between two stores at the end of them took 90 more registers.  Strips at the ends of
+  // the rows, which store element by element, need no third: Jacobi compiles in @ s instead of 6.7)
+  if (T >= 10 && inside && p.stream) acc_sweep_strip<T, false, (T >= 10)>(env, out, p, strip, y0, y1);
+  else if (inside) acc_sweep_strip<T, false, false>(env, out, p, strip, y0, y1);
+  else acc_sweep_strip<T, true, false>(env, out, p, strip, y0, y1);
 }
 
 #if ACC_SW_MAX >= 10
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK) acc_sweeps10(Spec::Env env, Spec::Out out, SweepParams p) {
   acc_sweep<10>(env, out, p);
-}
-extern "C" __global__ void __launch_bounds__(ACC_BLOCK) acc_sweeps10_stream(Spec::Env env, Spec::Out out, SweepParams p) {
-  acc_sweep<10, true>(env, out, p);
 }
 #endif
 #if ACC_SW_MAX >= 8

@@ -805,6 +805,7 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
         Operand src = operandOf(n.at(5), cgr, tenv, scratch);
         KernelSource rows;
         try {
+          if (!Codegen::stencilPlanesable(*f)) throw StencilNotStaged();
           Codegen cgp(aenvOf(tenv));
           Plan scratch2;
           rows = cgp.stencil3dPlanes(pats[0], outElt, *f, bnds[0], operandOf(n.at(5), cgp, tenv, scratch2));
@@ -1342,7 +1343,7 @@ DArrayP Program::launchSweeps(const Sweep& sw, DArrayP g, int64_t count) {
     const int64_t odd = ks.group >= 10;  // these kernels also do one sweep less than their number
     const int64_t T = count >= 10 - odd && ks.group >= 10 ? 10 : count >= 8 - odd && ks.group >= 8 ? 8 : count >= 4 - odd ? 4 : 2;
     const bool fewer = count < T;
-    const char* fn = T == 10 ? (2 * arrayBytes(*g) >= ctx_.knobs.stream_bytes ? "acc_sweeps10_stream" : "acc_sweeps10") : T == 8 ? "acc_sweeps8" : T == 4 ? "acc_sweeps4" : "acc_sweeps2";
+    const char* fn = T == 10 ? "acc_sweeps10" : T == 8 ? "acc_sweeps8" : T == 4 ? "acc_sweeps4" : "acc_sweeps2";
     const int64_t cols = 64 * v - 2 * ((T * hx + v - 1) / v * v);  // SweepGeo::U
     const int64_t strips = (w + cols - 1) / cols;
     // one generation of waves, as many as the device holds: a few more would run a second one
@@ -1358,7 +1359,8 @@ DArrayP Program::launchSweeps(const Sweep& sw, DArrayP g, int64_t count) {
     DArrayP out = alloc(g->r, g->shape);
     std::vector<uint64_t> args = packArgs(ks, {g}, {}, g->shape);
     packOut(args, *out);
-    for (int64_t a : {h, w, strips, strips * chunks, rows, (int64_t)fewer}) args.push_back((uint64_t)a);
+    const int64_t stream = 2 * arrayBytes(*g) >= ctx_.knobs.stream_bytes;
+    for (int64_t a : {h, w, strips, strips * chunks, rows, (int64_t)fewer | stream << 32}) args.push_back((uint64_t)a);
     ctx_.launch(sw.k, fn, (uint64_t)((strips * chunks + 3) / 4), 256, args);
     g = out;
     count -= fewer ? T - 1 : T;
