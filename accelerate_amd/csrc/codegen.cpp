@@ -2200,8 +2200,8 @@ static bool totalScalar(const Sx& e) {
 // About how many vector instructions one evaluation of a scalar function takes, equal subterms counted once;
 // past `most` the count is not finished.  What functions of nine taps added to a pass of eight sweeps, in units of
 // an addition: a division 12 (8-byte elements 15), a square root 15 (20), exp and log 13 (18), pow 140 (190); sin 33 (54) in
-// time, but its code for large arguments makes kernels of half a megabyte, like that of the others.
-static double scalarWeight(const Sx& e, double most, std::set<std::string>& seen) {
+// time, but its code for large arguments makes kernels of half a megabyte, like that of the others: `library` each.
+static double scalarWeight(const Sx& e, double most, std::set<std::string>& seen, double library = 150) {
   if (e.atom) return 0;
   double w = 0;
   if (e.is("prim")) {
@@ -2222,13 +2222,13 @@ static double scalarWeight(const Sx& e, double most, std::set<std::string>& seen
     else if (op == "sqrt") w = wide ? 20 : 15;
     else if (any({"exp", "log"})) w = wide ? 18 : 13;
     else if (op == "logbase") w = wide ? 51 : 38;
-    else if (any({"fpow", "sin", "cos", "tan", "asin", "acos", "atan", "sinh", "cosh", "tanh", "asinh", "acosh", "atanh", "atan2"})) w = 150;
+    else if (any({"fpow", "sin", "cos", "tan", "asin", "acos", "atan", "sinh", "cosh", "tanh", "asinh", "acosh", "atanh", "atan2"})) w = library;
     else if (any({"quot", "rem", "idiv", "mod", "quotrem", "divmod"})) w = wide ? 20 : 6;
     else if (op == "mul" && stIsInt(t)) w = byConst ? (wide ? 1.5 : 1) : wide ? 8 : 4;
     else if (op == "tofloating" && wide) w = 10;
   }
   if (e.is("cond") || e.is("case")) w = 1;
-  for (size_t k = 0; k < e.size() && w <= most; ++k) w += scalarWeight(e.at(k), most - w, seen);
+  for (size_t k = 0; k < e.size() && w <= most; ++k) w += scalarWeight(e.at(k), most - w, seen, library);
   return w;
 }
 
@@ -2434,6 +2434,18 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
   return ks;
 }
 
+// Is a function light enough to be taken plane by plane?  The kernel holds it about a hundred times: in every stage of every step for all
+// results of a lane, in two versions.  LDS / planes on 200^3, 401 x 387 x 393, us, and the seconds they compile, eight at a time: one sine of the sum of 7 Float32 taps
+// 28 / 15, 156 / 116, 1.0 / 3.4; of two taps among 7 34 / 28, 187 / 207, 2.8 / 8.9; of all 7 63 / 121, 420 / 1011, 2.7 / 20; 27 square roots 122 / 108, 882 /
+// 721, 1.1 / 3.5; 27 powers 852 / 202, 6500 / 1290, 5.2 / 22; Float64 27 reciprocals 153 / 113, 1119 / 790, 2.0 / 2.8; 27 exponentials 230 / 183, 1679 / 1168,
+// 4.0 / 9.0; 27 logarithms 703 / 636, 5417 / 4059, 5.4 / 29; 27 sines 817 / 849, 6340 / 6353, 5.2 / 41.  Beyond, what is read from registers at all
+// goes by stencil3d_rows.hpp, which compiles 27 Float64 sines in 13 s and exponentials in 2.
+bool Codegen::stencilPlanesable(const Sx& f) {
+  std::set<std::string> seen;
+  const double most = 480;
+  return scalarWeight(f, most, seen, 240) <= most;
+}
+
 // The same plane by plane (stencil3d_planes.hpp): the function's operations, each a line of generated code that defines one name, go
 // to the first of three stages by which all the planes they depend on have come; what a later stage needs of an earlier one is handed
 // on.  Throws StencilNotStaged where the function branches or hands on more than three values.
@@ -2474,7 +2486,9 @@ KernelSource Codegen::stencil3dPlanes(const Sx& pattern, const TypeP& outElt, co
   ValP r = applyFun(f, {arg}, {}, em);
   if (!typeEq(valType(r), outElt)) throw Error("stencil: function result does not match the declared element type");
   const std::string result = bindLeaf(outElt->st, r->ex, em)->ex;
-  static const std::regex line("const (\\w+) (v[0-9]+) = (.*);"), name("\\bv[0-9]+\\b");
+  auto isName = [](const std::string& u) {
+    return u.size() > 1 && u[0] == 'v' && u.find_first_not_of("0123456789", 1) == std::string::npos;
+  };
   struct Op {
     std::string name, type, text;
     std::vector<std::string> uses;
@@ -2489,16 +2503,26 @@ KernelSource Codegen::stencil3dPlanes(const Sx& pattern, const TypeP& outElt, co
     std::string text = em.code.substr(at, end - at);
     at = end + 1;
     text.erase(0, text.find_first_not_of(' '));
-    std::smatch m;
-    if (!std::regex_match(text, m, line)) throw StencilNotStaged();
+    // const TYPE NAME = EXPRESSION;
+    const size_t nameAt = text.find(' ', 6) + 1, eq = text.find(" = ");
+    if (text.compare(0, 6, "const ") != 0 || nameAt == 0 || eq == std::string::npos || eq < nameAt || text.back() != ';') throw StencilNotStaged();
     Op op;
-    op.type = m[1];
-    op.name = m[2];
+    op.type = text.substr(6, nameAt - 7);
+    op.name = text.substr(nameAt, eq - nameAt);
+    if (!isName(op.name)) throw StencilNotStaged();
     op.text = text;
     op.stage = -1;  // (of constants only: computed wherever it is used)
-    const std::string expr = m[3];
-    for (std::sregex_iterator it(expr.begin(), expr.end(), name), none; it != none; ++it) {
-      const std::string u = it->str();
+    auto word = [](char c) { return std::isalnum((unsigned char)c) || c == '_'; };
+    for (size_t p = eq + 3; p < text.size();) {
+      if (!word(text[p])) {
+        ++p;
+        continue;
+      }
+      size_t q = p;
+      while (word(text[q])) ++q;
+      const std::string u = text.substr(p, q - p);
+      p = q;
+      if (!isName(u)) continue;
       if (!stage.count(u)) throw StencilNotStaged();
       if (tap.count(u)) tapsRead.insert(u);
       op.uses.push_back(u);
@@ -2541,12 +2565,8 @@ KernelSource Codegen::stencil3dPlanes(const Sx& pattern, const TypeP& outElt, co
   const char* fns[3] = {"first", "second", "third"};
   for (int k = 0; k < 3; ++k) {
     std::string code;
-    std::set<std::string> have;
     if (k > 0)
-      for (const std::string& h : handed[k - 1]) {
-        code += "    const " + typeOf[h] + " " + h + " = in_." + h + ";\n";
-        have.insert(h);
-      }
+      for (const std::string& h : handed[k - 1]) code += "    const " + typeOf[h] + " " + h + " = in_." + h + ";\n";
     for (auto& t : tap)
       if (stage[t.first] == k) code += "    const " + E + " " + t.first + " = " + t.second + ";\n";
     for (const Op& op : ops)

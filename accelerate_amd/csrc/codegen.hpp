@@ -131,6 +131,7 @@ class Codegen {
   // rank 3 from registers (stencil3d_rows.hpp); only where stencilRowsable holds
   KernelSource stencil3dRows(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource stencil3dPlanes(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
+  static bool stencilPlanesable(const Sx& f);
   static bool stencilRowsable(const Sx& pattern, const TypeP& outElt, const Sx& f, const Sx& boundary, const Operand& src);
   KernelSource scalarKernel(const Sx& exp);  // evaluates a closed Exp with one thread
 

@@ -6,8 +6,6 @@ import pytest
 
 from accelerate_amd import ir as A
 
-from . import progs as Q
-
 pytestmark = pytest.mark.gpu
 
 # extents at the edges of a strip (124 columns of the 128 its lanes hold), of the four bands of 4 or 2 rows of a
@@ -16,33 +14,41 @@ SHAPES = [(2, 2, 2), (3, 3, 5), (1, 4, 7), (5, 1, 64), (4, 9, 123), (6, 8, 124),
           (33, 17, 126), (12, 100, 130), (5, 33, 248)]
 
 
-def _weighted(ty, nx, boundary):
-    """all taps of 3 x 3 x nx, distinct weights"""
-    return Q.stencil_weighted(ty, (3, 3, nx), boundary) if nx > 1 else _column(ty, boundary)
-
-
-def _column(ty, boundary):
-    """the 9 taps of 3 x 3 x 1, to a result of another type"""
-    row = A.sunit(1, ty)
+def _backward(ty, nx, out, boundary):
+    """all taps of 3 x 3 x nx from the last plane to the first, distinct weights: no function to be taken plane by plane"""
+    row = A.sunit(nx, ty)
     sr = A.stup(*[A.stup(row, row, row)] * 3)
 
     def f(st):
-        acc = A.const(A.i64, 1)
-        for p in A.untup(st):
-            for r in A.untup(p):
-                for t in A.untup(r):
-                    acc = A.add(A.i64, A.mul(A.i64, acc, A.constI(3)), A.fromintegral(ty, A.i64, t))
+        ts = [t for p in A.untup(st) for r in A.untup(p) for t in A.untup(r)]
+        acc = A.const(out, 1)
+        for k, t in enumerate(reversed(ts)):
+            t = t if ty == out else A.fromintegral(ty, out, t)
+            acc = A.add(out, acc, A.mul(out, A.const(out, k + 1), t))
         return acc
 
-    return A.alam([A.tarray(3, ty)], lambda g: A.stencil(sr, A.i64, A.lam([A.stencil_type(sr)], f), boundary, g))
+    return A.alam([A.tarray(3, ty)], lambda g: A.stencil(sr, out, A.lam([A.stencil_type(sr)], f), boundary, g))
+
+
+def _launched(ctx, capfd, prog, arg):
+    """the result, and the names of what was launched"""
+    before = ctx.flags
+    ctx.flags = before | ctx.FLAG_DUMP_EXEC
+    capfd.readouterr()
+    try:
+        out = prog.execute(arg)
+    finally:
+        ctx.flags = before
+    return out, capfd.readouterr().err
 
 
 @pytest.mark.parametrize("chain", [0, 7])
 @pytest.mark.parametrize("kind", ["clamp", "mirror", "wrap", "constant"])
 @pytest.mark.parametrize("ty,npty,nx", [(A.f32, np.float32, 3), (A.f64, np.float64, 3), (A.i32, np.int32, 3), (A.i64, np.int64, 3),
                                         (A.i32, np.int32, 1)], ids=str)
-def test_equal_to_the_lds_kernel(gpu_ctx, knobs, ty, npty, nx, kind, chain):
-    prog = _weighted(ty, nx, A.constant(ty, 3) if kind == "constant" else kind)
+def test_equal_to_the_lds_kernel(gpu_ctx, knobs, capfd, ty, npty, nx, kind, chain):
+    # (of 3 x 3 x 1 taps to a result of another type)
+    prog = _backward(ty, nx, ty if nx > 1 else A.i64, A.constant(ty, 3) if kind == "constant" else kind)
     knobs("stencil_rows3d", 0)
     lds = gpu_ctx.compile(prog)
     knobs("stencil_rows3d", 2)
@@ -58,9 +64,10 @@ def test_equal_to_the_lds_kernel(gpu_ctx, knobs, ty, npty, nx, kind, chain):
         d = gpu_ctx.to_device(g, A.tarray(3, ty))
         want = lds.execute(d).to_host()
         knobs("stencil_chain", chain)
-        got = rows.execute(d).to_host()
+        got, names = _launched(gpu_ctx, capfd, rows, d)
         knobs("stencil_chain", 0)
-        assert np.array_equal(got, want), shape
+        assert "acc_stencil3d_rows" in names, shape
+        assert np.array_equal(got.to_host(), want), shape
 
 
 # Both kernels are compiled; a launch takes the one that is faster on its extents.  Below 192 MiB of operand and
@@ -82,16 +89,11 @@ def test_the_kernel_a_launch_takes(gpu_ctx, knobs, capfd, shape, taps, rows):
 
     prog = gpu_ctx.compile(A.alam([A.tarray(3, A.f32)], lambda g: A.stencil(sr, A.f32, A.lam([A.stencil_type(sr)], f), A.clamp, g)))
     g = gpu_ctx.to_device(np.random.default_rng(9).random(shape, dtype=np.float32), A.tarray(3, A.f32))
-    got, before = {}, gpu_ctx.flags
+    got = {}
     for knob in (1, 0, 2):
         knobs("stencil_rows3d", knob)
-        gpu_ctx.flags = before | gpu_ctx.FLAG_DUMP_EXEC
-        capfd.readouterr()
-        try:
-            out = prog.execute(g)
-        finally:
-            gpu_ctx.flags = before
-        assert ("acc_stencil3d_rows" in capfd.readouterr().err) == (knob == 2 or knob == 1 and rows)
+        out, names = _launched(gpu_ctx, capfd, prog, g)
+        assert ("acc_stencil3d_rows" in names) == (knob == 2 or knob == 1 and rows)
         got[knob] = out.to_host()
     assert np.array_equal(got[0], got[2]) and np.array_equal(got[0], got[1])
 
@@ -101,7 +103,7 @@ def test_the_kernel_a_launch_takes(gpu_ctx, knobs, capfd, shape, taps, rows):
 @pytest.mark.parametrize("kind", ["clamp", "mirror", "wrap", "constant"])
 @pytest.mark.parametrize("ty,npty,taps", [(A.f32, np.float32, "all"), (A.f64, np.float64, "cross"), (A.i32, np.int32, "cross"),
                                           (A.i64, np.int64, "ends"), (A.f32, np.float32, "middle")], ids=str)
-def test_plane_by_plane(gpu_ctx, knobs, ty, npty, taps, kind):
+def test_plane_by_plane(gpu_ctx, knobs, capfd, ty, npty, taps, kind):
     row = A.sunit(3, ty)
     sr = A.stup(*[A.stup(row, row, row)] * 3)
     read = {"all": range(27), "cross": (4, 10, 12, 13, 14, 16, 22), "ends": (0, 26), "middle": (9, 13, 17)}[taps]
@@ -134,5 +136,37 @@ def test_plane_by_plane(gpu_ctx, knobs, ty, npty, taps, kind):
         want = lds.execute(d).to_host()
         for chain in (0, 1, 2, 3, 5):
             knobs("stencil_chain", chain)
-            assert np.array_equal(planes.execute(d).to_host(), want, equal_nan=np.dtype(npty).kind == "f"), (shape, chain)
+            got, names = _launched(gpu_ctx, capfd, planes, d)
+            # (rows shorter than a lane's columns go through LDS)
+            assert ("acc_stencil3d_planes" in names) == (shape[2] >= (8 if kind == "wrap" else 16) // np.dtype(npty).itemsize), shape
+            assert np.array_equal(got.to_host(), want, equal_nan=np.dtype(npty).kind == "f"), (shape, chain)
         knobs("stencil_chain", 0)
+
+
+@pytest.mark.parametrize("kind", ["clamp", "wrap"])
+@pytest.mark.parametrize("out,npout", [(A.u8, np.uint8), (A.i8, np.int8), (A.i16, np.int16), (A.u16, np.uint16)], ids=str)
+def test_plane_by_plane_to_small_results(gpu_ctx, knobs, capfd, out, npout, kind):
+    row = A.sunit(3, A.i32)
+    sr = A.stup(*[A.stup(row, row, row)] * 3)
+
+    def f(st):
+        ts = [t for p in A.untup(st) for r in A.untup(p) for t in A.untup(r)]
+        acc = ts[0]
+        for k in (4, 12, 13, 14, 22, 26):
+            acc = A.add(A.i32, acc, A.mul(A.i32, A.const(A.i32, k), ts[k]))
+        return A.fromintegral(A.i32, out, acc)
+
+    prog = A.alam([A.tarray(3, A.i32)], lambda g: A.stencil(sr, out, A.lam([A.stencil_type(sr)], f), kind, g))
+    knobs("stencil_rows3d", 0)
+    lds = gpu_ctx.compile(prog)
+    knobs("stencil_rows3d", 2)
+    planes = gpu_ctx.compile(prog)
+    rng = np.random.default_rng(3)
+    for shape in [(1, 1, 4), (3, 2, 5), (5, 4, 7), (2, 64, 61), (7, 7, 125), (4, 10, 249)]:
+        d = gpu_ctx.to_device(rng.integers(-9999, 9999, shape).astype(np.int32), A.tarray(3, A.i32))
+        got, names = _launched(gpu_ctx, capfd, planes, d)
+        assert "acc_stencil3d_planes" in names
+        knobs("stencil_rows3d", 0)
+        want = lds.execute(d).to_host()
+        knobs("stencil_rows3d", 2)
+        assert got.to_host().dtype == npout and np.array_equal(got.to_host(), want), shape
