@@ -1176,7 +1176,7 @@ bool Codegen::scanPipeable(const Operand& src, bool right) {
 }
 
 KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool right, int kind, int variant,
-                           const Sx* post, const TypeP& postElt, const Scanned* also) {
+                           const Sx* post, const TypeP& postElt, const Scanned* also, bool fill) {
   const TypeP elt = also ? tPair(src.r.elt, also->src.r.elt) : src.r.elt;
   const bool small = variant == 1, pipe = variant == 2;
   if (also && (pipe || post)) throw Error("scan: this variant takes no second scan");
@@ -1325,6 +1325,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
       // opposite, two million 41.5 -> 34.4 us a radix pass)
       allG = std::max(1, std::min(8, (also ? 128 : 64) / std::max(1, vec * std::max(1, eltBytes))));
       body += "#define ACC_SCAN_ALL_G " + std::to_string(allG) + "\n";
+      if (fill) body += "#define ACC_SCAN_FILL 1\n";
     }
     if (small && rowsG > 1 && (long)(block / 64) * (64 * (rowsG + 1) + 1) * sz <= 64 * 1024 && !(re && re[0] == '0'))
       body += "#define ACC_ROWS_RAKE 1\n";
@@ -1364,6 +1365,7 @@ KernelSource Codegen::scan(const Sx& f, const Sx* seed, const Operand& src, bool
   ks.pipeSlot = pipeSlot;
   ks.rowsGroup = rowsG;
   ks.allGroup = allG;
+  ks.scanFill = fill;
   return ks;
 }
 
@@ -2197,15 +2199,15 @@ static bool totalScalar(const Sx& e) {
   return true;
 }
 
-// About how many vector instructions one evaluation of a scalar function takes, equal subterms counted once;
-// past `most` the count is not finished.  What functions of nine taps added to a pass of eight sweeps, in units of
+// About how many vector instructions one evaluation of a scalar function takes, equal subterms counted once (where there
+// is a set for their texts); past `most` the count is not finished.  What functions of nine taps added to a pass of eight sweeps, in units of
 // an addition: a division 12 (8-byte elements 15), a square root 15 (20), exp and log 13 (18), pow 140 (190); sin 33 (54) in
 // time, but its code for large arguments makes kernels of half a megabyte, like that of the others: `library` each.
-static double scalarWeight(const Sx& e, double most, std::set<std::string>& seen, double library = 150) {
+static double scalarWeight(const Sx& e, double most, std::set<std::string>* seen, double library = 150) {
   if (e.atom) return 0;
   double w = 0;
   if (e.is("prim")) {
-    if (!seen.insert(e.str()).second) return 0;
+    if (seen && !seen->insert(e.str()).second) return 0;
     const std::string& op = e.at(1).s;
     const bool typed = e.at(2).atom && op != "land" && op != "lor" && op != "lnot";
     const ST t = typed ? parseST(e.at(2)) : ST::U8;
@@ -2244,7 +2246,7 @@ static double sweepLight(const TypeP& elt) { return stSize(elt->st) == 4 ? 32 : 
 static double sweepMost(const TypeP& elt) { return stSize(elt->st) == 4 ? 56 : 64; }
 static double sweepWeight(const TypeP& elt, const Sx& f) {
   std::set<std::string> seen;
-  return scalarWeight(f, sweepMost(elt), seen);
+  return scalarWeight(f, sweepMost(elt), &seen);
 }
 
 // Can several sweeps be computed in one pass?  (A boundary `function` has its values depend on the
@@ -2443,7 +2445,8 @@ KernelSource Codegen::stencil3dRows(const Sx& pattern, const TypeP& outElt, cons
 bool Codegen::stencilPlanesable(const Sx& f) {
   std::set<std::string> seen;
   const double most = 480;
-  return scalarWeight(f, most, seen, 240) <= most;
+  // (counted with its equal subterms first, which needs none of their texts)
+  return scalarWeight(f, most, nullptr, 240) <= most || scalarWeight(f, most, &seen, 240) <= most;
 }
 
 // The same plane by plane (stencil3d_planes.hpp): the function's operations, each a line of generated code that defines one name, go

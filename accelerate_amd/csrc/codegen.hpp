@@ -72,6 +72,7 @@ struct KernelSource {
   std::string pipeSlot;               // pipelined scan only: name of the array slot its loads move
   int rowsGroup = 1;                  // scan only: groups per wave of acc_scan_rows (small-tile variant)
   int allGroup = 0;                   // scan only: groups per wave of acc_scan_all (twice as many in acc_scan_all2); small-tile variant
+  bool scanFill = false;              // scan only: acc_scan_all and acc_scan_all2 take a ScanFill
   int64_t sweepLeast = 0;             // several sweeps only: bytes an array has to have for them to be taken together
   bool byPlanes = false;              // rank-3 stencils from registers only: acc_stencil3d_planes
   int taps = 0, moved = 0;            // rank-3 stencils from registers only: taps the function reads, bytes of an element and its result
@@ -105,13 +106,14 @@ class Codegen {
   // `map g` of `map g (scan f z xs)`, which then costs neither a launch nor an array of its own
   // also: a second scan of the same kind, direction and extents, computed together with the first (elements, results
   // and totals are pairs); not the pipelined kernel, no post
+  // fill: acc_scan_all and acc_scan_all2 take a buffer to fill along the way (ScanFill)
   struct Scanned {
     const Sx& f;
     const Sx* seed;
     const Operand& src;
   };
   KernelSource scan(const Sx& f, const Sx* seed, const Operand& src, bool right, int kind, int variant = 0,
-                    const Sx* post = nullptr, const TypeP& postElt = nullptr, const Scanned* also = nullptr);
+                    const Sx* post = nullptr, const TypeP& postElt = nullptr, const Scanned* also = nullptr, bool fill = false);
   static bool scanPipeable(const Operand& src, bool right);
   // half: tiles of half the length, for fused producers that read arrays (foldSegHalves) and not too many values
   KernelSource foldSeg(const Sx& f, const Sx* seed, const Operand& src, const Operand& seg, ST segType, bool half);

@@ -53,6 +53,7 @@ template <class S, bool ALL> ACC_DEV void acc_scan_body(const Spec::Env& env, co
   }
 }
 
+#ifdef ACC_SCAN_FILL
 // The launch is a chain of round trips with memory idle in between: the buffer of the next node's defaults is written by its
 // last instructions instead of by a launch of 3 us (a radix pass of one million keys 23.4 -> 19.6 us, of 1000 keys 12.1 -> 9.1).
 ACC_DEV void acc_scan_fill(const ScanFill& f) {
@@ -63,6 +64,10 @@ ACC_DEV void acc_scan_fill(const ScanFill& f) {
     *(Two*)(f.at + i) = w;
   }
 }
+#define ACC_SCAN_FILL_PARAM , ScanFill f
+#else
+#define ACC_SCAN_FILL_PARAM
+#endif
 
 extern "C" __global__ void __launch_bounds__(ACC_SCAN_BLOCK, ACC_SCAN_MINWAVES)
 acc_scan(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p) {
@@ -79,21 +84,29 @@ struct AccAllSpec : Spec {
   static constexpr int G = ACC_SCAN_ALL_G;
 };
 extern "C" __global__ void __launch_bounds__(ACC_SCAN_BLOCK, ACC_SCAN_MINWAVES)
-acc_scan_all(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p, ScanFill f) {
+acc_scan_all(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p ACC_SCAN_FILL_PARAM) {
+#ifdef ACC_SCAN_FILL
   const i64 words = f.n;
   asm volatile("" : : "s"(words));  // (read with the other parameters: a scalar load at the end costs 0.4 us)
+#endif
   acc_scan_body<AccAllSpec, true>(env, out, tot, p);
+#ifdef ACC_SCAN_FILL
   if (words) acc_scan_fill(f);
+#endif
 }
 struct AccAll2Spec : Spec {
   static constexpr int G = 2 * ACC_SCAN_ALL_G;
 };
 extern "C" __global__ void __launch_bounds__(ACC_SCAN_BLOCK, ACC_SCAN_MINWAVES)
-acc_scan_all2(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p, ScanFill f) {
+acc_scan_all2(Spec::Env env, Spec::Out out, Spec::Out tot, ScanParams p ACC_SCAN_FILL_PARAM) {
+#ifdef ACC_SCAN_FILL
   const i64 words = f.n;
   asm volatile("" : : "s"(words));  // (read with the other parameters: a scalar load at the end costs 0.4 us)
+#endif
   acc_scan_body<AccAll2Spec, true>(env, out, tot, p);
+#ifdef ACC_SCAN_FILL
   if (words) acc_scan_fill(f);
+#endif
 }
 #endif
 

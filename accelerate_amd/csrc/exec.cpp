@@ -602,6 +602,8 @@ ATyP Program::prepareFun(const Sx& f, TEnv& tenv, std::vector<ATyP>* params) {
   return prepare(f, tenv);
 }
 
+static const Sx* constantDefaults(const Sx& rest, uint64_t& word);
+
 ATyP Program::prepare(const Sx& n, TEnv& tenv) {
   if (n.isAtom("anil")) return atUnit();
   if (n.atom) throw Error("unexpected atom '" + n.s + "' in array term");
@@ -618,6 +620,8 @@ ATyP Program::prepare(const Sx& n, TEnv& tenv) {
     return atArr(tenv[tenv.size() - 1 - ix]);
   }
   if (h == "alet") {
+    uint64_t word;
+    if (constantDefaults(n.at(3), word)) fills_.insert(&n.at(2));
     prepare(n.at(2), tenv);
     size_t mark = tenv.size();
     pushTypes(n.at(1), tenv);
@@ -867,7 +871,7 @@ ATyP Program::prepareScan(const Sx& n, TEnv& tenv, Plan& plan, const Sx* post, c
     Codegen cgs(aenvOf(tenv));
     Plan scratch;
     Operand srcS = operandOf(n.at(4), cgs, tenv, scratch);
-    plan.k2 = ctx_.kernel(cgs.scan(n.at(2), z, srcS, dir == "r", kind, 1, post, postElt));
+    plan.k2 = ctx_.kernel(cgs.scan(n.at(2), z, srcS, dir == "r", kind, 1, post, postElt, nullptr, fills_.count(&n) != 0));
   }
   if (!post && Codegen::scanPipeable(src, dir == "r")) {
     // and as a pipeline in persistent workgroups, chosen at launch for long rows
@@ -930,7 +934,7 @@ void Program::prepareJoint(const Sx& n, TEnv& tenv) {
   auto seed = [&](const Sx& s) -> const Sx* { return prime ? &s.at(3) : s.at(3).is("just") ? &s.at(3).at(1) : nullptr; };
   const Codegen::Scanned also{j.second.at(2), seed(j.second), sb};
   const int kind = prime ? 2 : seed(a) ? 1 : 0;
-  j.k = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, 1, nullptr, nullptr, &also));
+  j.k = ctx_.kernel(cg.scan(a.at(2), seed(a), sa, a.at(1).s == "r", kind, 1, nullptr, nullptr, &also, fills_.count(&b) != 0));
   joints_.emplace(&n, std::move(j));
 }
 
@@ -956,27 +960,32 @@ static bool constantWord(const Sx& c, uint64_t& word) {
   return true;
 }
 
+// Is this what follows a scan (the rest of its alet) a permute whose defaults are one constant?  The permute, or nullptr.
+static const Sx* constantDefaults(const Sx& rest, uint64_t& word) {
+  const Sx& p = rest.is("alet") ? rest.at(2) : rest;
+  if (!p.is("permute") || !p.at(2).is("generate")) return nullptr;
+  const Sx& gen = p.at(2);
+  if (!gen.at(3).is("lam") || !gen.at(3).at(2).is("const") || !hostSupported(gen.at(2)) || !constantWord(gen.at(3).at(2), word)) return nullptr;
+  return &p;
+}
+
 void Program::prepareAhead(const Sx& n) {
   if (!n.at(2).is("scan") && !n.at(2).is("scan'")) return;
   TEnv inner;
   pushTypes(n.at(1), inner);
-  const Sx* next = &n.at(3);
+  const Sx* rest = &n.at(3);
   if (joints_.count(&n)) {
-    pushTypes(next->at(1), inner);
-    next = &next->at(3);
+    pushTypes(rest->at(1), inner);
+    rest = &rest->at(3);
   }
-  if (next->is("alet")) next = &next->at(2);
-  if (!next->is("permute") || !next->at(2).is("generate")) return;
-  const Sx& gen = next->at(2);
-  if (!gen.at(3).is("lam") || !gen.at(3).at(2).is("const") || !hostSupported(gen.at(2))) return;
-  // (defaults that the counting kernels write together with the counts are never filled)
-  if (plans_.at(next).k->meta.permuteCountSet) return;
   Ahead a;
-  a.defaults = &gen;
-  a.r = plans_.at(&gen).ty->r;
-  a.extent = gen.at(2);
-  if (typeLeaves(a.r.elt).size() != 1 || !constantWord(gen.at(3).at(2), a.word)) return;
-  if (!moveOut(a.extent, (long long)inner.size())) return;
+  const Sx* p = constantDefaults(*rest, a.word);
+  // (defaults that the counting kernels write together with the counts are never filled)
+  if (!p || plans_.at(p).k->meta.permuteCountSet) return;
+  a.defaults = &p->at(2);
+  a.r = plans_.at(a.defaults).ty->r;
+  a.extent = a.defaults->at(2);
+  if (typeLeaves(a.r.elt).size() != 1 || !moveOut(a.extent, (long long)inner.size())) return;
   aheads_.emplace(&n, std::move(a));
 }
 
@@ -1532,6 +1541,7 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
   // 6.1 / 6.4, 2^20 9.3 / 7.9 / 7.2, 2^21 12.6 / 12.0 / 9.8, 3 million (733) 15.0 / 16.6 / 13.0, 2^22 (1024) 17.1 / 26.2 / 17.3.
   const char* fn = "acc_scan";
   int64_t group = m.group;
+  bool atOnce = false;
   if (small && (forcedTiles == 0 || forcedTiles >= 5) && ctx_.knobs.scan_ticketless != 0 && ctx_.knobs.scan_test_skew == 0) {
     for (int two = forcedTiles == 6 ? 1 : 0; two < 2; ++two) {
       const char* f = two ? "acc_scan_all2" : "acc_scan_all";
@@ -1541,6 +1551,7 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
       if (all <= most && (all <= ctx_.computeUnits() || all <= ctx_.residentGroups(kern, f, (unsigned)m.block))) {
         fn = f;
         group = g;
+        atOnce = true;
         break;
       }
       if (forcedTiles == 5) break;
@@ -1553,6 +1564,7 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
   const size_t descBytes = (size_t)tiles * m.words * sizeof(uint64_t);
   ScanState& st = noAlloc_ ? staticScanState(ctx_.device(), ctx_.stream(), descBytes) : ctx_.scanState(descBytes);
   std::vector<uint64_t> args = packArgs(m, aenv, temps, {});
+  args.reserve(args.size() + 24);
   packOuts(args);
   args.push_back((uint64_t)rows);
   args.push_back((uint64_t)len);
@@ -1572,20 +1584,23 @@ void Program::launchScan(const KernelP& k, const KernelP& k2, const KernelP& k3,
   args.push_back((uint64_t)(uintptr_t)ctx_.errorWord());
   const int64_t tprFull = len / tile;
   args.push_back((uint64_t)tprFull);
-  if (std::strcmp(fn, "acc_scan") != 0) {
+  if (m.scanFill && atOnce) {
     // ScanFill: the defaults of a permute that follows, up to 64 KiB a workgroup, 16 stores a thread (blocks of the pool are a
-    // multiple of 16 bytes)
+    // multiple of 16 bytes).  They are allocated once it is known that they fit.
     int64_t fillWords = 0;
-    if (aenv.fill.of && !aenv.fill.done) {
-      const int64_t bytes = arrayBytes(*aenv.fill.array);
+    AEnv::Fill& fill = aenv.fill;
+    if (fill.of && !fill.array && aenv.size() == fill.depth) {
+      const std::vector<int64_t> shape = hostShape(fill.of->extent, aenv, Plan(), fill.of->r.rank);
+      int64_t bytes = stSize(typeLeaves(fill.of->r.elt)[0]);
+      for (int64_t d : shape) bytes = d <= 0 ? 0 : bytes > tiles << 16 ? bytes : bytes * d;
       if (bytes > 0 && bytes <= tiles << 16) {
         fillWords = (bytes + 7) / 8;
-        aenv.fill.done = true;
+        fill.array = alloc(fill.of->r, shape);
       }
     }
-    args.push_back(fillWords ? (uint64_t)(uintptr_t)aenv.fill.array->bufs[0]->p : 0);
+    args.push_back(fillWords ? (uint64_t)(uintptr_t)fill.array->bufs[0]->p : 0);
     args.push_back((uint64_t)fillWords);
-    args.push_back(fillWords ? aenv.fill.of->word : 0);
+    args.push_back(fillWords ? fill.of->word : 0);
   }
   if (pipe) {
     // the full tiles of every row; every workgroup takes tickets until it meets the first one
@@ -1620,25 +1635,24 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
     size_t mark = aenv.size();
     const Sx* body = &n.at(3);
     auto ahead = aheads_.find(&n);
-    auto fill = [&]() {  // offers the next permute's defaults to the scan
-      if (ahead == aheads_.end() || noAlloc_ || !ctx_.flag(Context::kInplace) || ctx_.knobs.permute_ahead == 0) return;
-      const Ahead& a = ahead->second;
-      aenv.fill = {&a, alloc(a.r, hostShape(a.extent, aenv, Plan(), a.r.rank)), false};
+    auto offer = [&]() {  // the next permute's defaults, to the scan
+      if (ahead != aheads_.end() && !noAlloc_ && ctx_.flag(Context::kInplace) && ctx_.knobs.permute_ahead != 0)
+        aenv.fill = {&ahead->second, aenv.size(), nullptr};
     };
     if (joints_.count(&n)) {
-      if (evalJoint(n, aenv, v, other, fill)) {
+      if (evalJoint(n, aenv, v, other, offer)) {
         pushVals(n.at(1), v, aenv);
         pushVals(body->at(1), other, aenv);
         body = &body->at(3);
       }
     } else {
-      fill();
+      offer();
     }
     if (!v) {
       v = eval(n.at(2), aenv);
       pushVals(n.at(1), v, aenv);
     }
-    if (!aenv.fill.done) aenv.fill = {};
+    if (!aenv.fill.array) aenv.fill = {};
     AValP r = eval(*body, aenv);
     aenv.resize(mark);
     return r;
@@ -2019,7 +2033,7 @@ AValP Program::eval(const Sx& n, AEnv& aenv) {
       }
     }
     // the scan before this node has filled the defaults already
-    if (!out && aenv.fill.done && aenv.fill.of->defaults == &n.at(2)) {
+    if (!out && aenv.fill.array && aenv.fill.of->defaults == &n.at(2)) {
       out = aenv.fill.array;
       aenv.fill = {};
     }

@@ -6,6 +6,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <set>
 #include <vector>
 
 #include "runtime.hpp"
@@ -131,6 +132,7 @@ class Program {
   std::map<const Sx*, Plan> plans_;
   std::map<const Sx*, Sweep> sweeps_;   // by awhile node
   std::map<const Sx*, Joint> joints_;   // by the outer alet node
+  std::set<const Sx*> fills_;           // scans whose small tiles can fill defaults along the way
   std::map<const Sx*, Ahead> aheads_;   // by the scan's alet node (the outer one of two)
   const std::vector<DArrayP>* uses_ = nullptr;
   // runInto: alloc() hands out the caller's arrays, in the order the node asks for its results,
@@ -146,8 +148,8 @@ class Program {
     // defaults of the next permute, which the scan about to be launched may fill (launchScan says whether it does)
     struct Fill {
       const Ahead* of = nullptr;
-      DArrayP array;
-      bool done = false;
+      size_t depth = 0;   // arrays bound where the scan stands
+      DArrayP array;      // once a launch has filled them
     } fill;
   };
 
