@@ -146,6 +146,31 @@ template <int CTRL, int ROW_MASK, class T> ACC_DEV T acc_dpp(const T& v) {
   return acc_from_words<T>(w);
 }
 
+// The value of the lane to the left (wave_shr:1 = 0x138) or right (wave_shl:1 = 0x130).  The wave's outermost lane, which has no such
+// neighbour, gets a value that nobody may use: its own, or, if the caller folds, 0.  Without an old value to keep the compiler makes
+// the move a modifier of the operation that uses it, which then costs no instruction of its own.  FOLD may be set only where all that is
+// computed with the values are floating-point additions, subtractions, multiplications and negations: an integer subtraction
+// with the modifier, whose other operand a 64-bit multiply-add had written two wait states before, came out wrong
+// (Int32, l + 3 c - r), as if it had read that register too early.  Why is not known, so elements that are not floating-point never fold.
+template <class T> struct AccFolds { static constexpr bool value = false; };
+template <> struct AccFolds<float> { static constexpr bool value = true; };
+template <> struct AccFolds<double> { static constexpr bool value = true; };
+template <int CTRL, bool FOLD, class T> ACC_DEV T acc_neighbour(const T& v) {
+  static_assert(CTRL == 0x138 || CTRL == 0x130, "a wave shift by one lane");
+  if constexpr (!FOLD || !AccFolds<T>::value) {
+    return acc_dpp<CTRL, 0xf>(v);
+  } else {
+    u32 w[AccWords<T>::N];
+    acc_to_words(v, w);
+#pragma unroll
+    for (int k = 0; k < AccWords<T>::N; ++k) w[k] = (u32)__builtin_amdgcn_update_dpp(0, (int)w[k], CTRL, 0xf, 0xf, true);
+    return acc_from_words<T>(w);
+  }
+}
+
+// a number as a type, for code that is unrolled by overloading
+template <int N> struct AccConst { static constexpr int value = N; };
+
 // value held by lane `src` (wave-uniform) of the wave
 template <class T> ACC_DEV T acc_readlane(const T& v, int src) {
   u32 w[AccWords<T>::N];

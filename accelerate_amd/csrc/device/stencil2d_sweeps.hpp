@@ -40,22 +40,6 @@ struct SweepParams {
   int stream;     // not 0: results go past the caches (acc_sweeps10)
 };
 
-template <int N> struct AccConst { static constexpr int value = N; };
-
-// The value of the lane to the left (wave_shr:1 = 0x138) or right (wave_shl:1 = 0x130), as acc_dpp gives it, but 0 instead of their
-// own in the outermost lanes, which lie in the margins.  Without an old value to keep the compiler makes the move a modifier of
-// the addition that uses it.  For Spec::LATE only, that is for functions of floating-point additions and multiplications: a
-// subtraction with the modifier whose other operand a 64-bit integer multiply-add had written two wait states before
-// came out wrong (Int32, l + 3 c - r), as if it had read that register too early.
-template <int CTRL, class T> ACC_DEV T acc_shift(const T& v) {
-  if constexpr (!Spec::LATE) return acc_dpp<CTRL, 0xf>(v);
-  u32 w[AccWords<T>::N];
-  acc_to_words(v, w);
-#pragma unroll
-  for (int k = 0; k < AccWords<T>::N; ++k) w[k] = (u32)__builtin_amdgcn_update_dpp(0, (int)w[k], CTRL, 0xf, 0xf, true);
-  return acc_from_words<T>(w);
-}
-
 struct SweepRow { Spec::E e[ACC_SW_E]; };
 
 // v with its neighbours; XE: the strip reaches beyond the first or last column; OWN: the lane's own columns may lie outside
@@ -69,8 +53,8 @@ template <bool XE, bool OWN> ACC_DEV SweepRow acc_sweep_expand(const Spec::Env& 
   for (int k = 0; k < V; ++k) r.e[HX + k] = v[k];
 #pragma unroll
   for (int j = 1; j <= HX; ++j) {
-    r.e[HX - j] = acc_shift<0x138>(v[V - j]);          // from the lane to the left
-    r.e[HX + V - 1 + j] = acc_shift<0x130>(v[j - 1]);  // from the lane to the right
+    r.e[HX - j] = acc_neighbour<0x138, S::LATE>(v[V - j]);          // from the lane to the left
+    r.e[HX + V - 1 + j] = acc_neighbour<0x130, S::LATE>(v[j - 1]);  // from the lane to the right
   }
   if constexpr (XE && S::BOUNDARY != 2) {
     // a lane starts at column 0 or at a multiple of V from it, so only the last column can lie

@@ -37,18 +37,6 @@ struct PlaneWin { PlaneRow r[ACC_SP_ROWS]; };
 static constexpr int kEnd = Spec::HX > 0 ? 1 : 0;  // lanes at either end of a wave that only lend their columns
 static constexpr int kOwn = ACC_WAVE - 2 * kEnd;
 
-// from the lane to the left (wave_shr:1 = 0x138) or right (wave_shl:1 = 0x130).  Functions of float additions and multiplications
-// (Spec::FOLD) need no old value kept in the outermost lanes, which makes the move a modifier of the operation that uses it; behind
-// 64-bit integer multiply-adds that modifier has given wrong values.
-template <int CTRL, class T> ACC_DEV T acc_side(const T& v) {
-  if constexpr (!Spec::FOLD) return acc_dpp<CTRL, 0xf>(v);
-  u32 w[AccWords<T>::N];
-  acc_to_words(v, w);
-#pragma unroll
-  for (int k = 0; k < AccWords<T>::N; ++k) w[k] = (u32)__builtin_amdgcn_update_dpp(0, (int)w[k], CTRL, 0xf, 0xf, true);
-  return acc_from_words<T>(w);
-}
-
 template <bool XE> ACC_DEV PlaneRow acc_plane_row(const Spec::Env& env, const Spec::E (&v)[Spec::V], int gx, int w) {
   typedef Spec S;
   const int V = S::V, HX = S::HX;
@@ -58,18 +46,18 @@ template <bool XE> ACC_DEV PlaneRow acc_plane_row(const Spec::Env& env, const Sp
   if constexpr (XE && S::BOUNDARY != 2) {
     // (columns of the lane itself that lie outside: mirror may need the left neighbour, so neighbours come first)
 #pragma unroll
-    for (int j = 1; j <= HX; ++j) r.e[HX - j] = acc_side<0x138>(v[V - j]);
+    for (int j = 1; j <= HX; ++j) r.e[HX - j] = acc_neighbour<0x138, S::FOLD>(v[V - j]);
     if constexpr (S::BOUNDARY == 0) {
 #pragma unroll
       for (int i = -1; i >= -HX; --i) r.e[HX + i] = gx + i < 0 ? r.e[HX + i + 1] : r.e[HX + i];
 #pragma unroll
-      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_side<0x130>(v[j - 1]);
+      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_neighbour<0x130, S::FOLD>(v[j - 1]);
       // (its own are right already: acc_planes moves a row's last element along)
 #pragma unroll
       for (int i = V; i < V + HX; ++i) r.e[HX + i] = gx + i >= w ? r.e[HX + i - 1] : r.e[HX + i];
     } else if constexpr (S::BOUNDARY == 1) {
 #pragma unroll
-      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_side<0x130>(v[j - 1]);
+      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_neighbour<0x130, S::FOLD>(v[j - 1]);
 #pragma unroll
       for (int j = 1; j <= HX; ++j) r.e[HX - j] = gx == 0 ? r.e[HX + j] : r.e[HX - j];
 #pragma unroll
@@ -79,7 +67,7 @@ template <bool XE> ACC_DEV PlaneRow acc_plane_row(const Spec::Env& env, const Sp
           if (i - 2 * j >= -HX) r.e[HX + i] = gx + i == w - 1 + j ? r.e[HX + i - 2 * j] : r.e[HX + i];
     } else {
 #pragma unroll
-      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_side<0x130>(v[j - 1]);
+      for (int j = 1; j <= HX; ++j) r.e[HX + V - 1 + j] = acc_neighbour<0x130, S::FOLD>(v[j - 1]);
       const S::E c = S::outside(env);
 #pragma unroll
       for (int i = -HX; i < V + HX; ++i) r.e[HX + i] = (gx + i < 0 || gx + i >= w) ? c : r.e[HX + i];
@@ -87,8 +75,8 @@ template <bool XE> ACC_DEV PlaneRow acc_plane_row(const Spec::Env& env, const Sp
   } else {
 #pragma unroll
     for (int j = 1; j <= HX; ++j) {
-      r.e[HX - j] = acc_side<0x138>(v[V - j]);
-      r.e[HX + V - 1 + j] = acc_side<0x130>(v[j - 1]);
+      r.e[HX - j] = acc_neighbour<0x138, S::FOLD>(v[V - j]);
+      r.e[HX + V - 1 + j] = acc_neighbour<0x130, S::FOLD>(v[j - 1]);
     }
   }
   return r;
@@ -106,8 +94,6 @@ ACC_DEV int acc_bounded(int j, int n) {
   }
   return j < 0 ? 0 : (j >= n ? n - 1 : j);
 }
-
-template <int N> struct AccConst { static constexpr int value = N; };
 
 template <bool XE> ACC_DEV void acc_planes(const Spec::Env& env, const Spec::Out& out, const Stencil3dPlanesParams& p, bool own,
                                            int gx, int y0, int z0, int z1) {

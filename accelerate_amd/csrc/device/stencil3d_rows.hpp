@@ -20,8 +20,6 @@
 #define ACC_SR_PZ (2 * Spec::HZ + 1)
 #define ACC_SR_E (Spec::V + 2 * Spec::HX)
 
-template <int N> struct AccConst { static constexpr int value = N; };
-
 struct Stencil3dRowsParams {
   i64 d, h, w;     // extents
   i64 strips;      // strips of columns

@@ -85,11 +85,8 @@ template <int N> struct acc_run<Res, N> {
   acc_run& operator=(const acc_run&) { result().touch(this, N); return *this; }
 };
 
-template <class T> struct AccWords { enum { N = sizeof(T) / 4 }; };
-template <class T> void acc_to_words(const T&, u32*) {}
-template <class T> T acc_from_words(const u32*) { return T(); }
-template <int CTRL, int ROWS, class T> T acc_dpp(const T&) { return T(); }
-static int __builtin_amdgcn_update_dpp(int, int v, int, int, int, bool) { return v; }
+template <int CTRL, bool FOLD, class T> T acc_neighbour(const T&) { return T(); }
+template <int N> struct AccConst { static constexpr int value = N; };
 
 struct Spec {
   struct Env {};

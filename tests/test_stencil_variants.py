@@ -1,4 +1,7 @@
 """Which stencils the code generator gives a variant of their own, compile-only (gfx950, no GPU)."""
+import os
+import re
+
 import pytest
 
 from accelerate_amd import hip, ir as A
@@ -79,3 +82,17 @@ def test_functions_taken_plane_by_plane(capfd, name):
     finally:
         ctx.close()
     assert [k for k in ("planes", "rows") if "acc_stencil3d_%s(" % k in source] == [kind]
+
+
+def test_moves_between_lanes_are_folded_in_one_place():
+    """A wave shift without an old value may become a modifier of the operation that uses it, which is known to be right behind
+    floating-point operations only: acc_neighbour is the one place that makes such a shift, and asks for the type."""
+    device = os.path.join(os.path.dirname(hip.LIB_PATH), "csrc", "device")
+    made = {}
+    for name in os.listdir(device):
+        with open(os.path.join(device, name)) as f:
+            text = f.read()
+        n = len(re.findall(r"__builtin_amdgcn_(?:update|mov)_dpp\w*\((?!\(int\)(\w+\[k\]), \(int\)\1)", text))
+        if n:
+            made[name] = n
+    assert made == {"prelude.hpp": 1}
