@@ -13,8 +13,9 @@
 // and moves them.
 //
 // Measured (smoothing with 27 taps, 401 x 387 x 393 Float32, floor of the traffic 76 us): 110 us; three planes in registers (stencil3d_rows.hpp)
-// 162, through LDS 194.  39 vector instructions a result, of which 26 are its additions, against 62 and 100; every row is loaded
-// 5 / 3 times (borders of bands) and every plane 8 / 6 times (borders of chunks), mostly from the L2.  Float64 210 / 319 / 333 us.
+// 162, through LDS 194.  49.5 vector instructions a result (47.2 million), of which 26 are its additions and about ten the planes
+// recomputed at the ends of chunks, against 62 and 100; every row is loaded 5 / 3 times (borders of bands) and every plane 8 / 6 times (borders
+// of chunks), mostly from the L2.  Float64 210 / 319 / 333 us.
 //
 // Outside the array a tap is replaced as `bounded` says (Interpreter.hs:797-839): columns in the registers, rows and
 // planes by the index that is loaded, or the constant.  Lanes outside the array compute values nobody uses, on taps that no
